@@ -446,6 +446,24 @@ int mnx_indexed_block_linear_f32(const float* a, int64_t a_stride, int32_t nseg,
                                  int64_t out_stride, int64_t out_off, int32_t out_comp, mnx_stream_t stream);
 
 /* ------------------------------------------------------------------------ */
+/* Weight gradient of a whole ir_mul linear (the cuet.Linear backward,        */
+/* src/molrep/interaction/linear.py:43-105): for each of npair pairs of an    */
+/* input and an output block of one irrep                                     */
+/*   gw[wo + c*N + p] = scale * sum_{n < R, i < d}                            */
+/*       x[n*x_stride + xcol + i*xcomp + c] * g[n*g_stride + gcol + i*gcomp + p] */
+/* for c < M, p < N (overwritten; R = 0 gives zeros).  desc holds 8 integers  */
+/* per pair (xcol, xcomp, M, gcol, gcomp, N, d, wo), scale one factor per     */
+/* pair; both are host memory.  fp32-accurate products (three-way bf16 splits), */
+/* summed in a fixed order (deterministic).  Widths, columns, component steps  */
+/* and row strides even; x and g 8-byte aligned.                              */
+/* ------------------------------------------------------------------------ */
+size_t mnx_block_linear_wgrad_workspace_bytes(const int64_t* desc, int32_t npair, int64_t x_stride,
+                                              int64_t g_stride, int64_t R);
+int mnx_block_linear_wgrad_f32(const float* x, int64_t x_stride, const float* g, int64_t g_stride, int64_t R,
+                               int32_t npair, const int64_t* desc, const float* scale, float* gw, void* ws,
+                               size_t ws_bytes, mnx_stream_t stream);
+
+/* ------------------------------------------------------------------------ */
 /* Bond vectors diff[e] = pos[ei[e][1]] - pos[ei[e][0]] - shifts[e] (shifts  */
 /* may be NULL) for edge_index rows [sender, receiver], the reference's      */
 /* bond_diff = pos[target] - pos[source] (src/molix/data/tasks/              */

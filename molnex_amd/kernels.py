@@ -2268,6 +2268,35 @@ def _(a, weights, blocks, out_dim):
     return a.new_empty(a.shape[0], out_dim)
 
 
+@torch.library.custom_op("molix::block_linear_weight_grad", mutates_args=(), device_types="cuda")
+def block_linear_weight_grad(x: Tensor, g: Tensor, pairs: list[int], scales: list[float], numel: int) -> Tensor:
+    """The weight gradient of an ir_mul linear (``src/molrep/interaction/linear.py:43-105``), flat
+    ``(numel,)``: 8 integers per pair of an input and an output block (column, component step and
+    width in ``x``, the same in ``g``, components, first weight), every weight in exactly one pair.
+    No autograd of its own (``Linear`` supplies it)."""
+    _require_gpu("block_linear_weight_grad", x, g)
+    if x.dtype != torch.float32 or g.dtype != torch.float32 or x.dim() != 2 or g.dim() != 2 or x.shape[0] != g.shape[0]:
+        raise TypeError("block_linear_weight_grad: x and g must be float32 with the same rows")
+    n = len(scales)
+    if len(pairs) != 8 * n or sum(pairs[8 * i + 2] * pairs[8 * i + 5] for i in range(n)) != numel or any(
+            pairs[8 * i + 7] < 0 or pairs[8 * i + 7] + pairs[8 * i + 2] * pairs[8 * i + 5] > numel for i in range(n)):
+        raise ValueError("block_linear_weight_grad: the pairs do not cover the weights")
+    lib = _lib.load()
+    x, g = _aligned16(x), _aligned16(g)
+    gw = x.new_empty(numel)
+    desc = (C.c_int64 * max(8 * n, 1))(*pairs)
+    R, sx, sg = x.shape[0], x.shape[1], g.shape[1]
+    ws = _ws(lib.mnx_block_linear_wgrad_workspace_bytes(desc, n, sx, sg, R), x.device)
+    check(lib.mnx_block_linear_wgrad_f32(ptr(x), sx, ptr(g), sg, R, n, desc, (C.c_float * max(n, 1))(*scales), ptr(gw),
+                                         ptr(ws), ws.numel(), _stream(x)), "block_linear weight gradient")
+    return gw
+
+
+@block_linear_weight_grad.register_fake
+def _(x, g, pairs, scales, numel):
+    return x.new_empty(numel)
+
+
 @torch.library.custom_op("molix::class_groups", mutates_args=(), device_types="cuda")
 def _class_groups_op(classes: Tensor, num_classes: int) -> tuple[Tensor, Tensor]:
     lib = _lib.load()

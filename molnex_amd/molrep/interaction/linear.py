@@ -16,7 +16,7 @@ the HIP kernel ``mnx_block_linear_f32`` instead (fp32-accurate split-bf16 matrix
 place from the ir_mul input (no gather copy), the 1/sqrt(fan_in) scale is folded
 into the stacked weights and each output block is written directly; the input
 gradient is the same kernel on the output-gradient blocks with transposed
-weights.  Weight gradients (training) use the torch path below.
+weights.  Weight gradients (training) are one launch over every block pair (mnx_block_linear_wgrad_f32).
 """
 
 from __future__ import annotations
@@ -277,7 +277,12 @@ def _hip_plan(lin: "Linear"):
             sc_b.append(s_)
             off += i_.numel()
     cat = lambda xs, dt: torch.cat(xs).to(dt) if xs else torch.zeros(0, dtype=dt)
-    return {"fwd": K.block_linear_desc(fwd), "bwd": K.block_linear_desc(bwd), "idx_f": cat(idx_f, torch.long),
+    pairs, scales = [], []
+    for off_o, mul_o, d, srcs, fan_in in lin.plan:
+        for o, m, wo in srcs:
+            pairs += [o, m, m, off_o, mul_o, mul_o, d, wo]
+            scales.append(1.0 / math.sqrt(fan_in))
+    return {"pairs": (pairs, scales), "fwd": K.block_linear_desc(fwd), "bwd": K.block_linear_desc(bwd), "idx_f": cat(idx_f, torch.long),
             "sc_f": cat(sc_f, torch.float32), "idx_b": cat(idx_b, torch.long), "sc_b": cat(sc_b, torch.float32)}
 
 
@@ -302,8 +307,29 @@ class _HipBlockLinear(torch.autograd.Function):
         if need_x:
             gx = _HipBlockLinearT.apply(g, w, lin)
         if need_w:
-            _, gw = _block_backward(x, w, g, lin.plan, False, True)
+            gw = _HipWeightGrad.apply(x, g, lin)
         return gx, gw, None
+
+
+class _HipWeightGrad(torch.autograd.Function):
+    """gw = d<g, F(x, w)>/dw, every block pair in one HIP launch that reads ``x`` and ``g`` in place.
+    Bilinear: for a seed s on gw, <s, gw(x, g)> = <g, F(x, s)>, so its gradients are F^T(g, s) for x
+    and F(x, s) for g."""
+
+    @staticmethod
+    def forward(ctx, x, g, lin):
+        ctx.save_for_backward(x, g)
+        ctx.lin = lin
+        pairs, scales = lin._hip_plan["pairs"]
+        return torch.ops.molix.block_linear_weight_grad(x, g, pairs, scales, lin.weight_numel)
+
+    @staticmethod
+    def backward(ctx, s):
+        x, g = ctx.saved_tensors
+        need_x, need_g = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
+        s = s.contiguous()
+        return (_HipBlockLinearT.apply(g, s, ctx.lin) if need_x else None,
+                _HipBlockLinear.apply(x, s, ctx.lin) if need_g else None, None)
 
 
 class _HipBlockLinearT(torch.autograd.Function):
@@ -327,7 +353,7 @@ class _HipBlockLinearT(torch.autograd.Function):
         need_g, need_w = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         ggx = ggx.contiguous()
         dg = _HipBlockLinear.apply(ggx, w, lin) if need_g else None
-        dw = _block_backward(ggx, w, g, lin.plan, False, True)[1] if need_w else None
+        dw = _HipWeightGrad.apply(ggx, g, lin) if need_w else None
         return dg, dw, None
 
 
