@@ -445,6 +445,20 @@ int mnx_indexed_block_linear_f32(const float* a, int64_t a_stride, int32_t nseg,
                                  const int32_t* class_start, int32_t N, int64_t R, int32_t d, float* out,
                                  int64_t out_stride, int64_t out_off, int32_t out_comp, mnx_stream_t stream);
 
+/* All output blocks of a linear at once, with the weights as the module      */
+/* keeps them.  desc (host memory) holds per block out_off, out_comp, N, d,   */
+/* nseg and per segment col, comp, len, woff, ld; segment s contributes the   */
+/* contraction rows k = 0..len-1 with weights scale * w[woff + k*ld + n], or  */
+/* scale * w[woff + n*ld + k] with `transposed` (the input gradient), scale   */
+/* one factor per segment in order.  order / class_start / num_classes as     */
+/* above with the weights of consecutive classes w_class_stride floats apart  */
+/* (order NULL: one weight set).  Alignment as above; woff and, transposed,   */
+/* ld multiples of 4.  Arithmetic as above.                                   */
+int mnx_linear_blocks_f32(const float* a, int64_t a_stride, int64_t R, const float* w, int32_t transposed,
+                          int64_t w_class_stride, int32_t num_classes, const int32_t* order,
+                          const int32_t* class_start, int32_t nblocks, const int64_t* desc, const float* scale,
+                          float* out, int64_t out_stride, mnx_stream_t stream);
+
 /* ------------------------------------------------------------------------ */
 /* Weight gradient of a whole ir_mul linear (the cuet.Linear backward,        */
 /* src/molrep/interaction/linear.py:43-105): for each of npair pairs of an    */

@@ -89,6 +89,8 @@ SIGNATURES = {
                                         c_i32, vp]),
     "mnx_indexed_block_linear_f32": (C.c_int, [vp, c_i64, c_i32, vp, vp, vp, vp, c_i64, c_i32, vp, vp, c_i32,
                                                 c_i64, c_i32, vp, c_i64, c_i64, c_i32, vp]),
+    "mnx_linear_blocks_f32": (C.c_int, [vp, c_i64, c_i64, vp, c_i32, c_i64, c_i32, vp, vp, c_i32, vp, vp, vp, c_i64,
+                                        vp]),
     "mnx_block_linear_wgrad_workspace_bytes": (c_sz, [vp, c_i32, c_i64, c_i64, c_i64]),
     "mnx_block_linear_wgrad_f32": (C.c_int, [vp, c_i64, vp, c_i64, c_i64, c_i32, vp, vp, vp, vp, c_sz, vp]),
     "mnx_bond_vectors_f32": (C.c_int, [vp, c_i64, vp, vp, c_i64, vp, vp]),

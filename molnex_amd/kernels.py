@@ -2268,6 +2268,56 @@ def _(a, weights, blocks, out_dim):
     return a.new_empty(a.shape[0], out_dim)
 
 
+@torch.library.custom_op("molix::block_linear_weights", mutates_args=(), device_types="cuda")
+def block_linear_weights(a: Tensor, weight: Tensor, blocks: list[int], scales: list[float], out_dim: int,
+                         transposed: bool, order: Tensor | None = None, class_start: Tensor | None = None) -> Tensor:
+    """Every output block of an ir_mul linear in one launch, with the weights in the module's own
+    layout (``mnx_linear_blocks_f32``): ``blocks`` holds per output block ``out_off, mul, d, nseg`` and
+    per segment ``col, comp, len, w_off, w_ld``, ``scales`` one factor per segment; ``transposed``
+    reads the weights transposed (the input gradient).  With ``order`` / ``class_start``
+    (``class_groups``) ``weight`` is ``(S, numel)`` and each row takes its class's.  Every column of
+    the result must belong to exactly one block.  No autograd of its own (``Linear`` supplies it)."""
+    _require_gpu("block_linear_weights", a, weight, order, class_start)
+    indexed = order is not None
+    if a.dtype != torch.float32 or weight.dtype != torch.float32 or a.dim() != 2 or weight.dim() != (2 if indexed else 1):
+        raise TypeError("block_linear_weights: a must be float32 (R, dim_in) and the weights float32")
+    if indexed and (class_start is None or order.dtype != torch.int32 or class_start.dtype != torch.int32
+                    or order.shape[0] != a.shape[0] or class_start.shape[0] != weight.shape[0] + 2):
+        raise ValueError("block_linear_weights: order / class_start do not match the rows and classes")
+    x, w = _aligned16(a), _aligned16(weight)
+    R, dim_in = x.shape
+    numel = w.shape[-1]
+    desc, covered, nblk, i, nseg = [], 0, 0, 0, 0
+    while i < len(blocks):
+        off, mul, d, n = blocks[i:i + 4]
+        segs = [blocks[i + 4 + 5 * s:i + 9 + 5 * s] for s in range(n)]
+        i += 4 + 5 * n
+        if off < 0 or off + d * mul > out_dim or mul <= 0 or d <= 0:
+            raise ValueError("block_linear_weights: output block outside the result")
+        for col, comp, ln, wo, ld in segs:
+            last = wo + ((mul - 1) * ld + ln - 1 if transposed else (ln - 1) * ld + mul - 1)
+            if min(col, comp, wo, ld) < 0 or ln <= 0 or col + (d - 1) * comp + ln > dim_in or last >= numel:
+                raise ValueError("block_linear_weights: segment outside the rows or the weights")
+        desc += [off, mul, mul, d, n] + [v for s in segs for v in s]
+        covered += d * mul
+        nblk += 1
+        nseg += n
+    if covered != out_dim or i != len(blocks) or nseg != len(scales):
+        raise ValueError("block_linear_weights: output blocks do not cover the result")
+    out = x.new_empty(R, out_dim)
+    order_, start_ = (order.contiguous(), class_start.contiguous()) if indexed else (None, None)
+    check(_lib.load().mnx_linear_blocks_f32(
+        ptr(x), dim_in, R, ptr(w), int(transposed), numel if indexed else 0, w.shape[0] if indexed else 0, ptr(order_),
+        ptr(start_), nblk, (C.c_int64 * max(len(desc), 1))(*desc), (C.c_float * max(nseg, 1))(*scales), ptr(out), out_dim,
+        _stream(x)), "block_linear")
+    return out
+
+
+@block_linear_weights.register_fake
+def _(a, weight, blocks, scales, out_dim, transposed, order=None, class_start=None):
+    return a.new_empty(a.shape[0], out_dim)
+
+
 @torch.library.custom_op("molix::block_linear_weight_grad", mutates_args=(), device_types="cuda")
 def block_linear_weight_grad(x: Tensor, g: Tensor, pairs: list[int], scales: list[float], numel: int) -> Tensor:
     """The weight gradient of an ir_mul linear (``src/molrep/interaction/linear.py:43-105``), flat

@@ -12,11 +12,11 @@ the GPU through torch.mm (hipBLASLt); forward and backward are written out so
 every gradient slice is produced once.
 
 On the GPU (float32, multiplicities that are multiples of 8) the blocks run in
-the HIP kernel ``mnx_block_linear_f32`` instead (fp32-accurate split-bf16 matrix-core products): rows (node, m) are read in
-place from the ir_mul input (no gather copy), the 1/sqrt(fan_in) scale is folded
-into the stacked weights and each output block is written directly; the input
-gradient is the same kernel on the output-gradient blocks with transposed
-weights.  Weight gradients (training) are one launch over every block pair (mnx_block_linear_wgrad_f32).
+the HIP kernel ``mnx_linear_blocks_f32`` instead (fp32-accurate split-bf16 matrix-core products), all of them
+in one launch: rows (node, m) are read in place from the ir_mul input (no gather copy), the
+weights where the parameter lies, scaled by 1/sqrt(fan_in) on the way, and each output block is
+written directly; the input gradient is the same kernel on the output-gradient blocks with the
+weights read transposed.  Weight gradients (training) are one launch over every block pair (mnx_block_linear_wgrad_f32).
 """
 
 from __future__ import annotations
@@ -73,10 +73,8 @@ class Linear(nn.Module):
         return self._hip_plan is not None
 
     def _setup_hip(self) -> None:
-        """Launch lists and fragment-order weight tables of the HIP block kernel, for shapes it
-        takes: every multiplicity a multiple of 8, at most 8 source blocks per output block and 8
-        consumers per input block.  The tables are non-persistent buffers, so they follow the
-        module's device and appear as constants when the module is traced."""
+        """Launch lists of the HIP block kernel, for shapes it takes: every multiplicity a multiple
+        of 8, at most 8 source blocks per output block and 8 consumers per input block."""
         ok = all(b.mul % 8 == 0 for b in self.irreps_in) and all(o.mul % 8 == 0 for o in self.irreps_out)
         users = {}
         for _, _, _, srcs, _ in self.plan:
@@ -85,8 +83,16 @@ class Linear(nn.Module):
                 users[o] = users.get(o, 0) + 1
         ok = ok and all(c <= 8 for c in users.values())
         self._hip_plan = _hip_plan(self) if ok else None
-        for name in ("idx_f", "sc_f", "idx_b", "sc_b"):
-            self.register_buffer("_hip_" + name, self._hip_plan.pop(name) if ok else None, persistent=False)
+
+    # the gather indices and scales that put ``weight`` into the fragment order of
+    # ``molix::block_linear`` (forward), for callers of that op
+    @property
+    def _hip_idx_f(self) -> torch.Tensor:
+        return _fragments(self)[0].to(self.weight.device)
+
+    @property
+    def _hip_sc_f(self) -> torch.Tensor:
+        return _fragments(self)[1].to(self.weight.device)
 
     def forward(self, x: torch.Tensor, weight: torch.Tensor | None = None,
                 weight_indices: torch.Tensor | None = None) -> torch.Tensor:
@@ -199,6 +205,12 @@ def _lin_tiles(N: int) -> int:
     return 4 if N >= 128 else -(-N // 32)
 
 
+def _frag_floats(K: int, N: int) -> int:
+    """Length of ``_frag_order`` (``mnx_block_linear_frag_floats``)."""
+    nt = _lin_tiles(N)
+    return -(-N // (nt * 32)) * -(-K // 64) * 4 * nt * 64 * 8
+
+
 def _frag_order(K: int, N: int):
     """(k, c, valid) of every element of the kernel's weight layout
     [column group][64-row chunk][k/16][tile][lane][8] (csrc/linear.hip): lane l of k-step q
@@ -239,51 +251,50 @@ def _frag_block(rows, N):
     return idx, sc
 
 
-def _hip_plan(lin: "Linear"):
-    """Launch descriptors and fragment-ordered weight indices for the HIP block kernel.
+def _fragments(lin: "Linear"):
+    """Gather indices and scales of the forward weights in ``molix::block_linear``'s fragment order."""
+    idx, sc = [], []
+    for _, mul_o, _, srcs, fan_in in lin.plan:
+        if srcs:
+            i_, s_ = _frag_block([(m, wo, mul_o, 1, 1.0 / math.sqrt(fan_in)) for _, m, wo in srcs], mul_o)
+            idx.append(i_)
+            sc.append(s_)
+    cat = lambda xs, dt: torch.cat(xs).to(dt) if xs else torch.zeros(0, dtype=dt)
+    return cat(idx, torch.long), cat(sc, torch.float32)
 
-    fwd: per output block (out offset, mul_o, d, segments [(col, comp, len)], float offset of its
-    weights); the weights are w[idx_f] * scale_f with the stacked source weights (sum of source
-    muls) x mul_o in the kernel's fragment order.
-    bwd: per input block (in offset, mul, d, segments over the output-gradient blocks, offset);
-    weights w[idx_b] * scale_b: the transposed blocks, (sum of consumer mul_o) x mul."""
-    fwd, idx_f, sc_f, off = [], [], [], 0
-    consumers = {}
+
+def _hip_plan(lin: "Linear"):
+    """Launch lists of the HIP block kernel.
+
+    rows: ``molix::block_linear_weights`` forward -- per output block (out offset, mul_o, d, segments
+    over its source blocks (col, comp, len, weight offset, weight row step)) and the segments'
+    1/sqrt(fan_in).
+    cols: the same per input block over the output-gradient blocks, weights transposed.
+    pairs: the (input, output) block pairs of the weight gradient.
+    fwd: the forward launch list of ``molix::block_linear`` (fragment-ordered weights)."""
+    rows, srow, fwd, off, consumers, pairs, spair = [], [], [], 0, {}, [], []
     for off_o, mul_o, d, srcs, fan_in in lin.plan:
         s = 1.0 / math.sqrt(fan_in) if srcs else 0.0
-        segs, rows = [], []
+        rows += [off_o, mul_o, d, len(srcs)]
         for o, m, wo in srcs:
-            segs.append((o, m, m))
-            rows.append((m, wo, mul_o, 1, s))  # W_src[c][p] = w[wo + c * mul_o + p]
+            rows += [o, m, m, wo, mul_o]
+            srow.append(s)
             consumers.setdefault(o, []).append((off_o, mul_o, wo, s))
-        fwd.append((off_o, mul_o, d, segs, off))
-        if segs:
-            i_, s_ = _frag_block(rows, mul_o)
-            idx_f.append(i_)
-            sc_f.append(s_)
-            off += i_.numel()
-    bwd, idx_b, sc_b, off = [], [], [], 0
-    in_off = lin.irreps_in.offsets()
-    for ib, b in enumerate(lin.irreps_in):
-        o, m, d = in_off[ib], b.mul, b.ir.dim
-        segs, rows = [], []
-        for off_o, mul_o, wo, s in consumers.get(o, []):
-            segs.append((off_o, mul_o, mul_o))
-            rows.append((mul_o, wo, 1, mul_o, s))  # W^T[p][c] = w[wo + c * mul_o + p]
-        bwd.append((o, m, d, segs, off))
-        if segs:
-            i_, s_ = _frag_block(rows, m)
-            idx_b.append(i_)
-            sc_b.append(s_)
-            off += i_.numel()
-    cat = lambda xs, dt: torch.cat(xs).to(dt) if xs else torch.zeros(0, dtype=dt)
-    pairs, scales = [], []
-    for off_o, mul_o, d, srcs, fan_in in lin.plan:
-        for o, m, wo in srcs:
             pairs += [o, m, m, off_o, mul_o, mul_o, d, wo]
-            scales.append(1.0 / math.sqrt(fan_in))
-    return {"pairs": (pairs, scales), "fwd": K.block_linear_desc(fwd), "bwd": K.block_linear_desc(bwd), "idx_f": cat(idx_f, torch.long),
-            "sc_f": cat(sc_f, torch.float32), "idx_b": cat(idx_b, torch.long), "sc_b": cat(sc_b, torch.float32)}
+            spair.append(s)
+        fwd.append((off_o, mul_o, d, [(o, m, m) for o, m, _ in srcs], off))
+        if srcs:
+            off += _frag_floats(sum(m for _, m, _ in srcs), mul_o)
+    # input blocks with the same consumers next to each other: they read the same gradient rows
+    cols, scol = [], []
+    in_off = lin.irreps_in.offsets()
+    blocks = [(in_off[i], b.mul, b.ir.dim, consumers.get(in_off[i], [])) for i, b in enumerate(lin.irreps_in)]
+    for o, m, d, users in sorted(blocks, key=lambda b: [u[0] for u in b[3]]):
+        cols += [o, m, d, len(users)]
+        for off_o, mul_o, wo, s in users:
+            cols += [off_o, mul_o, mul_o, wo, mul_o]
+            scol.append(s)
+    return {"rows": (rows, srow), "cols": (cols, scol), "pairs": (pairs, spair), "fwd": K.block_linear_desc(fwd)}
 
 
 class _HipBlockLinear(torch.autograd.Function):
@@ -291,8 +302,7 @@ class _HipBlockLinear(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w, lin):
-        ws = w.index_select(0, lin._hip_idx_f.to(w.device)) * lin._hip_sc_f.to(w.device)
-        out = torch.ops.molix.block_linear(x, ws, lin._hip_plan["fwd"], lin.irreps_out.dim)
+        out = torch.ops.molix.block_linear_weights(x, w, *lin._hip_plan["rows"], lin.irreps_out.dim, False)
         ctx.save_for_backward(x, w)
         ctx.lin = lin
         return out
@@ -340,8 +350,7 @@ class _HipBlockLinearT(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, g, w, lin):
-        wb = w.index_select(0, lin._hip_idx_b.to(w.device)) * lin._hip_sc_b.to(w.device)
-        gx = torch.ops.molix.block_linear(g, wb, lin._hip_plan["bwd"], lin.irreps_in.dim)
+        gx = torch.ops.molix.block_linear_weights(g, w, *lin._hip_plan["cols"], lin.irreps_in.dim, True)
         ctx.save_for_backward(g, w)
         ctx.lin = lin
         return gx
@@ -388,9 +397,7 @@ class _HipIndexedLinear(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, weight, groups, idx, lin):
-        ws = weight.index_select(1, lin._hip_idx_f.to(weight.device)) * lin._hip_sc_f.to(weight.device)
-        out = torch.ops.molix.indexed_block_linear(x, ws.contiguous(), *groups, lin._hip_plan["fwd"],
-                                                   lin.irreps_out.dim)
+        out = torch.ops.molix.block_linear_weights(x, weight, *lin._hip_plan["rows"], lin.irreps_out.dim, False, *groups)
         ctx.save_for_backward(x, weight, idx)
         ctx.groups, ctx.lin = groups, lin
         return out
@@ -411,9 +418,7 @@ class _HipIndexedLinearT(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, g, weight, groups, idx, lin):
-        wb = weight.index_select(1, lin._hip_idx_b.to(weight.device)) * lin._hip_sc_b.to(weight.device)
-        gx = torch.ops.molix.indexed_block_linear(g, wb.contiguous(), *groups, lin._hip_plan["bwd"],
-                                                  lin.irreps_in.dim)
+        gx = torch.ops.molix.block_linear_weights(g, weight, *lin._hip_plan["cols"], lin.irreps_in.dim, True, *groups)
         ctx.save_for_backward(g, weight, idx)
         ctx.groups, ctx.lin = groups, lin
         return gx
