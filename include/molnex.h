@@ -54,6 +54,7 @@ int mnx_abi_version(void);
 #define MNX_NLIST_COMPACT 0    /* pairs sorted by (i, j) at slots 0..total-1 */
 #define MNX_NLIST_TRIANGULAR 1 /* HALF only: pair (i, j) at slot i*(i-1)/2 + j
                                   (reference max_num_pairs == -1 layout) */
+#define MNX_NLIST_EXACT 2      /* COMPACT with capacity == total: nothing to pad */
 
 size_t mnx_nlist_workspace_bytes(int64_t num_atoms);
 

@@ -12,17 +12,35 @@
 // Output is sorted by (i, j) like the CPU enumeration order (.cpp:38-43), which
 // the CUDA reference does not guarantee (atomicAdd slots, .cu:69).
 //
-// Layout of the work: atoms are binned into cells whose slab widths exceed the
-// cutoff (fractional coordinates for periodic cells), each cell's atoms sorted by
-// id.  Four wavefronts share a cell (each takes every fourth atom of it as a
-// centre): they fetch the 27 neighbour cells' ranges in one round trip, load each
-// candidate once and test it against all of their centres (count pass: a screening
-// distance on positions moved into the primary cell, the reference arithmetic near
-// the cutoff; the accept ballots are kept), then the emit pass compacts the accepted
-// j of each centre from the ballots into LDS, sorts them in registers (bitonic,
-// <= 64) or by rank, and writes each centre's segment with coalesced stores.  Grids with
-// fewer than 3 cells along a periodic axis use one wavefront per atom over all
-// atoms (brute mode).  This translation unit is compiled with -ffp-contract=off.
+// Layout of the work.  Up to kNlSmall atoms: one wavefront per atom tests all
+// the others in id order and keeps the accept ballots, one workgroup scans the
+// counts, and the emit expands the ballots, already in (i, j) order: three
+// launches and the host's read of the count.
+//
+// Above that, a cell list.  Atoms are binned into cells whose slab widths exceed
+// the cutoff (fractional coordinates for periodic cells); a cell's atoms take a
+// run of the cell-ordered arrays in whatever order they arrive (nothing that is
+// written depends on it).  A workgroup takes a cell: its four wavefronts stage the
+// atoms of the 27 neighbour cells in LDS (wrapped next to the cell), then each
+// tests them against every fourth atom of the cell as a centre, whose position is
+// wave-uniform (a screening distance on positions moved into the primary cell, the
+// reference arithmetic near the cutoff), appends the accepted j to the centre's
+// list in LDS, sorts it in registers (bitonic) and leaves it in the centre's row of
+// kSlots entries in the workspace.  The emit then is a stream: half a wavefront per
+// atom reads its sorted row and writes the pairs, the vectors through LDS so that
+// every store is contiguous.  Atoms with more than kSlots neighbours, and grids
+// with fewer than 3 cells along a periodic axis (all-pairs scan), are listed and
+// sorted by the emit itself.  This translation unit is compiled with
+// -ffp-contract=off.
+//
+// Bound by the candidate tests and launches, not by its 36 bytes per pair:
+// 100k atoms, 5.24 M ordered pairs (189 MB written): 206 us in all, the count
+// pass 85 us (1100 vector and as many scalar instructions per wavefront: the
+// tests, the sort and each cell's set-up), the emit 68 us (2.8 TB/s), five binning
+// and scan launches and the host's read of the total the rest; 283 us with a
+// sorting emit behind accept ballots (130 us), a second sort inside the cells and
+// 18 launches.  96 atoms: 49 us (three launches of 3 us, the host's calls and its
+// read of the total), 116 us through the cell list.
 
 #include <math.h>
 
@@ -34,14 +52,15 @@
 namespace mnx {
 namespace {
 
-constexpr int kNlCap = 4096;  // max neighbours of one atom (LDS list of the per-atom emit)
-constexpr int kEmitBuf = 1024; // LDS list per wavefront of the cell emit; atoms with more
-                               // neighbours are written by the per-atom emit
-constexpr int64_t kNlBlocks = 16384;  // grid-stride launches of the count / emit kernels
-constexpr int kCellParts = 4;          // wavefronts per cell (each takes every 4th atom of it)
-constexpr int kMaskChunks = 16;        // acceptance masks kept per centre: 16 x 64 candidates; cells
-                                       // with more candidates are tested again by the emit
-constexpr int kPreChunks = 8;          // candidate chunks a cell unit loads into registers at once
+constexpr int kNlSmall = 2048;  // atoms of the all-pairs path (its lists hold 16-bit ids; where both were
+                                // timed the cell list passes it at about this size)
+constexpr int kNlCap = 4096;   // max neighbours of one atom
+constexpr int kSlots = 128;    // sorted neighbours kept per atom by the count pass
+constexpr int kMidCap = 1024;  // LDS list per wavefront of the emit for atoms with more
+constexpr int kCand = 512;     // candidates staged in LDS at once (394 on average at liquid density, cells of 5 A)
+constexpr int kCentres = 4;    // centres whose lists a wavefront holds in LDS at once
+constexpr int kParts = 4;      // wavefronts per cell (each takes every 4th atom of it)
+constexpr int64_t kNlBlocks = 8192;  // grid-stride launch of the count pass
 constexpr float kCellMargin = 1.0001f;
 
 struct NlGrid {
@@ -50,13 +69,17 @@ struct NlGrid {
     int32_t n[3];
     int32_t ncells;
     int32_t overflow;  // set when an atom has more than kNlCap neighbours
-    int32_t nbig;      // atoms with more than kEmitBuf neighbours (listed in NlWs::big)
+    int32_t nbig;      // atoms with more than kMidCap neighbours (listed from the end of NlWs::big)
+    int32_t nmid;      // atoms with more than kSlots, at most kMidCap neighbours (from its front)
+    int32_t filled;    // cell-ordered slots handed out
+    uint64_t lo_key[3], hi_key[3];  // bounding box of an open system, as ordered integers
     double lo[3];
     double inv_w[3];
     double rinv[6];  // inverse of the lower-triangular cell: f_c = z*r5, ...
 };
 
-// Position moved into the primary cell, in cell order (screening test of the count pass).
+// Position moved into the primary cell, in cell order (screening test of the count pass);
+// w carries nothing.
 template <typename T>
 struct alignas(4 * sizeof(T)) PosW {
     T x, y, z, w;
@@ -65,18 +88,17 @@ struct alignas(4 * sizeof(T)) PosW {
 struct NlWs {
     NlGrid* grid;
     int32_t* cell_of;
+    int32_t* rank;  // arrival number of the atom in its cell
     int32_t* cell_count;
     int32_t* cell_start;
-    int32_t* cell_fill;
     int32_t* atoms_sorted;
     int32_t* counts;
     int32_t* big;
-    uint64_t* masks;  // per centre: the count pass's accept ballot of each 64-candidate chunk
+    int32_t* slots;   // [n][kSlots]: an atom's neighbours, ascending
+    uint64_t* masks;  // small systems: [n][words] accept ballots
     void* posw;       // PosW<T> per cell-ordered slot
     int64_t* offsets;
-    int64_t* total;
     int64_t* tiles64;
-    int32_t* tiles32;
     int64_t max_cells;
 };
 
@@ -84,22 +106,24 @@ int64_t max_cells_for(int64_t n) { return 2 * n + 64; }
 
 NlWs carve(void* base, size_t bytes, int64_t n, size_t* used) {
     Workspace ws{static_cast<char*>(base), bytes};
-    NlWs w;
+    NlWs w{};
     w.max_cells = max_cells_for(n);
-    w.grid = ws.take<NlGrid>(1);
-    w.cell_of = ws.take<int32_t>(n > 0 ? n : 1);
-    w.cell_count = ws.take<int32_t>(w.max_cells);
-    w.cell_start = ws.take<int32_t>(w.max_cells + 1);
-    w.cell_fill = ws.take<int32_t>(w.max_cells);
-    w.atoms_sorted = ws.take<int32_t>(n > 0 ? n : 1);
-    w.counts = ws.take<int32_t>(n > 0 ? n : 1);
-    w.big = ws.take<int32_t>(n > 0 ? n : 1);
-    w.masks = ws.take<uint64_t>(size_t(n > 0 ? n : 1) * kMaskChunks);
-    w.posw = ws.take<PosW<double>>(n > 0 ? n : 1);
     w.offsets = ws.take<int64_t>(n + 1);
-    w.total = ws.take<int64_t>(1);
-    w.tiles64 = ws.take<int64_t>(scan_workspace_elems(n));
-    w.tiles32 = ws.take<int32_t>(scan_workspace_elems(w.max_cells));
+    w.counts = ws.take<int32_t>(n > 0 ? n : 1);
+    if (n <= kNlSmall) {
+        w.masks = ws.take<uint64_t>(size_t(n > 0 ? n : 1) * ((n + kWave - 1) / kWave + 1));
+    } else {
+        w.grid = ws.take<NlGrid>(1);
+        w.cell_of = ws.take<int32_t>(n);
+        w.rank = ws.take<int32_t>(n);
+        w.cell_count = ws.take<int32_t>(w.max_cells);
+        w.cell_start = ws.take<int32_t>(w.max_cells);
+        w.atoms_sorted = ws.take<int32_t>(n);
+        w.big = ws.take<int32_t>(n);
+        w.slots = ws.take<int32_t>(size_t(n) * kSlots);
+        w.posw = ws.take<PosW<double>>(n);
+        w.tiles64 = ws.take<int64_t>(scan_workspace_elems(n));
+    }
     *used = ws.used;
     return w;
 }
@@ -122,6 +146,20 @@ __device__ __forceinline__ double rint_(double a) { return rint(a); }
 __device__ __forceinline__ float sqrt_(float a) { return sqrtf(a); }
 __device__ __forceinline__ double sqrt_(double a) { return sqrt(a); }
 
+// rint(d / b), with 1 / b approximately inv: the product decides it except within 1e-3 (and its own
+// rounding) of a half-way point, where the quotient is formed.
+__device__ __forceinline__ float fabs_(float a) { return fabsf(a); }
+__device__ __forceinline__ double fabs_(double a) { return fabs(a); }
+__device__ __forceinline__ float rcp_(float a) { return __builtin_amdgcn_rcpf(a); }
+__device__ __forceinline__ double rcp_(double a) { return 1.0 / a; }
+template <typename T>
+__device__ __forceinline__ T rint_quotient(T d, T b, T inv) {
+    const T t = d * inv;
+    T s = rint_(t);
+    if (!(fabs_(t - s) < T(0.499) - fabs_(t) * T(1e-6))) s = rint_(d / b);
+    return s;
+}
+
 // Minimum image and distance of the difference vector d, the reference's arithmetic.
 template <typename T>
 __device__ __forceinline__ void geo_from_d(const T* __restrict__ box, T d0, T d1, T d2, bool periodic, bool want_shift,
@@ -131,7 +169,7 @@ __device__ __forceinline__ void geo_from_d(const T* __restrict__ box, T d0, T d1
 #pragma unroll
         for (int k = 2; k >= 0; --k) {
             const T dk = k == 2 ? d2 : (k == 1 ? d1 : d0);
-            const T s = rint_(dk / box[4 * k]);
+            const T s = rint_quotient(dk, box[4 * k], rcp_(box[4 * k]));
             const T b0 = s * box[3 * k + 0], b1 = s * box[3 * k + 1], b2 = s * box[3 * k + 2];
             d0 = d0 - b0;
             d1 = d1 - b1;
@@ -255,34 +293,19 @@ __device__ __forceinline__ bool accept(const T* pos, const T* box, int i, int j,
 // Grid set-up and binning
 // ---------------------------------------------------------------------------
 
+// Ordered integers of doubles (bounding box by integer atomics).
+__device__ __forceinline__ uint64_t to_key(double v) {
+    const uint64_t b = uint64_t(__double_as_longlong(v));
+    return b >> 63 ? ~b : b | (uint64_t(1) << 63);
+}
+__device__ __forceinline__ double from_key(uint64_t k) {
+    return __longlong_as_double((long long)(k >> 63 ? k & ~(uint64_t(1) << 63) : ~k));
+}
+
+// The cell grid of box (or of an open system's bounding box, from gp).
 template <typename T>
-__global__ void __launch_bounds__(1024) k_grid_setup(const T* __restrict__ pos, int64_t n, const T* __restrict__ box,
-                                                     double cutoff, int64_t max_cells, NlGrid* __restrict__ grid) {
-    __shared__ double smin[3][1024], smax[3][1024];
-    const int t = threadIdx.x;
-    double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
-    if (!box) {
-        for (int64_t i = t; i < n; i += 1024)
-            for (int k = 0; k < 3; ++k) {
-                double v = double(pos[3 * i + k]);
-                mn[k] = fmin(mn[k], v);
-                mx[k] = fmax(mx[k], v);
-            }
-    }
-    for (int k = 0; k < 3; ++k) {
-        smin[k][t] = mn[k];
-        smax[k][t] = mx[k];
-    }
-    __syncthreads();
-    for (int off = 512; off > 0; off >>= 1) {
-        if (t < off)
-            for (int k = 0; k < 3; ++k) {
-                smin[k][t] = fmin(smin[k][t], smin[k][t + off]);
-                smax[k][t] = fmax(smax[k][t], smax[k][t + off]);
-            }
-        __syncthreads();
-    }
-    if (t != 0) return;
+__device__ NlGrid make_grid(int64_t n, const T* __restrict__ box, double cutoff, int64_t max_cells,
+                            const NlGrid* __restrict__ gp) {
     NlGrid g{};
     const double cw = cutoff * double(kCellMargin) + 1e-12;
     if (box) {
@@ -311,7 +334,7 @@ __global__ void __launch_bounds__(1024) k_grid_setup(const T* __restrict__ pos, 
     } else {
         g.periodic = 0;
         for (int k = 0; k < 3; ++k) {
-            double lo = n > 0 ? smin[k][0] : 0.0, hi = n > 0 ? smax[k][0] : 0.0;
+            double lo = n > 0 ? from_key(gp->lo_key[k]) : 0.0, hi = n > 0 ? from_key(gp->hi_key[k]) : 0.0;
             double ext = hi - lo;
             double m = floor(ext / cw);
             g.n[k] = m < 1 ? 1 : (m > 1024 ? 1024 : int(m));
@@ -322,13 +345,62 @@ __global__ void __launch_bounds__(1024) k_grid_setup(const T* __restrict__ pos, 
             g.n[kmax] = (g.n[kmax] + 1) / 2;
         }
         for (int k = 0; k < 3; ++k) {
-            double ext = (n > 0 ? smax[k][0] : 0.0) - g.lo[k];
+            double ext = (n > 0 ? from_key(gp->hi_key[k]) : 0.0) - g.lo[k];
             g.inv_w[k] = ext > 0 ? double(g.n[k]) / ext : 0.0;
         }
         g.brute = 0;
     }
     g.ncells = g.brute ? 1 : g.n[0] * g.n[1] * g.n[2];
-    *grid = g;
+    return g;
+}
+
+
+// Zeroes the cell counters; the first thread sets up the grid of a periodic system (an open one
+// waits for its bounding box).
+template <typename T>
+__global__ void __launch_bounds__(256) k_nl_clear(int32_t* __restrict__ cell_count, int64_t n, const T* __restrict__ box,
+                                                  double cutoff, int64_t max_cells, NlGrid* __restrict__ gp) {
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < max_cells) cell_count[i] = 0;
+    if (i) return;
+    if (box) {
+        *gp = make_grid<T>(n, box, cutoff, max_cells, nullptr);
+    } else {
+        NlGrid g{};
+        for (int k = 0; k < 3; ++k) {
+            g.lo_key[k] = to_key(1e300);
+            g.hi_key[k] = to_key(-1e300);
+        }
+        *gp = g;
+    }
+}
+
+// Bounding box of an open system (NaN coordinates left out).
+template <typename T>
+__global__ void __launch_bounds__(256) k_nl_bounds(const T* __restrict__ pos, int64_t n, NlGrid* __restrict__ gp) {
+    double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
+    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x)
+        for (int k = 0; k < 3; ++k) {
+            const double v = double(pos[3 * i + k]);
+            mn[k] = fmin(mn[k], v);
+            mx[k] = fmax(mx[k], v);
+        }
+    for (int k = 0; k < 3; ++k) {
+        for (int o = 32; o > 0; o >>= 1) {
+            mn[k] = fmin(mn[k], __shfl_xor(mn[k], o, kWave));
+            mx[k] = fmax(mx[k], __shfl_xor(mx[k], o, kWave));
+        }
+        if ((threadIdx.x & (kWave - 1)) == 0) {
+            atomicMin(reinterpret_cast<unsigned long long*>(&gp->lo_key[k]), (unsigned long long)to_key(mn[k]));
+            atomicMax(reinterpret_cast<unsigned long long*>(&gp->hi_key[k]), (unsigned long long)to_key(mx[k]));
+        }
+    }
+}
+
+template <typename T>
+__global__ void k_nl_open_grid(int64_t n, double cutoff, int64_t max_cells, NlGrid* __restrict__ gp) {
+    const NlGrid g = make_grid<T>(n, nullptr, cutoff, max_cells, gp);
+    *gp = g;
 }
 
 template <typename T>
@@ -355,46 +427,57 @@ __device__ __forceinline__ void cell_coords(const T* pos, int64_t i, const NlGri
 
 template <typename T>
 __global__ void k_bin(const T* __restrict__ pos, int64_t n, const NlGrid* __restrict__ gp, int32_t* __restrict__ cell_of,
-                      int32_t* __restrict__ cell_count) {
+                      int32_t* __restrict__ rank, int32_t* __restrict__ cell_count) {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const NlGrid g = *gp;
-    int cid = 0;
-    if (!g.brute) {
-        int c[3];
-        cell_coords<T>(pos, i, g, c);
-        cid = (c[2] * g.n[1] + c[1]) * g.n[0] + c[0];
-    }
+    if (g.brute) return;  // no cells
+    int c[3];
+    cell_coords<T>(pos, i, g, c);
+    const int cid = (c[2] * g.n[1] + c[1]) * g.n[0] + c[0];
     cell_of[i] = cid;
-    atomicAdd(&cell_count[cid], 1);
+    rank[i] = atomicAdd(&cell_count[cid], 1);
 }
 
-__global__ void k_place(int64_t n, const int32_t* __restrict__ cell_of, const int32_t* __restrict__ cell_start,
-                        int32_t* __restrict__ cell_fill, int32_t* __restrict__ atoms_sorted) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int cid = cell_of[i];
-    const int slot = cell_start[cid] + atomicAdd(&cell_fill[cid], 1);
-    atoms_sorted[slot] = int32_t(i);
+// Each cell's run of the cell-ordered arrays: contiguous in cell order within a workgroup's 2048
+// cells, the workgroups' runs in the order they arrive.
+__global__ void __launch_bounds__(kScanThreads) k_cell_runs(NlGrid* __restrict__ gp,
+                                                            const int32_t* __restrict__ cell_count,
+                                                            int32_t* __restrict__ cell_start) {
+    __shared__ int32_t sh[kScanThreads];
+    __shared__ int32_t s_base;
+    const int ncells = gp->brute ? 0 : gp->ncells;
+    const int base = int(blockIdx.x) * kScanTile + int(threadIdx.x) * kScanItems;
+    if (int(blockIdx.x) * kScanTile >= ncells) return;
+    int32_t v[kScanItems], sum = 0, total;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        v[k] = base + k < ncells ? cell_count[base + k] : 0;
+        sum += v[k];
+    }
+    int32_t run = block_exclusive_scan<int32_t>(sum, sh, &total);
+    if (threadIdx.x == 0) s_base = atomicAdd(&gp->filled, total);
+    __syncthreads();
+    run += s_base;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        if (base + k < ncells) cell_start[base + k] = run;
+        run += v[k];
+    }
 }
 
-// Each cell's atom list in ascending order (deterministic after the atomic placement into
-// `slots`): the atom in slot k moves to its rank within its cell.  The same slot of `posw`
-// receives the atom's position moved into the primary cell (by whole box vectors, from the
-// fractional coordinates that binned it), which the count pass's screening test reads.
+// Each atom into its slot of the cell order, with its position moved into the primary cell (by
+// whole box vectors, from the fractional coordinates that binned it), which the count pass's
+// screening test reads.
 template <typename T>
-__global__ void k_rank_cells(int64_t n, const T* __restrict__ pos, const T* __restrict__ box,
-                             const NlGrid* __restrict__ gp, const int32_t* __restrict__ cell_of,
-                             const int32_t* __restrict__ cell_start, const int32_t* __restrict__ slots,
-                             int32_t* __restrict__ atoms_sorted, PosW<T>* __restrict__ posw) {
-    const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const int a = slots[k];
-    const int c = cell_of[a];
-    const int b = cell_start[c], e = cell_start[c + 1];
-    int r = 0;
-    for (int t = b; t < e; ++t) r += slots[t] < a;
-    atoms_sorted[b + r] = a;
+__global__ void k_place(int64_t n, const T* __restrict__ pos, const T* __restrict__ box,
+                        const NlGrid* __restrict__ gp, const int32_t* __restrict__ cell_of,
+                        const int32_t* __restrict__ rank, const int32_t* __restrict__ cell_start,
+                        int32_t* __restrict__ atoms_sorted, PosW<T>* __restrict__ posw) {
+    const int64_t a = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (a >= n || gp->brute) return;
+    const int slot = cell_start[cell_of[a]] + rank[a];
+    atoms_sorted[slot] = int32_t(a);
     const double x = pos[3 * a], y = pos[3 * a + 1], z = pos[3 * a + 2];
     PosW<T> p;
     if (gp->periodic) {
@@ -413,7 +496,7 @@ __global__ void k_rank_cells(int64_t n, const T* __restrict__ pos, const T* __re
         p.z = T(z);
     }
     p.w = T(0);
-    posw[b + r] = p;
+    posw[slot] = p;
 }
 
 // ---------------------------------------------------------------------------
@@ -428,22 +511,24 @@ struct CellRanges {
 };
 
 __device__ __forceinline__ CellRanges cell_ranges(const NlGrid& g, int cx, int cy, int cz,
-                                                  const int32_t* __restrict__ cell_start, int lane) {
+                                                  const int32_t* __restrict__ cell_start,
+                                                  const int32_t* __restrict__ cell_count, int lane) {
     CellRanges cr{0, 0, 0, 0};
     if (lane < 27) {
         int z = cz + lane / 9 - 1, y = cy + (lane / 3) % 3 - 1, x = cx + lane % 3 - 1;
         bool in = true;
         if (g.periodic) {
-            z = (z + g.n[2]) % g.n[2];
-            y = (y + g.n[1]) % g.n[1];
-            x = (x + g.n[0]) % g.n[0];
+            // one step outside at most
+            z += z < 0 ? g.n[2] : (z >= g.n[2] ? -g.n[2] : 0);
+            y += y < 0 ? g.n[1] : (y >= g.n[1] ? -g.n[1] : 0);
+            x += x < 0 ? g.n[0] : (x >= g.n[0] ? -g.n[0] : 0);
         } else {
             in = z >= 0 && z < g.n[2] && y >= 0 && y < g.n[1] && x >= 0 && x < g.n[0];
         }
         if (in) {
             const int cid = (z * g.n[1] + y) * g.n[0] + x;
             cr.rb = cell_start[cid];
-            cr.rlen = cell_start[cid + 1] - cr.rb;
+            cr.rlen = cell_count[cid];
         }
     }
     int incl = cr.rlen;  // lanes >= 27 add 0
@@ -474,6 +559,7 @@ __device__ __forceinline__ int cell_candidate(const CellRanges& cr, int k, const
 template <typename T, typename F>
 __device__ __forceinline__ void for_candidates(const T* pos, int i, int64_t n, const NlGrid& g,
                                                const int32_t* __restrict__ cell_start,
+                                               const int32_t* __restrict__ cell_count,
                                                const int32_t* __restrict__ atoms_sorted, int mode, F&& f) {
     const int lane = threadIdx.x & (kWave - 1);
     if (g.brute) {
@@ -486,7 +572,7 @@ __device__ __forceinline__ void for_candidates(const T* pos, int i, int64_t n, c
     }
     int c[3];
     cell_coords<T>(pos, i, g, c);
-    const CellRanges cr = cell_ranges(g, c[0], c[1], c[2], cell_start, lane);
+    const CellRanges cr = cell_ranges(g, c[0], c[1], c[2], cell_start, cell_count, lane);
     for (int base = 0; base < cr.total; base += kWave) {
         int j = cell_candidate(cr, base + lane, atoms_sorted);
         if (mode == MNX_NLIST_HALF ? j >= i : j == i) j = -1;
@@ -494,38 +580,43 @@ __device__ __forceinline__ void for_candidates(const T* pos, int i, int64_t n, c
     }
 }
 
-// All-pairs fallback (a periodic axis with fewer than 3 cells): one wavefront per atom,
-// grid-stride; cell grids are handled by k_count_cells / k_emit_cells.
+// All-pairs fallback (a periodic axis with fewer than 3 cells): one wavefront per atom, grid-stride.
 template <typename T>
-__global__ void __launch_bounds__(kWave) k_count(const T* __restrict__ pos, int64_t n, const T* __restrict__ box,
-                                                 T cutoff, int mode, NlGrid* __restrict__ gp,
-                                                 const int32_t* __restrict__ cell_start,
-                                                 const int32_t* __restrict__ atoms_sorted,
-                                                 int32_t* __restrict__ counts) {
-    const NlGrid g = *gp;
-    if (!g.brute) return;
+__device__ __forceinline__ void count_all_pairs(const T* __restrict__ pos, int64_t n, const T* __restrict__ box,
+                                                T cutoff, int mode, NlGrid* __restrict__ gp, const NlGrid& g,
+                                                int32_t* __restrict__ counts) {
     const bool periodic = g.periodic;
     const AcceptTest<T> at = accept_test<T>(box, periodic, true, cutoff);
-    for (int i = blockIdx.x; i < n; i += gridDim.x) {
+    const int lane = threadIdx.x & (kWave - 1);
+    for (int64_t i = int64_t(blockIdx.x) * kParts + (threadIdx.x >> 6); i < n; i += int64_t(gridDim.x) * kParts) {
         int count = 0;
-        for_candidates<T>(pos, i, n, g, cell_start, atoms_sorted, mode, [&](int j) {
-            const bool ok = j >= 0 && accept<T>(pos, box, i, j, periodic, cutoff, at);
+        for_candidates<T>(pos, int(i), n, g, nullptr, nullptr, nullptr, mode, [&](int j) {
+            const bool ok = j >= 0 && accept<T>(pos, box, int(i), j, periodic, cutoff, at);
             count += __popcll(__ballot(ok));
         });
-        if (threadIdx.x == 0) {
+        if (lane == 0) {
             counts[i] = count;
             if (count > kNlCap) atomicExch(&gp->overflow, 1);
         }
     }
 }
 
-// Bitonic sort of `len` ints in LDS (len <= kNlCap), ascending; pads with INT_MAX.
+// Orders this wavefront's LDS writes before its reads (LDS operations of one wavefront complete in
+// order; the compiler must not move them).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Bitonic sort of `len` ints in LDS by one wavefront, ascending; buf has room for the next power of
+// two of len (padded with INT_MAX).
 __device__ void lds_sort(int32_t* buf, int len) {
     int m = 1;
     while (m < len) m <<= 1;
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & (kWave - 1);
     for (int k = len + lane; k < m; k += kWave) buf[k] = 0x7fffffff;
-    __syncthreads();
+    wave_lds_fence();
     for (int size = 2; size <= m; size <<= 1) {
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
             for (int t = lane; t < (m >> 1); t += kWave) {
@@ -538,9 +629,30 @@ __device__ void lds_sort(int32_t* buf, int len) {
                     buf[hi] = a;
                 }
             }
-            __syncthreads();
+            wave_lds_fence();
         }
     }
+}
+
+// One compare-exchange step of a bitonic sort over the lanes' values: the smaller of a pair stays in
+// the lane where `keep_low`.  The median of the two and an extreme value is their minimum or maximum.
+__device__ __forceinline__ int bitonic_step(int v, int stride, bool keep_low) {
+    const int other = lane_xor(v, stride);
+    const int bound = keep_low ? INT32_MIN : INT32_MAX;
+    int r;
+    asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "v"(other), "v"(bound));
+    return r;
+}
+
+// The lanes' values sorted over the wavefront, ascending or descending.
+__device__ __forceinline__ int wave_sort(int v, bool ascending, int lane) {
+#pragma unroll
+    for (int size = 2; size <= kWave; size <<= 1) {
+#pragma unroll
+        for (int stride = size >> 1; stride > 0; stride >>= 1)
+            v = bitonic_step(v, stride, ((size == kWave || (lane & size) == 0) == ascending) == ((lane & stride) == 0));
+    }
+    return v;
 }
 
 // Writes pair (i, j) at `slot` with the reference geometry (row = the larger index).
@@ -567,61 +679,155 @@ __device__ __forceinline__ void write_pair(const T* __restrict__ pos, const T* _
     }
 }
 
+// What the emit's stream leaves: atoms with more than kSlots neighbours (listed by the count pass),
+// and every atom of an all-pairs grid.  Candidates are tested again, collected in LDS and sorted: a
+// wavefront each with a list of kMidCap for the former, then one wavefront of the workgroup with the
+// whole buffer for atoms with still more and for all-pairs grids.  Called by whole workgroups.
 template <typename T>
-__global__ void __launch_bounds__(kWave) k_emit(const T* __restrict__ pos, int64_t n, const T* __restrict__ box,
-                                                T cutoff, int mode, int layout, const NlGrid* __restrict__ gp,
-                                                const int32_t* __restrict__ cell_start,
-                                                const int32_t* __restrict__ atoms_sorted,
-                                                const int32_t* __restrict__ big,
-                                                const int64_t* __restrict__ offsets, int64_t capacity,
-                                                int32_t* __restrict__ idx_i, int32_t* __restrict__ idx_j,
-                                                T* __restrict__ deltas, T* __restrict__ dist,
-                                                T* __restrict__ shifts) {
-    __shared__ int32_t buf[kNlCap];
-    const NlGrid g = *gp;
-    // brute grids: every atom; cell grids: the atoms the cell emit leaves (> kEmitBuf
-    // neighbours, listed by the count pass)
-    const bool only_big = !g.brute;
-    const int64_t items = only_big ? g.nbig : n;
+__device__ void emit_rest(int32_t* buf, const T* __restrict__ pos, int64_t n, const T* __restrict__ box, T cutoff,
+                          int mode, int layout, const NlGrid& g, const int32_t* __restrict__ cell_start,
+                          const int32_t* __restrict__ cell_count, const int32_t* __restrict__ atoms_sorted,
+                          const int32_t* __restrict__ big, const int64_t* __restrict__ offsets, int64_t capacity,
+                          int32_t* __restrict__ idx_i, int32_t* __restrict__ idx_j, T* __restrict__ deltas,
+                          T* __restrict__ dist, T* __restrict__ shifts) {
+    static_assert(kNlCap == 4 * kMidCap, "one list per wavefront");
     const bool periodic = g.periodic;
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
     const AcceptTest<T> at = accept_test<T>(box, periodic, true, cutoff);
-    for (int64_t t = blockIdx.x; t < items; t += gridDim.x) {
-        const int i = only_big ? big[t] : int(t);
+    auto one = [&](int i, int32_t* list, int cap) {
         int count = 0;
-        __syncthreads();  // buf is reused across atoms
-        for_candidates<T>(pos, i, n, g, cell_start, atoms_sorted, mode, [&](int j) {
+        wave_lds_fence();  // the list is reused across atoms
+        for_candidates<T>(pos, i, n, g, cell_start, cell_count, atoms_sorted, mode, [&](int j) {
             const bool ok = j >= 0 && accept<T>(pos, box, i, j, periodic, cutoff, at);
             const uint64_t m = __ballot(ok);
             const int before = __popcll(m & ((uint64_t(1) << lane) - 1));
-            if (ok && count + before < kNlCap) buf[count + before] = j;
+            if (ok && count + before < cap) list[count + before] = j;
             count += __popcll(m);
         });
-        if (count > kNlCap) count = kNlCap;  // flagged by k_count; host reports the error
-        __syncthreads();
-        lds_sort(buf, count);
+        if (count > cap) count = cap;  // more than kNlCap: flagged by the count pass; host reports the error
+        lds_sort(list, count);
         const int64_t base = layout == MNX_NLIST_TRIANGULAR ? 0 : offsets[i];
         for (int k = lane; k < count; k += kWave) {
-            const int j = buf[k];
+            const int j = list[k];
             const int64_t slot = layout == MNX_NLIST_TRIANGULAR ? int64_t(i) * (i - 1) / 2 + j : base + k;
             if (slot < capacity) write_pair<T>(pos, box, periodic, i, j, slot, idx_i, idx_j, deltas, dist, shifts);
         }
+    };
+    __syncthreads();  // the caller's use of the buffer is over
+    if (!g.brute)
+        for (int64_t t = int64_t(blockIdx.x) * 4 + wave; t < g.nmid; t += int64_t(gridDim.x) * 4)
+            one(big[t], buf + wave * kMidCap, kMidCap);
+    __syncthreads();
+    if (wave) return;
+    for (int64_t t = blockIdx.x; t < (g.brute ? n : g.nbig); t += gridDim.x)
+        one(g.brute ? int(t) : big[n - 1 - t], buf, kNlCap);
+}
+
+// ---------------------------------------------------------------------------
+// Small systems: all pairs, one wavefront per atom, candidates in id order.
+// ---------------------------------------------------------------------------
+
+// Whether the cheap test of AcceptTest applies: every box height at least 3 cutoffs (the cell
+// grid's condition), or an open system.
+template <typename T>
+__device__ __forceinline__ bool wide_box(const T* __restrict__ box, double cutoff) {
+    if (!box) return true;
+    const double ax = box[0], bx = box[3], by = box[4], cx = box[6], cy = box[7], cz = box[8];
+    const double vol = fabs(ax * by * cz), cw = cutoff * double(kCellMargin) + 1e-12;
+    const double bxc = sqrt((by * cz) * (by * cz) + (bx * cz) * (bx * cz) + (bx * cy - by * cx) * (bx * cy - by * cx));
+    const double axc = sqrt((ax * cz) * (ax * cz) + (ax * cy) * (ax * cy));
+    return vol >= 3 * cw * bxc && vol >= 3 * cw * axc && fabs(cz) >= 3 * cw;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) k_small_count(const T* __restrict__ pos, int n, const T* __restrict__ box,
+                                                     T cutoff, int mode, int words, int32_t* __restrict__ counts,
+                                                     uint64_t* __restrict__ masks) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int i = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * 4 + (threadIdx.x >> 6));
+    if (i >= n) return;
+    const bool periodic = box != nullptr;
+    const AcceptTest<T> at = accept_test<T>(box, periodic, !wide_box<T>(box, double(cutoff)), cutoff);
+    const T ax = pos[3 * i], ay = pos[3 * i + 1], az = pos[3 * i + 2];
+    const int end = mode == MNX_NLIST_HALF ? i : n;
+    int count = 0;
+    for (int base = 0; base < end; base += kWave) {
+        const int j = base + lane;
+        bool ok = j < end && j != i;
+        if (ok) ok = accept_xyz<T>(box, ax, ay, az, pos[3 * j], pos[3 * j + 1], pos[3 * j + 2], periodic, cutoff, at);
+        const uint64_t m = __ballot(ok);
+        if (lane == 0) masks[int64_t(i) * words + base / kWave] = m;
+        count += __popcll(m);
+    }
+    if (lane == 0) counts[i] = count;
+}
+
+// Offsets of up to kNlSmall counts and their total, one workgroup.
+__global__ void __launch_bounds__(kScanThreads) k_small_scan(const int32_t* __restrict__ counts, int n,
+                                                             int64_t* __restrict__ offsets,
+                                                             int64_t* __restrict__ d_total) {
+    static_assert(kNlSmall <= kScanTile, "one tile");
+    __shared__ int32_t sh[kScanThreads];
+    const int base = int(threadIdx.x) * kScanItems;
+    int32_t v[kScanItems], sum = 0, total;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        v[k] = base + k < n ? counts[base + k] : 0;
+        sum += v[k];
+    }
+    int32_t run = block_exclusive_scan<int32_t>(sum, sh, &total);
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        if (base + k < n) offsets[base + k] = run;
+        run += v[k];
+    }
+    if (threadIdx.x == 0) {
+        offsets[n] = total;
+        if (d_total) *d_total = total;
+    }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) k_small_emit(const T* __restrict__ pos, int n, const T* __restrict__ box,
+                                                    int mode, int layout, int words,
+                                                    const uint64_t* __restrict__ masks,
+                                                    const int64_t* __restrict__ offsets, int64_t capacity,
+                                                    int32_t* __restrict__ idx_i, int32_t* __restrict__ idx_j,
+                                                    T* __restrict__ deltas, T* __restrict__ dist,
+                                                    T* __restrict__ shifts) {
+    __shared__ uint16_t lists[4][kNlSmall];
+    static_assert(kNlSmall <= 65536, "16-bit ids");
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+    const int i = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * 4 + wave);
+    if (i >= n) return;
+    uint16_t* list = lists[wave];
+    const int end = mode == MNX_NLIST_HALF ? i : n;
+    const uint64_t below = (uint64_t(1) << lane) - 1;
+    int count = 0;
+    for (int base = 0; base < end; base += kWave) {
+        const uint64_t m = masks[int64_t(i) * words + base / kWave];
+        if ((m >> lane) & 1) list[count + __popcll(m & below)] = uint16_t(base + lane);
+        count += __popcll(m);
+    }
+    wave_lds_fence();
+    const int64_t off = layout == MNX_NLIST_TRIANGULAR ? 0 : offsets[i];
+    for (int k = lane; k < count; k += kWave) {
+        const int j = list[k];
+        const int64_t slot = layout == MNX_NLIST_TRIANGULAR ? int64_t(i) * (i - 1) / 2 + j : off + k;
+        if (slot < capacity) write_pair<T>(pos, box, box != nullptr, i, j, slot, idx_i, idx_j, deltas, dist, shifts);
     }
 }
 
 // ---------------------------------------------------------------------------
-// Cell grids: kCellParts wavefronts per cell, each taking every kCellParts-th atom of
-// the cell as a "centre".  All centres share the 27 neighbour cells, so each
-// candidate position is loaded once per wavefront and tested against all of its
-// centres (whose coordinates are wave-uniform).  Grid-stride over (cell, part); the
-// all-pairs fallback (k_count / k_emit) handles brute-force grids.
+// Cell grids: a workgroup per cell, grid-stride.
 // ---------------------------------------------------------------------------
 
-__device__ __forceinline__ int64_t cell_of_block(int64_t c, const NlGrid& g, int* cx, int* cy, int* cz) {
-    *cx = int(c % g.n[0]);
-    *cy = int((c / g.n[0]) % g.n[1]);
-    *cz = int(c / (int64_t(g.n[0]) * g.n[1]));
-    return c;
+__device__ __forceinline__ void cell_coords_of(uint32_t c, const NlGrid& g, int* cx, int* cy, int* cz) {
+    const uint32_t t = c / uint32_t(g.n[0]);
+    *cx = int(c - t * uint32_t(g.n[0]));
+    const uint32_t z = t / uint32_t(g.n[1]);
+    *cy = int(t - z * uint32_t(g.n[1]));
+    *cz = int(z);
 }
 
 // Slot (index into the cell-ordered arrays) of candidate number k of the flattened ranges,
@@ -649,27 +855,33 @@ __device__ __forceinline__ int cell_candidate_slot(const CellRanges& cr, int k, 
 // smaller -- and the reference arithmetic on the original positions decides the band and
 // zero distances, so the accepted set is the reference's.
 template <typename T, bool HALF>
-__global__ void __launch_bounds__(kWave) k_count_cells(const T* __restrict__ pos, const T* __restrict__ box, T cutoff,
-                                                       NlGrid* __restrict__ gp, const int32_t* __restrict__ cell_start,
-                                                       const int32_t* __restrict__ atoms_sorted,
-                                                       const PosW<T>* __restrict__ posw,
-                                                       int32_t* __restrict__ counts, int32_t* __restrict__ big,
-                                                       uint64_t* __restrict__ masks) {
+__global__ void __launch_bounds__(256) k_count_cells(const T* __restrict__ pos, int64_t n, const T* __restrict__ box,
+                                                     T cutoff, NlGrid* __restrict__ gp,
+                                                     const int32_t* __restrict__ cell_start,
+                                                     const int32_t* __restrict__ cell_count,
+                                                     const int32_t* __restrict__ atoms_sorted,
+                                                     const PosW<T>* __restrict__ posw,
+                                                     int32_t* __restrict__ counts, int32_t* __restrict__ big,
+                                                     int32_t* __restrict__ slots) {
+    __shared__ T s_x[kCand], s_y[kCand], s_z[kCand];
+    __shared__ int32_t s_id[kCand];
+    __shared__ int32_t s_list[kParts][kCentres][kSlots];
     const NlGrid g = *gp;
-    if (g.brute) return;
-    const int lane = threadIdx.x;
+    if (g.brute) {
+        count_all_pairs<T>(pos, n, box, cutoff, HALF ? MNX_NLIST_HALF : MNX_NLIST_FULL, gp, g, counts);
+        return;
+    }
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool periodic = g.periodic;
     const T c2 = cutoff * cutoff;
     const T c2lo = c2 * T(0.999), c2hi = c2 * T(1.001), c2tiny = c2 * T(1e-20);
-    for (int64_t v = blockIdx.x; v < g.ncells * kCellParts; v += gridDim.x) {
-        const int64_t c = v / kCellParts;
-        const int part = int(v - c * kCellParts);
-        const int cb = cell_start[c], ce = cell_start[c + 1];
-        const int ncent = (ce - cb - part + kCellParts - 1) / kCellParts;  // centres part, part + P, ...
-        if (ncent <= 0) continue;
+    for (int c = blockIdx.x; c < g.ncells; c += gridDim.x) {
+        const int cb = cell_start[c], ncell = cell_count[c];
         int cx, cy, cz;
-        cell_of_block(c, g, &cx, &cy, &cz);
-        const CellRanges cr = cell_ranges(g, cx, cy, cz, cell_start, lane);
+        cell_coords_of(uint32_t(c), g, &cx, &cy, &cz);
+        const CellRanges cr = cell_ranges(g, cx, cy, cz, cell_start, cell_count, lane);
+        if (ncell == 0) continue;
         // lanes 0..26: the box vectors that bring neighbour cell `lane` next to this cell
         T shx = T(0), shy = T(0), shz = T(0);
         if (periodic && lane < 27) {
@@ -680,209 +892,204 @@ __global__ void __launch_bounds__(kWave) k_count_cells(const T* __restrict__ pos
             shy = T(wy) * box[4] + T(wz) * box[7];
             shz = T(wz) * box[8];
         }
-        for (int q0 = 0; q0 < ncent; q0 += kWave) {
-            const int nq = ncent - q0 < kWave ? ncent - q0 : kWave;
-            const int my_slot = lane < nq ? cb + part + (q0 + lane) * kCellParts : -1;
-            const int my_i = my_slot >= 0 ? atoms_sorted[my_slot] : -1;
-            PosW<T> mp{T(0), T(0), T(0), T(0)};
-            if (my_slot >= 0) mp = posw[my_slot];
-            int my_count = 0;
-            const bool keep_masks = cr.total <= kWave * kMaskChunks;  // wave-uniform
-            for (int base = 0; base < cr.total; base += kWave) {
-                int r;
-                const int slot = cell_candidate_slot(cr, base + lane, &r);
-                const T sx = __shfl(shx, r, kWave), sy = __shfl(shy, r, kWave), sz = __shfl(shz, r, kWave);
-                const int j = slot >= 0 ? atoms_sorted[slot] : -1;
-                PosW<T> jp{T(0), T(0), T(0), T(0)};
-                if (slot >= 0) jp = posw[slot];
-                const T jx = jp.x + sx, jy = jp.y + sy, jz = jp.z + sz;
-                for (int q = 0; q < nq; ++q) {
-                    const int i = lane_value(my_i, q);
-                    const T dx = lane_value(mp.x, q) - jx, dy = lane_value(mp.y, q) - jy,
-                            dz = lane_value(mp.z, q) - jz;
-                    const T r2 = dx * dx + dy * dy + dz * dz;
-                    bool ok = j >= 0 && (HALF ? j < i : j != i) && !(r2 > c2hi);
-                    if (ok && !(r2 < c2lo && r2 > c2tiny)) {
-                        // the band around the cutoff and (near-)zero distances: reference arithmetic
-                        Geo<T> gg;
-                        pair_geo<T>(pos, box, i, j, periodic, false, gg);
-                        ok = gg.dist <= cutoff && gg.dist > T(0);
+        int staged = -1;  // first candidate of those in LDS
+        for (int q0 = 0; q0 < ncell; q0 += kParts * kCentres) {
+            // this wavefront's centres q0 + wave, q0 + wave + 4, ...
+            const int left = ncell - q0 - wave;
+            const int nq = left <= 0 ? 0 : min((left + kParts - 1) / kParts, kCentres);
+            int ci[kCentres], cnt[kCentres];
+            T px[kCentres], py[kCentres], pz[kCentres];
+#pragma unroll
+            for (int q = 0; q < kCentres; ++q) {
+                const int slot = cb + (q < nq ? q0 + wave + q * kParts : 0);
+                ci[q] = atoms_sorted[slot];
+                const PosW<T> p = posw[slot];
+                px[q] = p.x;
+                py[q] = p.y;
+                pz[q] = p.z;
+                cnt[q] = 0;
+            }
+            for (int b0 = 0; b0 < cr.total; b0 += kCand) {
+                const int nb = min(kCand, cr.total - b0);
+                if (staged != b0) {  // (a cell's only batch is kept for its further centres)
+                    __syncthreads();
+                    for (int base = wave * kWave; base < nb; base += kParts * kWave) {
+                        int r;
+                        const int slot = cell_candidate_slot(cr, b0 + base + lane, &r);
+                        const T sx = __shfl(shx, r, kWave), sy = __shfl(shy, r, kWave), sz = __shfl(shz, r, kWave);
+                        if (slot >= 0) {
+                            const PosW<T> p = posw[slot];
+                            s_x[base + lane] = p.x + sx;
+                            s_y[base + lane] = p.y + sy;
+                            s_z[base + lane] = p.z + sz;
+                            s_id[base + lane] = atoms_sorted[slot];
+                        } else {  // past the end (of the last 64): too far from everything
+                            s_x[base + lane] = s_y[base + lane] = s_z[base + lane] = T(1e30);
+                            s_id[base + lane] = INT32_MAX;
+                        }
                     }
-                    const uint64_t m = __ballot(ok);
-                    if (lane == q) {
-                        my_count += __popcll(m);
-                        if (keep_masks) masks[int64_t(my_i) * kMaskChunks + base / kWave] = m;
+                    __syncthreads();
+                    staged = b0;
+                }
+                if (nq == 0) continue;
+                for (int base = 0; base < nb; base += kWave) {
+                    const T jx = s_x[base + lane], jy = s_y[base + lane], jz = s_z[base + lane];
+                    const int j = s_id[base + lane];
+#pragma unroll
+                    for (int q = 0; q < kCentres; ++q) {
+                        if (q >= nq) break;
+                        const T dx = px[q] - jx, dy = py[q] - jy, dz = pz[q] - jz;
+                        const T r2 = dx * dx + dy * dy + dz * dz;
+                        bool ok = r2 <= c2hi && (HALF ? j < ci[q] : j != ci[q]);
+                        // the band around the cutoff and (near-)zero distances: reference arithmetic
+                        const bool band = ok && !(r2 < c2lo && r2 > c2tiny);
+                        if (__ballot(band)) {
+                            if (band) {
+                                Geo<T> gg;
+                                pair_geo<T>(pos, box, ci[q], j, periodic, false, gg);
+                                ok = gg.dist <= cutoff && gg.dist > T(0);
+                            }
+                        }
+                        const uint64_t m = __ballot(ok);
+                        const int at = cnt[q] + __popcll(m & ((uint64_t(1) << lane) - 1));
+                        if (ok && at < kSlots) s_list[wave][q][at] = j;
+                        cnt[q] += __popcll(m);
                     }
                 }
             }
-            if (lane < nq) {
-                counts[my_i] = my_count;
-                if (my_count > kNlCap) atomicExch(&gp->overflow, 1);
-                if (my_count > kEmitBuf) big[atomicAdd(&gp->nbig, 1)] = my_i;
+            wave_lds_fence();
+            // each centre's list in ascending order into its row
+            for (int q = 0; q < nq; ++q) {
+                const int* list = s_list[wave][q];
+                int count = cnt[0], i = ci[0];
+#pragma unroll
+                for (int k = 1; k < kCentres; ++k) {
+                    count = q == k ? cnt[k] : count;
+                    i = q == k ? ci[k] : i;
+                }
+                if (lane == 0) {
+                    counts[i] = count;
+                    if (count > kNlCap) atomicExch(&gp->overflow, 1);
+                    if (count > kMidCap) big[n - 1 - atomicAdd(&gp->nbig, 1)] = i;
+                    else if (count > kSlots) big[atomicAdd(&gp->nmid, 1)] = i;
+                }
+                if (count > kSlots) continue;
+                int32_t* row = slots + int64_t(i) * kSlots;
+                int a = lane < count ? list[lane] : INT32_MAX;
+                a = wave_sort(a, true, lane);
+                if (count > kWave) {
+                    // two runs, the second descending: one bitonic sequence of 128, merged
+                    int b = kWave + lane < count ? list[kWave + lane] : INT32_MAX;
+                    b = wave_sort(b, false, lane);
+                    const int lo = min(a, b);
+                    b = max(a, b);
+                    a = lo;
+#pragma unroll
+                    for (int stride = kWave / 2; stride > 0; stride >>= 1) {
+                        a = bitonic_step(a, stride, (lane & stride) == 0);
+                        b = bitonic_step(b, stride, (lane & stride) == 0);
+                    }
+                    if (kWave + lane < count) row[kWave + lane] = b;
+                }
+                if (lane < count) row[lane] = a;
             }
+            wave_lds_fence();  // the lists are reused
         }
     }
 }
 
+// The pairs of every atom with at most kSlots neighbours, from its sorted row: half a wavefront per
+// atom (52 neighbours of a full list at liquid density fill two passes of 32 lanes, 26 of a half
+// list one); then what needs its own search.
 template <typename T>
-__global__ void __launch_bounds__(kWave) k_emit_cells(const T* __restrict__ pos, const T* __restrict__ box, T cutoff,
-                                                      int mode, int layout, const NlGrid* __restrict__ gp,
-                                                      const int32_t* __restrict__ cell_start,
-                                                      const int32_t* __restrict__ atoms_sorted,
-                                                      const int32_t* __restrict__ counts,
-                                                      const uint64_t* __restrict__ masks,
-                                                      const int64_t* __restrict__ offsets, int64_t capacity,
-                                                      int32_t* __restrict__ idx_i, int32_t* __restrict__ idx_j,
-                                                      T* __restrict__ deltas, T* __restrict__ dist,
-                                                      T* __restrict__ shifts) {
-    __shared__ int32_t buf[kEmitBuf];  // accepted j of a batch of centres, one segment per centre
-    const NlGrid g = *gp;
-    if (g.brute) return;
-    const int lane = threadIdx.x;
-    const bool periodic = g.periodic;
-    const AcceptTest<T> at = accept_test<T>(box, periodic, false, cutoff);
-    for (int64_t v = blockIdx.x; v < g.ncells * kCellParts; v += gridDim.x) {
-        const int64_t c = v / kCellParts;
-        const int part = int(v - c * kCellParts);
-        const int cb = cell_start[c], ce = cell_start[c + 1];
-        const int ncent = (ce - cb - part + kCellParts - 1) / kCellParts;  // centres part, part + P, ...
-        if (ncent <= 0) continue;
-        int cx, cy, cz;
-        cell_of_block(c, g, &cx, &cy, &cz);
-        const CellRanges cr = cell_ranges(g, cx, cy, cz, cell_start, lane);
-        // as in the count pass: the candidate ids of up to kPreChunks chunks loaded at once
-        const int nchunks = (cr.total + kWave - 1) / kWave;  // wave-uniform
-        const bool pre = nchunks <= kPreChunks;               // implies the count pass kept the masks
-        int jr[kPreChunks];
-        if (pre) {
+__global__ void __launch_bounds__(256) k_emit_slots(const T* __restrict__ pos, int64_t n, const T* __restrict__ box,
+                                                    T cutoff, int mode, int layout, const NlGrid* __restrict__ gp,
+                                                    const int32_t* __restrict__ cell_start,
+                                                    const int32_t* __restrict__ cell_count,
+                                                    const int32_t* __restrict__ atoms_sorted,
+                                                    const int32_t* __restrict__ counts,
+                                                    const int32_t* __restrict__ slots, const int32_t* __restrict__ big,
+                                                    const int64_t* __restrict__ offsets, int64_t capacity,
+                                                    int32_t* __restrict__ idx_i, int32_t* __restrict__ idx_j,
+                                                    T* __restrict__ deltas, T* __restrict__ dist,
+                                                    T* __restrict__ shifts) {
+    __shared__ int32_t buf[kNlCap];
+    static_assert(sizeof(buf) >= 8 * 2 * 96 * sizeof(double), "the vectors of 32 pairs per half wavefront");
+    const int64_t i = int64_t(blockIdx.x) * 8 + (threadIdx.x >> 5);
+    const int l = threadIdx.x & 31;
+    if (!gp->brute && i < n) {
+        T* vec = reinterpret_cast<T*>(buf) + (threadIdx.x >> 5) * 192;  // [delta | shift] of 32 pairs
+        // the row's first 64 entries with the count and the offset (entries past the count are in the
+        // row too), then the positions of both halves together: two round trips
+        const int32_t* row = slots + i * kSlots;
+        int jn[2] = {row[l], row[32 + l]};
+        const int cnt = counts[i] > kSlots ? 0 : counts[i];
+        const int64_t off = layout == MNX_NLIST_TRIANGULAR ? 0 : offsets[i];
+        const T xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
+        for (int k0 = 0; k0 < cnt; k0 += 64) {
+            const int j[2] = {k0 + l < cnt ? jn[0] : -1, k0 + 32 + l < cnt ? jn[1] : -1};
+            T px[2], py[2], pz[2];
 #pragma unroll
-            for (int b = 0; b < kPreChunks; ++b) jr[b] = b < nchunks ? cell_candidate(cr, b * kWave + lane, atoms_sorted) : -1;
-        }
-        for (int q0 = 0; q0 < ncent;) {
-            // a batch of centres whose segments fit the buffer (kEmitBuf entries)
-            const int avail = ncent - q0 < kWave ? ncent - q0 : kWave;
-            const int my_i = lane < avail ? atoms_sorted[cb + part + (q0 + lane) * kCellParts] : -1;
-            // centres with more than kEmitBuf neighbours take no buffer space here (per-atom emit)
-            const int cnt_i = lane < avail ? counts[my_i] : 0;
-            const int my_cnt = cnt_i > kEmitBuf ? 0 : cnt_i;
-            const T mx = my_i >= 0 ? pos[3 * my_i] : T(0), my = my_i >= 0 ? pos[3 * my_i + 1] : T(0),
-                    mz = my_i >= 0 ? pos[3 * my_i + 2] : T(0);
-            int incl = my_cnt;
-#pragma unroll
-            for (int o = 1; o < kWave; o <<= 1) {
-                const int v = __shfl_up(incl, o, kWave);
-                if (lane >= o) incl += v;
+            for (int h = 0; h < 2; ++h) {
+                const int64_t a = j[h] < 0 ? i : j[h];
+                px[h] = pos[3 * a];
+                py[h] = pos[3 * a + 1];
+                pz[h] = pos[3 * a + 2];
             }
-            int nq = __popcll(__ballot(lane < avail && incl <= kEmitBuf));  // incl is non-decreasing
-            if (nq == 0) nq = 1;
-            const int my_off = incl - my_cnt;
-            int my_fill = 0;
-            __syncthreads();  // previous batch's segments fully read
-            // the count pass left each centre's accept ballots (the same candidates in the same
-            // order): reuse them instead of testing again, unless the cell had too many candidates
-            const bool use_masks = cr.total <= kWave * kMaskChunks;  // wave-uniform
-            // appends candidate j (accepted or not by this lane's `ok`) to centre q's segment
-            auto place = [&](int q, int j, bool ok) {
-                const int seg = lane_value(my_off, q);
-                const int cap = lane_value(my_cnt, q);
-                const int fill = lane_value(my_fill, q);
-                const uint64_t m = __ballot(ok);
-                const int before = __popcll(m & ((uint64_t(1) << lane) - 1));
-                if (ok && fill + before < cap) buf[seg + fill + before] = j;
-                if (lane == q) my_fill += __popcll(m);
-            };
-            if (pre) {
-                // each lane holds its own centre's ballots of every chunk; centre q's are read
-                // from lane q, and its segment is filled chunk after chunk with a uniform count
-                uint64_t mk[kPreChunks];
+            if (k0 + 64 < cnt) {
+                jn[0] = row[k0 + 64 + l];
+                jn[1] = row[k0 + 96 + l];
+            }
 #pragma unroll
-                for (int b = 0; b < kPreChunks; ++b)
-                    mk[b] = (b < nchunks && my_i >= 0) ? masks[int64_t(my_i) * kMaskChunks + b] : 0;
-                const uint64_t below = (uint64_t(1) << lane) - 1;
-                for (int q = 0; q < nq; ++q) {
-                    const int seg = lane_value(my_off, q);
-                    const int cap = lane_value(my_cnt, q);
-                    int fill = 0;
-#pragma unroll
-                    for (int b = 0; b < kPreChunks; ++b) {
-                        if (b < nchunks) {
-                            const uint64_t m = lane_value(mk[b], q);
-                            const int at = fill + __popcll(m & below);
-                            if (((m >> lane) & 1) && at < cap) buf[seg + at] = jr[b];
-                            fill += __popcll(m);
-                        }
-                    }
-                    if (lane == q) my_fill = fill;
+            for (int h = 0; h < 2; ++h) {
+                const int first_k = k0 + 32 * h;
+                if (first_k >= cnt) break;
+                Geo<T> gg;
+                const bool flip = i < j[h];  // the reference's orientation: larger index first
+                geo_from_d<T>(box, flip ? px[h] - xi : xi - px[h], flip ? py[h] - yi : yi - py[h],
+                              flip ? pz[h] - zi : zi - pz[h], box != nullptr, shifts != nullptr, gg);
+                const int64_t slot = layout == MNX_NLIST_TRIANGULAR ? i * (i - 1) / 2 + j[h] : off + first_k + l;
+                const bool in = j[h] >= 0 && slot < capacity;
+                if (in) {
+                    if (idx_i) idx_i[slot] = int32_t(i);
+                    if (idx_j) idx_j[slot] = j[h];
+                    if (dist) dist[slot] = gg.dist;
                 }
-            } else {
-                for (int base = 0; base < cr.total; base += kWave) {
-                    const int j = cell_candidate(cr, base + lane, atoms_sorted);
-                    T jx = T(0), jy = T(0), jz = T(0);
-                    if (!use_masks && j >= 0) {
-                        jx = pos[3 * j];
-                        jy = pos[3 * j + 1];
-                        jz = pos[3 * j + 2];
+#pragma unroll
+                for (int x = 0; x < 3; ++x) {
+                    gg.d[x] = flip ? -gg.d[x] : gg.d[x];
+                    gg.shift[x] = flip ? -gg.shift[x] : gg.shift[x];
+                }
+                if (layout == MNX_NLIST_TRIANGULAR) {
+                    for (int x = 0; in && x < 3; ++x) {
+                        if (deltas) deltas[3 * slot + x] = gg.d[x];
+                        if (shifts) shifts[3 * slot + x] = gg.shift[x];
                     }
-                    for (int q = 0; q < nq; ++q) {
-                        const int i = lane_value(my_i, q);
-                        bool ok;
-                        if (use_masks) {
-                            const uint64_t cm =
-                                masks[int64_t(__builtin_amdgcn_readfirstlane(i)) * kMaskChunks + base / kWave];
-                            ok = (cm >> lane) & 1;
-                        } else {
-                            const bool keep = j >= 0 && (mode == MNX_NLIST_HALF ? j < i : j != i);
-                            ok = keep && accept_xyz<T>(box, lane_value(mx, q), lane_value(my, q), lane_value(mz, q),
-                                                       jx, jy, jz, periodic, cutoff, at);
-                        }
-                        place(q, j, ok);
+                    continue;
+                }
+                wave_lds_fence();  // the vectors of the pass before are read
+#pragma unroll
+                for (int x = 0; x < 3; ++x) {
+                    vec[3 * l + x] = gg.d[x];
+                    vec[96 + 3 * l + x] = gg.shift[x];
+                }
+                wave_lds_fence();
+                const int64_t first = 3 * (off + first_k);
+                const int here = int(min(int64_t(3 * min(32, cnt - first_k)), 3 * capacity - first));
+#pragma unroll
+                for (int x = l; x < 96; x += 32) {
+                    if (x < here) {
+                        if (deltas) deltas[first + x] = vec[x];
+                        if (shifts) shifts[first + x] = vec[96 + x];
                     }
                 }
             }
-            __syncthreads();
-            // each centre's segment, ranked by j (the j are distinct), written at its offset
-            for (int q = 0; q < nq; ++q) {
-                const int i = lane_value(my_i, q);
-                const int seg = lane_value(my_off, q);
-                // entries actually written (equal to the count pass's unless it overflowed)
-                const int cap = lane_value(my_cnt, q);
-                const int got = lane_value(my_fill, q);
-                const int len = got < cap ? got : cap;
-                const int64_t obase = layout == MNX_NLIST_TRIANGULAR ? 0 : offsets[i];
-                if (len <= kWave) {
-                    // one element per lane, bitonic-sorted across the wavefront, written in order
-                    int v = lane < len ? buf[seg + lane] : INT32_MAX;
-#pragma unroll
-                    for (int size = 2; size <= kWave; size <<= 1) {
-#pragma unroll
-                        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-                            const int other = lane_xor(v, stride);
-                            const bool up = (lane & size) == 0 || size == kWave;
-                            const bool low = (lane & stride) == 0;
-                            v = (low == up) ? min(v, other) : max(v, other);
-                        }
-                    }
-                    if (lane < len) {
-                        const int64_t slot =
-                            layout == MNX_NLIST_TRIANGULAR ? int64_t(i) * (i - 1) / 2 + v : obase + lane;
-                        if (slot < capacity) write_pair<T>(pos, box, periodic, i, v, slot, idx_i, idx_j, deltas, dist,
-                                                           shifts);
-                    }
-                } else {
-                    for (int k = lane; k < len; k += kWave) {
-                        const int v = buf[seg + k];
-                        int rank = 0;
-                        for (int t = 0; t < len; ++t) rank += buf[seg + t] < v ? 1 : 0;
-                        const int64_t slot =
-                            layout == MNX_NLIST_TRIANGULAR ? int64_t(i) * (i - 1) / 2 + v : obase + rank;
-                        if (slot < capacity) write_pair<T>(pos, box, periodic, i, v, slot, idx_i, idx_j, deltas, dist,
-                                                           shifts);
-                    }
-                }
-            }
-            q0 += nq;
         }
     }
+    if (!gp->brute && gp->nmid == 0 && gp->nbig == 0) return;
+    const NlGrid g = *gp;
+    emit_rest<T>(buf, pos, n, box, cutoff, mode, layout, g, cell_start, cell_count, atoms_sorted, big, offsets,
+                 capacity, idx_i, idx_j, deltas, dist, shifts);
 }
 
 // Reference padding (-1 / NaN) for slots [from, capacity); `from` read from device when from_dev != null.
@@ -903,21 +1110,36 @@ __global__ void k_pad(int64_t from_host, const int64_t* __restrict__ from_dev, i
     }
 }
 
-// Zeroes the per-cell counters and the grid header.
-__global__ void k_nl_clear(int32_t* __restrict__ cell_count, int32_t* __restrict__ cell_fill, int64_t ncells,
-                           int32_t* __restrict__ grid_words, int64_t ngrid) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < ncells) {
-        cell_count[i] = 0;
-        cell_fill[i] = 0;
+// offsets = exclusive scan of the counts (tile sums in `tiles`), offsets[n] and *d_total their sum;
+// *d_total = -1 when some atom exceeded kNlCap neighbours.
+__global__ void __launch_bounds__(kScanThreads) k_nl_offsets(const int32_t* __restrict__ counts, int64_t n,
+                                                             const int64_t* __restrict__ tiles,
+                                                             const NlGrid* __restrict__ gp,
+                                                             int64_t* __restrict__ offsets,
+                                                             int64_t* __restrict__ d_total) {
+    __shared__ int64_t sh[kScanThreads];
+    // the tiles before this one
+    int64_t before = 0;
+    for (int64_t t = threadIdx.x; t < blockIdx.x; t += kScanThreads) before += tiles[t];
+    int64_t head;
+    block_exclusive_scan<int64_t>(before, sh, &head);
+    const int64_t base = int64_t(blockIdx.x) * kScanTile + int64_t(threadIdx.x) * kScanItems;
+    int64_t v[kScanItems], sum = 0, total;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        v[k] = base + k < n ? counts[base + k] : 0;
+        sum += v[k];
     }
-    if (i < ngrid) grid_words[i] = 0;
-}
-
-// *d_total = pair count, or -1 when some atom exceeded kNlCap neighbours.
-__global__ void k_report_total(const NlGrid* __restrict__ gp, const int64_t* __restrict__ total,
-                               int64_t* __restrict__ d_total) {
-    *d_total = gp->overflow ? int64_t(-1) : *total;
+    int64_t run = head + block_exclusive_scan<int64_t>(sum, sh, &total);
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        if (base + k < n) offsets[base + k] = run;
+        run += v[k];
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        offsets[n] = head + total;
+        if (d_total) *d_total = gp->overflow ? int64_t(-1) : head + total;
+    }
 }
 
 template <typename T>
@@ -931,52 +1153,54 @@ int nlist_count(const T* pos, int64_t n, double cutoff, const T* box, int mode, 
     size_t need = 0;
     NlWs w = carve(ws, ws_bytes, n, &need);
     if (ws_bytes < need || !ws) return set_error(MNX_ERR_WORKSPACE, "workspace %zu < %zu bytes", ws_bytes, need);
-    {
-        // cleared by a kernel rather than hipMemsetAsync, so the sequence can sit in a captured HIP graph
-        const int64_t ng = int64_t(sizeof(NlGrid) / sizeof(int32_t));
-        const int64_t m = w.max_cells > ng ? w.max_cells : ng;
-        hipLaunchKernelGGL(k_nl_clear, dim3(ceil_div(m, 256)), dim3(256), 0, stream, w.cell_count, w.cell_fill,
-                           int64_t(w.max_cells), reinterpret_cast<int32_t*>(w.grid), ng);
+    const int tb = 256;
+    if (n <= kNlSmall) {
+        if (n > 0) {
+            hipLaunchKernelGGL((k_small_count<T>), dim3(ceil_div(n, 4)), dim3(tb), 0, stream, pos, int(n), box,
+                               T(cutoff), mode, int(ceil_div(n, kWave)), w.counts, w.masks);
+            MNX_CHECK_LAUNCH();
+        }
+        hipLaunchKernelGGL(k_small_scan, dim3(1), dim3(kScanThreads), 0, stream, w.counts, int(n), w.offsets, d_total);
         MNX_CHECK_LAUNCH();
+        return MNX_OK;
     }
-    hipLaunchKernelGGL((k_grid_setup<T>), dim3(1), dim3(1024), 0, stream, pos, n, box, cutoff, w.max_cells, w.grid);
+    MNX_REQUIRE(w.max_cells < (int64_t(1) << 31), "too many atoms");
+    // cleared by a kernel rather than hipMemsetAsync, so the sequence can sit in a captured HIP graph
+    hipLaunchKernelGGL((k_nl_clear<T>), dim3(ceil_div(w.max_cells, tb)), dim3(tb), 0, stream, w.cell_count, n, box,
+                       cutoff, w.max_cells, w.grid);
     MNX_CHECK_LAUNCH();
-    if (n > 0) {
-        const int tb = 256;
-        hipLaunchKernelGGL((k_bin<T>), dim3(ceil_div(n, tb)), dim3(tb), 0, stream, pos, n, w.grid, w.cell_of, w.cell_count);
+    if (!box) {
+        hipLaunchKernelGGL((k_nl_bounds<T>), dim3(std::min<int64_t>(ceil_div(n, tb), 256)), dim3(tb), 0, stream, pos, n,
+                           w.grid);
+        MNX_CHECK_LAUNCH();
+        hipLaunchKernelGGL((k_nl_open_grid<T>), dim3(1), dim3(1), 0, stream, n, cutoff, w.max_cells, w.grid);
         MNX_CHECK_LAUNCH();
     }
-    int rc = exclusive_scan<int32_t, int32_t>(w.cell_count, w.max_cells, w.cell_start, w.tiles32,
-                                              w.cell_start + w.max_cells, stream);
-    if (rc) return rc;
-    if (n > 0) {
-        const int tb = 256;
-        // place into `counts` (free until the count pass), then rank within each cell
-        hipLaunchKernelGGL(k_place, dim3(ceil_div(n, tb)), dim3(tb), 0, stream, n, w.cell_of, w.cell_start,
-                           w.cell_fill, w.counts);
-        MNX_CHECK_LAUNCH();
-        PosW<T>* posw = static_cast<PosW<T>*>(w.posw);
-        hipLaunchKernelGGL((k_rank_cells<T>), dim3(ceil_div(n, tb)), dim3(tb), 0, stream, n, pos, box, w.grid,
-                           w.cell_of, w.cell_start, w.counts, w.atoms_sorted, posw);
-        MNX_CHECK_LAUNCH();
-        const unsigned blocks = unsigned(std::min<int64_t>(std::max<int64_t>(n, w.max_cells * kCellParts), kNlBlocks));
-        if (mode == MNX_NLIST_HALF)
-            hipLaunchKernelGGL((k_count_cells<T, true>), dim3(blocks), dim3(kWave), 0, stream, pos, box, T(cutoff),
-                               w.grid, w.cell_start, w.atoms_sorted, posw, w.counts, w.big, w.masks);
-        else
-            hipLaunchKernelGGL((k_count_cells<T, false>), dim3(blocks), dim3(kWave), 0, stream, pos, box, T(cutoff),
-                               w.grid, w.cell_start, w.atoms_sorted, posw, w.counts, w.big, w.masks);
-        MNX_CHECK_LAUNCH();
-        hipLaunchKernelGGL((k_count<T>), dim3(blocks), dim3(kWave), 0, stream, pos, n, box, T(cutoff), mode, w.grid,
-                           w.cell_start, w.atoms_sorted, w.counts);
-        MNX_CHECK_LAUNCH();
-    }
-    rc = exclusive_scan<int32_t, int64_t>(w.counts, n, w.offsets, w.tiles64, w.total, stream);
-    if (rc) return rc;
-    if (d_total) {
-        hipLaunchKernelGGL(k_report_total, dim3(1), dim3(1), 0, stream, w.grid, w.total, d_total);
-        MNX_CHECK_LAUNCH();
-    }
+    hipLaunchKernelGGL((k_bin<T>), dim3(ceil_div(n, tb)), dim3(tb), 0, stream, pos, n, w.grid, w.cell_of, w.rank,
+                       w.cell_count);
+    MNX_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_cell_runs, dim3(ceil_div(w.max_cells, kScanTile)), dim3(kScanThreads), 0, stream, w.grid,
+                       w.cell_count, w.cell_start);
+    MNX_CHECK_LAUNCH();
+    PosW<T>* posw = static_cast<PosW<T>*>(w.posw);
+    hipLaunchKernelGGL((k_place<T>), dim3(ceil_div(n, tb)), dim3(tb), 0, stream, n, pos, box, w.grid, w.cell_of, w.rank,
+                       w.cell_start, w.atoms_sorted, posw);
+    MNX_CHECK_LAUNCH();
+    const unsigned blocks = unsigned(std::min<int64_t>(w.max_cells, kNlBlocks));
+    if (mode == MNX_NLIST_HALF)
+        hipLaunchKernelGGL((k_count_cells<T, true>), dim3(blocks), dim3(tb), 0, stream, pos, n, box, T(cutoff),
+                           w.grid, w.cell_start, w.cell_count, w.atoms_sorted, posw, w.counts, w.big, w.slots);
+    else
+        hipLaunchKernelGGL((k_count_cells<T, false>), dim3(blocks), dim3(tb), 0, stream, pos, n, box, T(cutoff),
+                           w.grid, w.cell_start, w.cell_count, w.atoms_sorted, posw, w.counts, w.big, w.slots);
+    MNX_CHECK_LAUNCH();
+    const unsigned tiles = unsigned(ceil_div(n, kScanTile));
+    hipLaunchKernelGGL((k_scan_tile_sums<int32_t, int64_t>), dim3(tiles), dim3(kScanThreads), 0, stream, w.counts, n,
+                       w.tiles64);
+    MNX_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_nl_offsets, dim3(tiles), dim3(kScanThreads), 0, stream, w.counts, n, w.tiles64, w.grid,
+                       w.offsets, d_total);
+    MNX_CHECK_LAUNCH();
     return MNX_OK;
 }
 
@@ -986,34 +1210,32 @@ int nlist_emit(const T* pos, int64_t n, double cutoff, const T* box, int mode, i
                hipStream_t stream) {
     clear_error();
     MNX_REQUIRE(capacity >= 0, "capacity must be >= 0");
-    MNX_REQUIRE(layout == MNX_NLIST_COMPACT || (layout == MNX_NLIST_TRIANGULAR && mode == MNX_NLIST_HALF),
+    MNX_REQUIRE(layout == MNX_NLIST_COMPACT || layout == MNX_NLIST_EXACT ||
+                    (layout == MNX_NLIST_TRIANGULAR && mode == MNX_NLIST_HALF),
                 "triangular layout needs the half list");
     size_t need = 0;
     NlWs w = carve(const_cast<void*>(ws), ws_bytes, n, &need);
     if (ws_bytes < need || !ws) return set_error(MNX_ERR_WORKSPACE, "workspace %zu < %zu bytes", ws_bytes, need);
     if (capacity == 0) return MNX_OK;
     const int tb = 256;
-    const int64_t pad_blocks = std::min<int64_t>(ceil_div(capacity, tb), 65536);
-    if (layout == MNX_NLIST_TRIANGULAR) {
-        hipLaunchKernelGGL((k_pad<T>), dim3(pad_blocks), dim3(tb), 0, stream, int64_t(0), (const int64_t*)nullptr,
-                           capacity, idx_i, idx_j, deltas, dist, shifts);
-        MNX_CHECK_LAUNCH();
-    } else {
-        hipLaunchKernelGGL((k_pad<T>), dim3(pad_blocks), dim3(tb), 0, stream, int64_t(0), (const int64_t*)w.total,
-                           capacity, idx_i, idx_j, deltas, dist, shifts);
-        MNX_CHECK_LAUNCH();
-    }
-    if (n > 0) {
-        const unsigned blocks = unsigned(std::min<int64_t>(std::max<int64_t>(n, w.max_cells * kCellParts), kNlBlocks));
-        hipLaunchKernelGGL((k_emit_cells<T>), dim3(blocks), dim3(kWave), 0, stream, pos, box, T(cutoff), mode, layout,
-                           w.grid, w.cell_start, w.atoms_sorted, w.counts, w.masks, w.offsets, capacity, idx_i, idx_j,
+    if (layout != MNX_NLIST_EXACT) {
+        const int64_t pad_blocks = std::min<int64_t>(ceil_div(capacity, tb), 65536);
+        const int64_t* from = layout == MNX_NLIST_TRIANGULAR ? nullptr : w.offsets + n;  // the pair count
+        hipLaunchKernelGGL((k_pad<T>), dim3(pad_blocks), dim3(tb), 0, stream, int64_t(0), from, capacity, idx_i, idx_j,
                            deltas, dist, shifts);
         MNX_CHECK_LAUNCH();
-        hipLaunchKernelGGL((k_emit<T>), dim3(blocks), dim3(kWave), 0, stream, pos, n, box, T(cutoff), mode, layout,
-                           w.grid, w.cell_start, w.atoms_sorted, w.big, w.offsets, capacity, idx_i, idx_j, deltas,
-                           dist, shifts);
-        MNX_CHECK_LAUNCH();
     }
+    if (n == 0) return MNX_OK;
+    if (n <= kNlSmall) {
+        hipLaunchKernelGGL((k_small_emit<T>), dim3(ceil_div(n, 4)), dim3(tb), 0, stream, pos, int(n), box, mode, layout,
+                           int(ceil_div(n, kWave)), w.masks, w.offsets, capacity, idx_i, idx_j, deltas, dist, shifts);
+        MNX_CHECK_LAUNCH();
+        return MNX_OK;
+    }
+    hipLaunchKernelGGL((k_emit_slots<T>), dim3(ceil_div(n, 8)), dim3(tb), 0, stream, pos, n, box, T(cutoff), mode,
+                       layout, w.grid, w.cell_start, w.cell_count, w.atoms_sorted, w.counts, w.slots, w.big, w.offsets,
+                       capacity, idx_i, idx_j, deltas, dist, shifts);
+    MNX_CHECK_LAUNCH();
     return MNX_OK;
 }
 

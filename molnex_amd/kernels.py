@@ -42,7 +42,7 @@ from ._lib import check, ptr
 from .config import config as _settings
 
 MNX_NLIST_HALF, MNX_NLIST_FULL = 0, 1
-MNX_NLIST_COMPACT, MNX_NLIST_TRIANGULAR = 0, 1
+MNX_NLIST_COMPACT, MNX_NLIST_TRIANGULAR, MNX_NLIST_EXACT = 0, 1, 2
 
 
 def _stream(t: Tensor) -> int:
@@ -211,7 +211,7 @@ def neighbor_list(positions: Tensor, cutoff: float, box_vectors: Tensor, full: b
     sh = torch.empty((total, 3), dtype=dt, device=dev)
     dd = torch.empty((total, 3), dtype=dt, device=dev)
     dist = torch.empty(total, dtype=dt, device=dev)
-    _nlist_emit(pos, cutoff, box, mode, MNX_NLIST_COMPACT, ws, total, ii, jj, dd, dist, sh)
+    _nlist_emit(pos, cutoff, box, mode, MNX_NLIST_EXACT, ws, total, ii, jj, dd, dist, sh)
     return ii, jj, sh, dd, dist
 
 
