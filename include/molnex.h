@@ -342,6 +342,34 @@ int mnx_pme_gather_f64(const double* pos, const double* charges, const double* b
  * *energy, dpos [n][3], dq [n] are overwritten; dpos and dq may both be NULL (energy only, no
  * atomics).  The reference computes both in its forward (pme_cpu.cpp:168-205); the torch op
  * here computes the energy in the forward and the derivatives in the backward. */
+/* Real-space Ewald sum and self term of a periodic system within `cutoff` (minimum image), without a
+ * pair list: sum over the neighbor list's pairs (bit for bit its geometry) of coulomb q_i q_j
+ * erfc(alpha r) / r, minus coulomb alpha / sqrt(pi) sum q^2 (pme_cpu.cpp:95-135,195-215).  The energy
+ * is the sum of the mnx_pme_real_partials(n) doubles written to `partials`; dpos [n][3] and dq [n]
+ * (both or neither) its derivatives.  *overflow (device) becomes non-zero when an atom has more than
+ * 4096 neighbours; it is written only for more than 2048 atoms.  Workspace: mnx_nlist_workspace_bytes.
+ * convolve_add: mnx_pme_convolve whose energy also includes sum(more[0..nmore)).  gather_add:
+ * mnx_pme_gather whose derivatives are (reciprocal + dpos_add / dq_add) * *grad, where these device
+ * pointers are not NULL. */
+int64_t mnx_pme_real_partials(int64_t num_atoms);
+int mnx_pme_convolve_add_f32(float* cgrid, const float* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
+                             const float* xm, const float* ym, const float* zm, const double* more, int64_t nmore,
+                             float* energy, void* ws, size_t ws_bytes, mnx_stream_t s);
+int mnx_pme_gather_add_f32(const float* pos, const float* q, const float* box, int64_t n, const float* grid, int32_t gx,
+                           int32_t gy, int32_t gz, int32_t order, double coulomb, const float* grad,
+                           const float* dpos_add, const float* dq_add, float* dpos, float* dq, mnx_stream_t s);
+int mnx_pme_real_f32(const float* pos, const float* q, int64_t n, const float* box, double cutoff, double alpha,
+                     double coulomb, float* dpos, float* dq, double* partials, int32_t* overflow, void* ws,
+                     size_t ws_bytes, mnx_stream_t stream);
+int mnx_pme_convolve_add_f64(double* cgrid, const double* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
+                             const double* xm, const double* ym, const double* zm, const double* more, int64_t nmore,
+                             double* energy, void* ws, size_t ws_bytes, mnx_stream_t s);
+int mnx_pme_gather_add_f64(const double* pos, const double* q, const double* box, int64_t n, const double* grid, int32_t gx,
+                           int32_t gy, int32_t gz, int32_t order, double coulomb, const double* grad,
+                           const double* dpos_add, const double* dq_add, double* dpos, double* dq, mnx_stream_t s);
+int mnx_pme_real_f64(const double* pos, const double* q, int64_t n, const double* box, double cutoff, double alpha,
+                     double coulomb, double* dpos, double* dq, double* partials, int32_t* overflow, void* ws,
+                     size_t ws_bytes, mnx_stream_t stream);
 size_t mnx_pme_direct_workspace_bytes(int64_t num_atoms, int64_t num_pairs);
 int mnx_pme_direct_f32(const float* pos, const float* charges, int64_t num_atoms, const int32_t* neighbors,
                        int64_t num_pairs, const float* deltas, const float* distances,

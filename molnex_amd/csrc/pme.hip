@@ -15,6 +15,8 @@
 
 #include <math.h>
 
+#include <type_traits>
+
 #include "common.h"
 #include "scan.h"
 #include "wave.h"
@@ -66,34 +68,43 @@ __device__ __forceinline__ void grid_coord(const T* __restrict__ pos, int64_t at
     }
 }
 
-// Grid origin and B-spline weights (and derivatives when dd != nullptr) of one atom.
-template <typename T>
-__device__ __forceinline__ void spline(const T* __restrict__ pos, int64_t atom, const T* __restrict__ box,
-                                       const Recip<T>& R, const int grid[3], int order, int gidx[3],
-                                       T (&d)[kMaxOrder][3], T (*dd)[3]) {
-    T frac[3];
-    grid_coord<T>(pos, atom, box, R, grid, gidx, frac);
-    for (int i = 0; i < 3; ++i) {
-        const T dr = frac[i];
-        d[order - 1][i] = 0;
-        d[1][i] = dr;
-        d[0][i] = 1 - dr;
-        for (int j = 3; j < order; ++j) {
-            const T div = T(1) / (j - 1);
-            d[j - 1][i] = div * dr * d[j - 2][i];
-            for (int k = 1; k < j - 1; ++k)
-                d[j - k - 1][i] = div * ((dr + k) * d[j - k - 2][i] + (j - k - dr) * d[j - k - 1][i]);
-            d[0][i] = div * (1 - dr) * d[0][i];
-        }
-        if (dd) {
-            dd[0][i] = -d[0][i];
-            for (int j = 1; j < order; ++j) dd[j][i] = d[j - 1][i] - d[j][i];
-        }
-        const T sc = T(1) / (order - 1);
-        d[order - 1][i] = sc * dr * d[order - 2][i];
-        for (int j = 1; j < order - 1; ++j)
-            d[order - j - 1][i] = sc * ((dr + j) * d[order - j - 2][i] + (order - j - dr) * d[order - j - 1][i]);
-        d[0][i] = sc * (1 - dr) * d[0][i];
+// B-spline weights d and (when DD) derivatives dd of a fractional offset dr along one axis.
+template <typename T, int ORDER, bool DD>
+__device__ __forceinline__ void spline(T dr, T (&d)[ORDER], T (&dd)[ORDER]) {
+    d[ORDER - 1] = 0;
+    d[1] = dr;
+    d[0] = 1 - dr;
+#pragma unroll
+    for (int j = 3; j < ORDER; ++j) {
+        const T div = T(1) / (j - 1);
+        d[j - 1] = div * dr * d[j - 2];
+#pragma unroll
+        for (int k = 1; k < j - 1; ++k) d[j - k - 1] = div * ((dr + k) * d[j - k - 2] + (j - k - dr) * d[j - k - 1]);
+        d[0] = div * (1 - dr) * d[0];
+    }
+    if (DD) {
+        dd[0] = -d[0];
+#pragma unroll
+        for (int j = 1; j < ORDER; ++j) dd[j] = d[j - 1] - d[j];
+    }
+    const T sc = T(1) / (ORDER - 1);
+    d[ORDER - 1] = sc * dr * d[ORDER - 2];
+#pragma unroll
+    for (int j = 1; j < ORDER - 1; ++j)
+        d[ORDER - j - 1] = sc * ((dr + j) * d[ORDER - j - 2] + (ORDER - j - dr) * d[ORDER - j - 1]);
+    d[0] = sc * (1 - dr) * d[0];
+}
+
+// Calls f(integral_constant ORDER) for the order, 3..kMaxOrder.
+template <typename F>
+void with_order(int order, F&& f) {
+    switch (order) {
+        case 3: f(std::integral_constant<int, 3>{}); break;
+        case 4: f(std::integral_constant<int, 4>{}); break;
+        case 5: f(std::integral_constant<int, 5>{}); break;
+        case 6: f(std::integral_constant<int, 6>{}); break;
+        case 7: f(std::integral_constant<int, 7>{}); break;
+        default: f(std::integral_constant<int, kMaxOrder>{}); break;
     }
 }
 
@@ -101,28 +112,42 @@ __device__ __forceinline__ void spline(const T* __restrict__ pos, int64_t atom, 
 // Spreading as a gather over mesh bricks.  The mesh is cut into bricks of
 // kBrick^3 points (the last brick along an axis may be partial).  Atoms are
 // binned by the brick holding their spline origin, in ascending atom order
-// inside each brick.  One workgroup owns one brick: it stages the splines of
-// every atom whose origin lies in the brick or in the bricks that precede it
-// within order-1 points (cyclically).  Each lane owns one (y, z) column of the
-// brick, each of the four wavefronts sums a quarter of the staged atoms into
-// its lanes' columns, and the four partial sums are added in wave order and
-// stored once.  No atomics, every mesh point written exactly once (no
-// clearing pass), and a fixed summation order.
+// inside each brick, as records of origin, offset and scaled charge.  One
+// workgroup owns one brick: it goes through the records of the brick and of the
+// bricks that precede it within order-1 points (cyclically), keeps those whose
+// support reaches it (about one in six), evaluates their splines, one axis per
+// thread, straight into the brick's 8 positions along that axis (zero outside
+// the support), and sums them: each lane owns one (y, z) column of the brick,
+// each of the four wavefronts takes every fourth atom, and the four partial sums
+// are added in wave order and stored once.  No atomics, every mesh point written
+// exactly once (no clearing pass), and a fixed summation order.
+// Measured, 50k atoms on 128^3, order 6: 18.5 us, bound by the per-brick passes over records; 81 us
+// when every brick evaluated the splines of all candidates and one thread looked up its sources.
 // ---------------------------------------------------------------------------
 constexpr int kBrick = 8;          // mesh points per brick edge (>= kMaxOrder - 1)
-constexpr int kBrickThreads = 256; // two mesh points per thread
-constexpr int kBrickStage = 256;   // atom splines staged in LDS per pass
+constexpr int kBrickThreads = 256;
+constexpr int kBrickStage = 128;   // atoms summed per pass
 constexpr int kAxisSrc = 3;        // source bricks per axis (see axis_sources)
 static_assert(kBrick * kBrick == kWave, "one lane per (y, z) column of a brick");
-static_assert(kBrickStage * 3 * kMaxOrder >= kBrickThreads * kBrick, "reduction fits the staging area");
+static_assert(kBrickStage * 3 * kBrick >= kBrickThreads * kBrick, "reduction fits the staging area");
 
 __device__ __forceinline__ int brick_of(const int gi[3], int nby, int nbz) {
     return ((gi[0] / kBrick) * nby + gi[1] / kBrick) * nbz + gi[2] / kBrick;
 }
 
+// An atom as the spread reads it: mesh origin, offset from it, charge x sqrt(coulomb).
+template <typename T>
+struct alignas(16) SpreadRec {
+    int32_t g[3];
+    int32_t pad;
+    T frac[3];
+    T qs;
+};
+
 template <typename T>
 __global__ void k_bin_count(const T* __restrict__ pos, const T* __restrict__ box, int64_t n, int gx, int gy, int gz,
-                            int nby, int nbz, int32_t* __restrict__ brick, int32_t* __restrict__ counts) {
+                            int nby, int nbz, int32_t* __restrict__ brick, int32_t* __restrict__ rank,
+                            int32_t* __restrict__ counts) {
     const int64_t a = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (a >= n) return;
     const int G[3] = {gx, gy, gz};
@@ -132,20 +157,21 @@ __global__ void k_bin_count(const T* __restrict__ pos, const T* __restrict__ box
     grid_coord<T>(pos, a, box, R, G, gi, frac);
     const int b = brick_of(gi, nby, nbz);
     brick[a] = b;
-    atomicAdd(counts + b, 1);
+    rank[a] = atomicAdd(counts + b, 1);
 }
 
 __global__ void k_bin_place(const int32_t* __restrict__ brick, int64_t n, const int32_t* __restrict__ ptr,
-                            int32_t* __restrict__ fill, int32_t* __restrict__ slots) {
+                            const int32_t* __restrict__ rank, int32_t* __restrict__ slots) {
     const int64_t a = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (a >= n) return;
-    const int b = brick[a];
-    slots[ptr[b] + atomicAdd(fill + b, 1)] = int32_t(a);
+    if (a < n) slots[ptr[brick[a]] + rank[a]] = int32_t(a);
 }
 
-// Ascending atom order inside each brick: slot j moves to its rank within its brick.
-__global__ void k_bin_rank(const int32_t* __restrict__ brick, const int32_t* __restrict__ ptr,
-                           const int32_t* __restrict__ slots, int64_t n, int32_t* __restrict__ perm) {
+// Ascending atom order inside each brick: the atom in slot j moves to its rank within its brick, as
+// a record.
+template <typename T>
+__global__ void k_bin_rank(const T* __restrict__ pos, const T* __restrict__ q, const T* __restrict__ box, int gx, int gy,
+                           int gz, T sqrt_k, const int32_t* __restrict__ brick, const int32_t* __restrict__ ptr,
+                           const int32_t* __restrict__ slots, int64_t n, SpreadRec<T>* __restrict__ recs) {
     const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (j >= n) return;
     const int a = slots[j];
@@ -153,7 +179,13 @@ __global__ void k_bin_rank(const int32_t* __restrict__ brick, const int32_t* __r
     const int lo = ptr[b], hi = ptr[b + 1];
     int r = 0;
     for (int k = lo; k < hi; ++k) r += slots[k] < a;
-    perm[lo + r] = a;
+    const int G[3] = {gx, gy, gz};
+    const Recip<T> R = invert_box<T>(box);
+    SpreadRec<T> rec;
+    grid_coord<T>(pos, a, box, R, G, rec.g, rec.frac);
+    rec.pad = 0;
+    rec.qs = q[a] * sqrt_k;
+    recs[lo + r] = rec;
 }
 
 // Bricks along one axis whose atoms reach destination brick b: b itself and the
@@ -172,98 +204,123 @@ __device__ __forceinline__ int axis_sources(int b, int nb, int G, int order, int
     return k;
 }
 
-template <typename T>
+template <typename T, int ORDER>
 __global__ void __launch_bounds__(kBrickThreads)
-    k_spread_bricks(const T* __restrict__ pos, const T* __restrict__ q, const T* __restrict__ box, int gx, int gy,
-                    int gz, int nbx, int nby, int nbz, int order, T sqrt_k, const int32_t* __restrict__ ptr,
-                    const int32_t* __restrict__ perm, T* __restrict__ grid) {
+    k_spread_bricks(int gx, int gy, int gz, int nbx, int nby, int nbz, const int32_t* __restrict__ ptr,
+                    const SpreadRec<T>* __restrict__ recs, T* __restrict__ grid) {
     constexpr int kSrc = kAxisSrc * kAxisSrc * kAxisSrc;
-    __shared__ int s_src[kSrc];
-    __shared__ int s_off[kSrc + 1];
-    __shared__ int s_nsrc;
-    __shared__ int s_rel[kBrickStage];             // packed brick-relative origin, -1: misses the brick
-    __shared__ T s_w[kBrickStage][3 * kMaxOrder];  // [x weights * q sqrt(k) | y weights | z weights]
+    __shared__ int s_src[kSrc + 1];      // first record of each source brick
+    __shared__ int s_end[kSrc + 1];      // candidates up to and including it
+    __shared__ int s_cnt[2][4];          // reaching candidates of each wavefront, this pass and the next
+    __shared__ int s_rec[kBrickStage + kBrickThreads];  // records of the reaching atoms found
+    __shared__ T s_w[kBrickStage][3 * kBrick];          // [x weights * q | y weights | z weights] per position
     const int bid = blockIdx.x;
     const int bz = bid % nbz, by = (bid / nbz) % nby, bx = bid / (nbz * nby);
-    if (threadIdx.x == 0) {
-        int sx[kAxisSrc], sy[kAxisSrc], sz[kAxisSrc];
-        const int nx = axis_sources(bx, nbx, gx, order, sx);
-        const int ny = axis_sources(by, nby, gy, order, sy);
-        const int nz = axis_sources(bz, nbz, gz, order, sz);
-        int k = 0, off = 0;
-        for (int i = 0; i < nx; ++i)
-            for (int j = 0; j < ny; ++j)
-                for (int l = 0; l < nz; ++l) {
-                    const int s = (sx[i] * nby + sy[j]) * nbz + sz[l];
-                    s_src[k] = s;
-                    s_off[k] = off;
-                    off += ptr[s + 1] - ptr[s];
-                    ++k;
-                }
-        s_off[k] = off;
-        s_nsrc = k;
+    const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+    int sx[kAxisSrc], sy[kAxisSrc], sz[kAxisSrc];
+    const int nx = axis_sources(bx, nbx, gx, ORDER, sx);
+    const int ny = axis_sources(by, nby, gy, ORDER, sy);
+    const int nz = axis_sources(bz, nbz, gz, ORDER, sz);
+    const int nsrc = nx * ny * nz;
+    if (wave == 0) {
+        // lane s: source brick s, in (x, y, z) source order
+        int first = 0, len = 0;
+        if (lane < nsrc) {
+            const int ix = lane / (ny * nz), iy = (lane / nz) % ny, iz = lane % nz;
+            auto pick = [](const int (&v)[kAxisSrc], int k) { return k == 0 ? v[0] : (k == 1 ? v[1] : v[2]); };
+            const int s = (pick(sx, ix) * nby + pick(sy, iy)) * nbz + pick(sz, iz);
+            first = ptr[s];
+            len = ptr[s + 1] - first;
+        }
+        int incl = len;
+#pragma unroll
+        for (int o = 1; o < 32; o <<= 1) {
+            const int u = __shfl_up(incl, o, kWave);
+            if (lane >= o) incl += u;
+        }
+        if (lane <= kSrc) {
+            s_src[lane] = first;
+            s_end[lane] = incl;
+        }
     }
     __syncthreads();
-    const int total = s_off[s_nsrc];
+    const int total = s_end[nsrc - 1];
     const int G[3] = {gx, gy, gz};
     const int S[3] = {bx * kBrick, by * kBrick, bz * kBrick};
-    const Recip<T> R = invert_box<T>(box);
-    const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+    // origin relative to the brick start along axis a, cyclically in (-G, brick size); the atom
+    // reaches the brick along the axis iff that offset is > -ORDER
+    auto relative = [&](int g, int a) {
+        int r = g - S[a];
+        r += r < 0 ? G[a] : 0;
+        if (r >= min(kBrick, G[a] - S[a])) r -= G[a];
+        return r;
+    };
     // lane -> (y, z) column of the brick; acc[x] for its 8 points along x
     const int ly = lane >> 3, lz = lane & 7;
     T acc[kBrick];
     for (int x = 0; x < kBrick; ++x) acc[x] = 0;
-    for (int base = 0; base < total; base += kBrickStage) {
-        const int cnt = min(kBrickStage, total - base);
-        for (int c = t; c < cnt; c += kBrickThreads) {
-            const int g = base + c;
-            int s = 0;
-            while (s_off[s + 1] <= g) ++s;
-            const int atom = perm[ptr[s_src[s]] + (g - s_off[s])];
-            int gi[3];
-            T d[kMaxOrder][3];
-            spline<T>(pos, atom, box, R, G, order, gi, d, nullptr);
-            // origin relative to the brick start, cyclically in (-G, brick size); the atom
-            // reaches the brick along an axis iff that offset is > -order
-            int rel[3];
-            bool reach = true;
-            for (int a = 0; a < 3; ++a) {
-                int r = gi[a] - S[a];
-                r += r < 0 ? G[a] : 0;
-                if (r >= min(kBrick, G[a] - S[a])) r -= G[a];
-                reach = reach && r > -order;
-                rel[a] = r;
-            }
-            s_rel[c] = reach ? (rel[0] + 8) | ((rel[1] + 8) << 4) | ((rel[2] + 8) << 8) : -1;
-            if (reach) {
-                const T qs = q[atom] * sqrt_k;
-                for (int k = 0; k < order; ++k) {
-                    s_w[c][k] = qs * d[k][0];
-                    s_w[c][kMaxOrder + k] = d[k][1];
-                    s_w[c][2 * kMaxOrder + k] = d[k][2];
+    int held = 0;  // reaching atoms in s_rec
+    for (int base = 0, pass = 0; base < total; base += kBrickThreads, ++pass) {
+        // this thread's candidate: does its support reach the brick?
+        int rec = -1;
+        if (base + t < total) {
+            int s = 0;  // sources that end at or before it
+#pragma unroll
+            for (int step = 16; step > 0; step >>= 1)
+                if (s + step <= nsrc - 1 && s_end[s + step - 1] <= base + t) s += step;
+            rec = s_src[s] + (base + t - (s ? s_end[s - 1] : 0));
+            const SpreadRec<T>& r = recs[rec];
+            if (!(relative(r.g[0], 0) > -ORDER && relative(r.g[1], 1) > -ORDER && relative(r.g[2], 2) > -ORDER)) rec = -1;
+        }
+        const uint64_t m = __ballot(rec >= 0);
+        if (lane == 0) s_cnt[pass & 1][wave] = __popcll(m);
+        __syncthreads();
+        int at = held + __popcll(m & ((uint64_t(1) << lane) - 1));
+        for (int w = 0; w < kBrickThreads / kWave; ++w) {
+            const int c = s_cnt[pass & 1][w];
+            if (w < wave) at += c;
+            held += c;
+        }
+        if (rec >= 0) s_rec[at] = rec;
+        const bool last = base + kBrickThreads >= total;
+        __syncthreads();
+        while (held >= kBrickStage || (last && held > 0)) {
+            const int cnt = min(held, kBrickStage);
+            // one axis of one atom per thread
+            for (int e = t; e < 3 * cnt; e += kBrickThreads) {
+                const int c = e / 3, a = e - 3 * c;
+                const SpreadRec<T>& r = recs[s_rec[c]];
+                const int rel = relative(a == 0 ? r.g[0] : (a == 1 ? r.g[1] : r.g[2]), a);
+                const T fr = a == 0 ? r.frac[0] : (a == 1 ? r.frac[1] : r.frac[2]);
+                const int period = a == 0 ? gx : (a == 1 ? gy : gz);
+                T d[ORDER], dd[ORDER];
+                spline<T, ORDER, false>(fr, d, dd);
+                const T sc = a == 0 ? r.qs : T(1);
+                T* w = &s_w[c][a * kBrick];
+#pragma unroll
+                for (int x = 0; x < kBrick; ++x) w[x] = 0;
+#pragma unroll
+                for (int k = 0; k < ORDER; ++k) {
+                    const int x = rel + k, y = x - period;  // y: around a mesh shorter than brick + order
+                    if (x >= 0 && x < kBrick) w[x] = sc * d[k];
+                    if (y >= 0 && y < kBrick) w[y] = sc * d[k];
                 }
             }
-        }
-        __syncthreads();
-        // wave w sums candidates w, w + 4, ... in order (wave-uniform skip of non-reaching ones)
-        for (int c = wave; c < cnt; c += kBrickThreads / kWave) {
-            const int pk = s_rel[c];
-            if (pk < 0) continue;
-            const int rx = (pk & 15) - 8, ry = ((pk >> 4) & 15) - 8, rz = (pk >> 8) - 8;
-            int dy = ly - ry;
-            dy += dy < 0 ? gy : 0;
-            int dz = lz - rz;
-            dz += dz < 0 ? gz : 0;
-            const bool in = dy < order && dz < order;
-            const T wyz = in ? s_w[c][kMaxOrder + dy] * s_w[c][2 * kMaxOrder + dz] : T(0);
+            __syncthreads();
+            for (int c = wave; c < cnt; c += kBrickThreads / kWave) {
+                const T wyz = s_w[c][kBrick + ly] * s_w[c][2 * kBrick + lz];
 #pragma unroll
-            for (int x = 0; x < kBrick; ++x) {
-                int dx = x - rx;
-                dx += dx < 0 ? gx : 0;
-                if (dx < order) acc[x] += s_w[c][dx] * wyz;
+                for (int x = 0; x < kBrick; ++x) acc[x] += s_w[c][x] * wyz;
             }
+            __syncthreads();
+            // the atoms left over move to the front
+            const int keep = held - cnt;
+            const int moved = t < keep ? s_rec[cnt + t] : 0;
+            __syncthreads();
+            if (t < keep) s_rec[t] = moved;
+            held = keep;
+            __syncthreads();
         }
-        __syncthreads();
     }
     // the four waves' partial sums, added in wave order (reuses the staging area)
     T* red = &s_w[0][0];
@@ -294,10 +351,12 @@ __global__ void __launch_bounds__(kConvThreads) k_convolve(T* __restrict__ cgrid
     double e = 0.0;
     if (idx < total) {
         const Recip<T> R = invert_box<T>(box);
-        const int kx = int(idx / (int64_t(gy) * zs));
-        const int rem = int(idx - int64_t(kx) * gy * zs);
-        const int ky = rem / zs;
-        const int kz = rem - ky * zs;
+        // the mesh has fewer than 2^31 points
+        const uint32_t i32 = uint32_t(idx), plane = uint32_t(gy) * zs;
+        const int kx = int(i32 / plane);
+        const uint32_t rem = i32 - uint32_t(kx) * plane;
+        const int ky = int(rem / uint32_t(zs));
+        const int kz = int(rem - uint32_t(ky) * zs);
         const int mx = kx < (gx + 1) / 2 ? kx : kx - gx;
         const int my = ky < (gy + 1) / 2 ? ky : ky - gy;
         const int mz = kz < (gz + 1) / 2 ? kz : kz - gz;
@@ -325,55 +384,120 @@ __global__ void __launch_bounds__(kConvThreads) k_convolve(T* __restrict__ cgrid
     if (threadIdx.x == 0) partials[blockIdx.x] = red[0];
 }
 
-// energy = scale * sum(partials), summed by one block in a fixed order.
+// energy = scale * sum(partials) + sum(more), summed by one block in a fixed order.
 template <typename T>
 __global__ void __launch_bounds__(1024) k_sum_partials(const double* __restrict__ partials, int64_t n, double scale,
+                                                       const double* __restrict__ more, int64_t nmore,
                                                        T* __restrict__ energy) {
     __shared__ double red[1024];
     double s = 0.0;
     for (int64_t i = threadIdx.x; i < n; i += 1024) s += partials[i];
+    s *= scale;
+    for (int64_t i = threadIdx.x; i < nmore; i += 1024) s += more[i];
     red[threadIdx.x] = s;
     __syncthreads();
     for (int off = 512; off > 0; off >>= 1) {
         if (threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
         __syncthreads();
     }
-    if (threadIdx.x == 0) *energy = T(scale * red[0]);
+    if (threadIdx.x == 0) *energy = T(red[0]);
 }
 
-// d/dpos and d/dq of the reciprocal energy from the back-transformed grid (pme_cpu.cpp:311-343).
-template <typename T>
-__global__ void k_gather(const T* __restrict__ pos, const T* __restrict__ q, const T* __restrict__ box, int64_t n,
-                         const T* __restrict__ grid, int gx, int gy, int gz, int order, T sqrt_k,
-                         T* __restrict__ dpos, T* __restrict__ dq) {
-    const int64_t atom = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (atom >= n) return;
+// d/dpos and d/dq of the reciprocal energy from the back-transformed grid (pme_cpu.cpp:311-343), plus
+// the given derivatives (dpos_add, dq_add) when there are any, times *grad when it is given.
+//
+// ORDER^2 columns of ORDER consecutive mesh points per atom: L lanes share an atom (16 up to order
+// 4, else 32), each taking whole columns; three of them evaluate the atom's splines, one axis each,
+// into LDS.  (One thread per atom left 50k atoms on 782 wavefronts, each with 216 dependent loads.)
+// Measured, 50k atoms on 128^3, order 6: 33 us (10.8 M mesh reads from L2), 88 us before.
+constexpr int kGatherThreads = 256;
+
+template <typename T, int ORDER>
+__global__ void __launch_bounds__(kGatherThreads) k_gather(const T* __restrict__ pos, const T* __restrict__ q,
+                                                           const T* __restrict__ box, int64_t n,
+                                                           const T* __restrict__ grid, int gx, int gy, int gz, T sqrt_k,
+                                                           const T* __restrict__ grad, const T* __restrict__ dpos_add,
+                                                           const T* __restrict__ dq_add, T* __restrict__ dpos,
+                                                           T* __restrict__ dq) {
+    constexpr int L = ORDER <= 4 ? 16 : 32, ATOMS = kGatherThreads / L;
+    __shared__ T s_w[ATOMS][3][2][ORDER];  // weights and derivatives
+    const int slot = threadIdx.x / L, l = threadIdx.x % L;
+    const int64_t atom = int64_t(blockIdx.x) * ATOMS + slot;
+    const bool in = atom < n;
     const int G[3] = {gx, gy, gz};
     const Recip<T> R = invert_box<T>(box);
-    int gi[3];
-    T d[kMaxOrder][3], dd[kMaxOrder][3];
-    spline<T>(pos, atom, box, R, G, order, gi, d, dd);
-    T p0 = 0, p1 = 0, p2 = 0, s = 0;
-    for (int ix = 0; ix < order; ++ix) {
-        const int x = (gi[0] + ix) % gx;
-        for (int iy = 0; iy < order; ++iy) {
-            const int y = (gi[1] + iy) % gy;
-            const T* row = grid + (int64_t(x) * gy + y) * gz;
-            const T dxy = d[ix][0] * d[iy][1], dxdy = dd[ix][0] * d[iy][1], xdy = d[ix][0] * dd[iy][1];
-            for (int iz = 0; iz < order; ++iz) {
-                const T g = row[(gi[2] + iz) % gz];
-                p0 += dxdy * d[iz][2] * g;
-                p1 += xdy * d[iz][2] * g;
-                p2 += dxy * dd[iz][2] * g;
-                s += dxy * d[iz][2] * g;
+    int gi[3] = {0, 0, 0};
+    if (in) {
+        T frac[3];
+        grid_coord<T>(pos, atom, box, R, G, gi, frac);
+        if (l < 3) {
+            T d[ORDER], dd[ORDER];
+            spline<T, ORDER, true>(l == 0 ? frac[0] : (l == 1 ? frac[1] : frac[2]), d, dd);
+#pragma unroll
+            for (int k = 0; k < ORDER; ++k) {
+                s_w[slot][l][0][k] = d[k];
+                s_w[slot][l][1][k] = dd[k];
             }
         }
     }
+    __syncthreads();
+    T p0 = 0, p1 = 0, p2 = 0, s = 0;
+    if (in) {
+        T wz[ORDER], dz[ORDER];
+        int oz[ORDER];
+#pragma unroll
+        for (int k = 0; k < ORDER; ++k) {
+            wz[k] = s_w[slot][2][0][k];
+            dz[k] = s_w[slot][2][1][k];
+            oz[k] = gi[2] + k < gz ? gi[2] + k : gi[2] + k - gz;
+        }
+#pragma unroll
+        for (int c0 = 0; c0 < ORDER * ORDER; c0 += L) {
+            const int c = c0 + l;
+            if (c < ORDER * ORDER) {
+                const int ix = c / ORDER, iy = c - ix * ORDER;
+                const int x = gi[0] + ix < gx ? gi[0] + ix : gi[0] + ix - gx;
+                const int y = gi[1] + iy < gy ? gi[1] + iy : gi[1] + iy - gy;
+                const T* row = grid + (int64_t(x) * gy + y) * gz;
+                T v = 0, dv = 0;
+#pragma unroll
+                for (int k = 0; k < ORDER; ++k) {
+                    const T g = row[oz[k]];
+                    v += wz[k] * g;
+                    dv += dz[k] * g;
+                }
+                const T wx = s_w[slot][0][0][ix], dx = s_w[slot][0][1][ix], wy = s_w[slot][1][0][iy],
+                        dy = s_w[slot][1][1][iy];
+                p0 += dx * wy * v;
+                p1 += wx * dy * v;
+                p2 += wx * wy * dv;
+                s += wx * wy * v;
+            }
+        }
+    }
+#pragma unroll
+    for (int o = L / 2; o > 0; o >>= 1) {
+        p0 += __shfl_xor(p0, o, kWave);
+        p1 += __shfl_xor(p1, o, kWave);
+        p2 += __shfl_xor(p2, o, kWave);
+        s += __shfl_xor(s, o, kWave);
+    }
+    if (!in || l) return;
     const T sc = q[atom] * sqrt_k;
-    dpos[3 * atom + 0] = sc * (p0 * gx * R.r[0][0]);
-    dpos[3 * atom + 1] = sc * (p0 * gx * R.r[1][0] + p1 * gy * R.r[1][1]);
-    dpos[3 * atom + 2] = sc * (p0 * gx * R.r[2][0] + p1 * gy * R.r[2][1] + p2 * gz * R.r[2][2]);
-    dq[atom] = s * sqrt_k;
+    T f[3] = {sc * (p0 * gx * R.r[0][0]), sc * (p0 * gx * R.r[1][0] + p1 * gy * R.r[1][1]),
+              sc * (p0 * gx * R.r[2][0] + p1 * gy * R.r[2][1] + p2 * gz * R.r[2][2])};
+    T fq = s * sqrt_k;
+    if (dpos_add) {
+        for (int k = 0; k < 3; ++k) f[k] += dpos_add[3 * atom + k];
+        fq += dq_add[atom];
+    }
+    if (grad) {
+        const T w = *grad;
+        for (int k = 0; k < 3; ++k) f[k] *= w;
+        fq *= w;
+    }
+    for (int k = 0; k < 3; ++k) dpos[3 * atom + k] = f[k];
+    dq[atom] = fq;
 }
 
 // Block-wide fp64 sum of one value per thread into partials[blockIdx.x].
@@ -504,19 +628,20 @@ int check_grid(int gx, int gy, int gz, int order) {
 }
 
 struct BrickWs {
-    int32_t *counts, *fill, *ptr, *tiles, *brick, *slots, *perm;
+    int32_t *counts, *ptr, *tiles, *brick, *rank, *slots;
+    void* recs;  // SpreadRec<T>
 };
 
 BrickWs carve_bricks(void* base, int64_t n, int64_t nbricks, size_t* used) {
     Workspace ws{static_cast<char*>(base), 0};
     BrickWs w;
     w.counts = ws.take<int32_t>(nbricks + 1);
-    w.fill = ws.take<int32_t>(nbricks + 1);
     w.ptr = ws.take<int32_t>(nbricks + 1);
     w.tiles = ws.take<int32_t>(scan_workspace_elems(nbricks + 1));
     w.brick = ws.take<int32_t>(n);
+    w.rank = ws.take<int32_t>(n);
     w.slots = ws.take<int32_t>(n);
-    w.perm = ws.take<int32_t>(n);
+    w.recs = ws.take<SpreadRec<double>>(n);
     *used = ws.used;
     return w;
 }
@@ -543,25 +668,27 @@ int spread(const T* pos, const T* q, const T* box, int64_t n, int gx, int gy, in
     BrickWs w = carve_bricks(ws, n, nbricks, &need);
     if (!ws || ws_bytes < need) return set_error(MNX_ERR_WORKSPACE, "workspace %zu < %zu bytes", ws_bytes, need);
     const int tb = 256;
-    for (int32_t* p : {w.counts, w.fill}) {
-        hipLaunchKernelGGL((k_fill<int32_t>), dim3(ceil_div(nbricks + 1, tb)), dim3(tb), 0, s, p, nbricks + 1);
-        MNX_CHECK_LAUNCH();
-    }
+    hipLaunchKernelGGL((k_fill<int32_t>), dim3(ceil_div(nbricks + 1, tb)), dim3(tb), 0, s, w.counts, nbricks + 1);
+    MNX_CHECK_LAUNCH();
     if (n > 0) {
         hipLaunchKernelGGL((k_bin_count<T>), dim3(ceil_div(n, tb)), dim3(tb), 0, s, pos, box, n, gx, gy, gz, nby, nbz,
-                           w.brick, w.counts);
+                           w.brick, w.rank, w.counts);
         MNX_CHECK_LAUNCH();
     }
     rc = exclusive_scan<int32_t, int32_t>(w.counts, nbricks + 1, w.ptr, w.tiles, (int32_t*)nullptr, s);
     if (rc) return rc;
+    SpreadRec<T>* recs = static_cast<SpreadRec<T>*>(w.recs);
     if (n > 0) {
-        hipLaunchKernelGGL(k_bin_place, dim3(ceil_div(n, tb)), dim3(tb), 0, s, w.brick, n, w.ptr, w.fill, w.slots);
+        hipLaunchKernelGGL(k_bin_place, dim3(ceil_div(n, tb)), dim3(tb), 0, s, w.brick, n, w.ptr, w.rank, w.slots);
         MNX_CHECK_LAUNCH();
-        hipLaunchKernelGGL(k_bin_rank, dim3(ceil_div(n, tb)), dim3(tb), 0, s, w.brick, w.ptr, w.slots, n, w.perm);
+        hipLaunchKernelGGL((k_bin_rank<T>), dim3(ceil_div(n, tb)), dim3(tb), 0, s, pos, q, box, gx, gy, gz,
+                           T(sqrt(coulomb)), w.brick, w.ptr, w.slots, n, recs);
         MNX_CHECK_LAUNCH();
     }
-    hipLaunchKernelGGL((k_spread_bricks<T>), dim3(nbricks), dim3(kBrickThreads), 0, s, pos, q, box, gx, gy, gz, nbx,
-                       nby, nbz, order, T(sqrt(coulomb)), w.ptr, w.perm, grid);
+    with_order(order, [&](auto o) {
+        hipLaunchKernelGGL((k_spread_bricks<T, decltype(o)::value>), dim3(nbricks), dim3(kBrickThreads), 0, s, gx, gy, gz,
+                           nbx, nby, nbz, w.ptr, recs, grid);
+    });
     MNX_CHECK_LAUNCH();
     return MNX_OK;
 }
@@ -570,9 +697,10 @@ int64_t conv_blocks(int gx, int gy, int gz) { return ceil_div(int64_t(gx) * gy *
 
 template <typename T>
 int convolve(T* cgrid, const T* box, int gx, int gy, int gz, double alpha, const T* xm, const T* ym, const T* zm,
-             T* energy, void* ws, size_t ws_bytes, hipStream_t s) {
+             const double* more, int64_t nmore, T* energy, void* ws, size_t ws_bytes, hipStream_t s) {
     clear_error();
     int rc = check_grid(gx, gy, gz, 3);
+    MNX_REQUIRE(rc || nmore == 0 || more, "null pointer argument");
     if (rc) return rc;
     MNX_REQUIRE(cgrid && box && xm && ym && zm && energy, "null pointer argument");
     const int64_t nb = conv_blocks(gx, gy, gz);
@@ -582,21 +710,25 @@ int convolve(T* cgrid, const T* box, int gx, int gy, int gz, double alpha, const
     hipLaunchKernelGGL((k_convolve<T>), dim3(nb), dim3(kConvThreads), 0, s, cgrid, box, gx, gy, gz, T(alpha), xm, ym,
                        zm, part);
     MNX_CHECK_LAUNCH();
-    hipLaunchKernelGGL((k_sum_partials<T>), dim3(1), dim3(1024), 0, s, part, nb, 0.5, energy);
+    hipLaunchKernelGGL((k_sum_partials<T>), dim3(1), dim3(1024), 0, s, part, nb, 0.5, more, nmore, energy);
     MNX_CHECK_LAUNCH();
     return MNX_OK;
 }
 
 template <typename T>
 int gather(const T* pos, const T* q, const T* box, int64_t n, const T* grid, int gx, int gy, int gz, int order,
-           double coulomb, T* dpos, T* dq, hipStream_t s) {
+           double coulomb, const T* grad, const T* dpos_add, const T* dq_add, T* dpos, T* dq, hipStream_t s) {
     clear_error();
     int rc = check_grid(gx, gy, gz, order);
     if (rc) return rc;
     if (n == 0) return MNX_OK;
     MNX_REQUIRE(pos && q && box && grid && dpos && dq, "null pointer argument");
-    hipLaunchKernelGGL((k_gather<T>), dim3(ceil_div(n, 128)), dim3(128), 0, s, pos, q, box, n, grid, gx, gy, gz, order,
-                       T(sqrt(coulomb)), dpos, dq);
+    MNX_REQUIRE((dpos_add == nullptr) == (dq_add == nullptr), "dpos_add and dq_add must both be given or both be null");
+    with_order(order, [&](auto o) {
+        constexpr int kOrder = decltype(o)::value, kAtoms = kGatherThreads / (kOrder <= 4 ? 16 : 32);
+        hipLaunchKernelGGL((k_gather<T, kOrder>), dim3(ceil_div(n, kAtoms)), dim3(kGatherThreads), 0, s, pos, q, box, n,
+                           grid, gx, gy, gz, T(sqrt(coulomb)), grad, dpos_add, dq_add, dpos, dq);
+    });
     MNX_CHECK_LAUNCH();
     return MNX_OK;
 }
@@ -644,7 +776,8 @@ int direct(const T* pos, const T* q, int64_t n, const int32_t* nb, int64_t P, co
                                 b2, s);
     MNX_CHECK_LAUNCH();
     // every launched block wrote its partial; with no blocks the energy is 0
-    hipLaunchKernelGGL((k_sum_partials<T>), dim3(1), dim3(1024), 0, s, part, b1 + b2, 1.0, energy);
+    hipLaunchKernelGGL((k_sum_partials<T>), dim3(1), dim3(1024), 0, s, part, b1 + b2, 1.0,
+                       (const double*)nullptr, int64_t(0), energy);
     MNX_CHECK_LAUNCH();
     return MNX_OK;
 }
@@ -675,21 +808,21 @@ size_t mnx_pme_convolve_workspace_bytes(int32_t gx, int32_t gy, int32_t gz) {
 int mnx_pme_convolve_f32(float* cgrid, const float* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
                          const float* xm, const float* ym, const float* zm, float* energy, void* ws, size_t ws_bytes,
                          mnx_stream_t s) {
-    return convolve<float>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, energy, ws, ws_bytes, (hipStream_t)s);
+    return convolve<float>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, nullptr, 0, energy, ws, ws_bytes, (hipStream_t)s);
 }
 int mnx_pme_convolve_f64(double* cgrid, const double* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
                          const double* xm, const double* ym, const double* zm, double* energy, void* ws,
                          size_t ws_bytes, mnx_stream_t s) {
-    return convolve<double>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, energy, ws, ws_bytes, (hipStream_t)s);
+    return convolve<double>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, nullptr, 0, energy, ws, ws_bytes, (hipStream_t)s);
 }
 int mnx_pme_gather_f32(const float* pos, const float* q, const float* box, int64_t n, const float* grid, int32_t gx,
                        int32_t gy, int32_t gz, int32_t order, double coulomb, float* dpos, float* dq, mnx_stream_t s) {
-    return gather<float>(pos, q, box, n, grid, gx, gy, gz, order, coulomb, dpos, dq, (hipStream_t)s);
+    return gather<float>(pos, q, box, n, grid, gx, gy, gz, order, coulomb, nullptr, nullptr, nullptr, dpos, dq, (hipStream_t)s);
 }
 int mnx_pme_gather_f64(const double* pos, const double* q, const double* box, int64_t n, const double* grid,
                        int32_t gx, int32_t gy, int32_t gz, int32_t order, double coulomb, double* dpos, double* dq,
                        mnx_stream_t s) {
-    return gather<double>(pos, q, box, n, grid, gx, gy, gz, order, coulomb, dpos, dq, (hipStream_t)s);
+    return gather<double>(pos, q, box, n, grid, gx, gy, gz, order, coulomb, nullptr, nullptr, nullptr, dpos, dq, (hipStream_t)s);
 }
 size_t mnx_pme_direct_workspace_bytes(int64_t n, int64_t num_pairs) { return direct_ws(n, num_pairs) + 256; }
 int mnx_pme_direct_f32(const float* pos, const float* q, int64_t n, const int32_t* neighbors, int64_t num_pairs,
@@ -705,6 +838,27 @@ int mnx_pme_direct_f64(const double* pos, const double* q, int64_t n, const int3
                        size_t ws_bytes, mnx_stream_t s) {
     return direct<double>(pos, q, n, neighbors, num_pairs, deltas, distances, exclusions, max_excl, alpha, coulomb,
                           energy, dpos, dq, ws, ws_bytes, (hipStream_t)s);
+}
+
+int mnx_pme_convolve_add_f32(float* cgrid, const float* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
+                             const float* xm, const float* ym, const float* zm, const double* more, int64_t nmore,
+                             float* energy, void* ws, size_t ws_bytes, mnx_stream_t s) {
+    return convolve<float>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, more, nmore, energy, ws, ws_bytes, (hipStream_t)s);
+}
+int mnx_pme_gather_add_f32(const float* pos, const float* q, const float* box, int64_t n, const float* grid, int32_t gx,
+                           int32_t gy, int32_t gz, int32_t order, double coulomb, const float* grad, const float* dpos_add,
+                           const float* dq_add, float* dpos, float* dq, mnx_stream_t s) {
+    return gather<float>(pos, q, box, n, grid, gx, gy, gz, order, coulomb, grad, dpos_add, dq_add, dpos, dq, (hipStream_t)s);
+}
+int mnx_pme_convolve_add_f64(double* cgrid, const double* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
+                             const double* xm, const double* ym, const double* zm, const double* more, int64_t nmore,
+                             double* energy, void* ws, size_t ws_bytes, mnx_stream_t s) {
+    return convolve<double>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, more, nmore, energy, ws, ws_bytes, (hipStream_t)s);
+}
+int mnx_pme_gather_add_f64(const double* pos, const double* q, const double* box, int64_t n, const double* grid, int32_t gx,
+                           int32_t gy, int32_t gz, int32_t order, double coulomb, const double* grad, const double* dpos_add,
+                           const double* dq_add, double* dpos, double* dq, mnx_stream_t s) {
+    return gather<double>(pos, q, box, n, grid, gx, gy, gz, order, coulomb, grad, dpos_add, dq_add, dpos, dq, (hipStream_t)s);
 }
 
 }  // extern "C"

@@ -1,6 +1,8 @@
 // Device-wide exclusive prefix sum used by the cell list and the CSR builder.
 // Three launches: per-tile sums, one-block scan of the tile sums, per-tile
-// rescan with the tile's offset.  Deterministic (integer adds, fixed order).
+// rescan with the tile's offset; one launch of one workgroup up to kScanOne
+// elements (a few microseconds each either way, so the launches are what counts).
+// Deterministic (integer adds, fixed order).
 #pragma once
 
 #include "common.h"
@@ -97,6 +99,41 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_apply(const TIn* __restri
     }
 }
 
+constexpr int kScanOne = 1024 * 8;
+
+template <typename TIn, typename TOut>
+__global__ void __launch_bounds__(1024) k_scan_one(const TIn* __restrict__ in, int n, TOut* __restrict__ out,
+                                                   TOut* __restrict__ grand_total) {
+    __shared__ TOut sh[16];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+    const int base = int(threadIdx.x) * 8;
+    TOut v[8], s = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        v[k] = base + k < n ? TOut(in[base + k]) : TOut(0);
+        s += v[k];
+    }
+    TOut incl = s;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const TOut u = __shfl_up(incl, o, kWave);
+        if (lane >= o) incl += u;
+    }
+    if (lane == kWave - 1) sh[wave] = incl;
+    __syncthreads();
+    TOut run = incl - s, total = 0;
+    for (int w = 0; w < 16; ++w) {
+        if (w < wave) run += sh[w];
+        total += sh[w];
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        if (base + k < n) out[base + k] = run;
+        run += v[k];
+    }
+    if (threadIdx.x == 0 && grand_total) *grand_total = total;
+}
+
 inline size_t scan_workspace_elems(int64_t n) { return size_t(ceil_div(n > 0 ? n : 1, kScanTile)); }
 
 // out[k] = sum_{q<k} in[q] for k < n; *grand_total (device, may be null) = sum of all.
@@ -104,6 +141,11 @@ template <typename TIn, typename TOut>
 int exclusive_scan(const TIn* in, int64_t n, TOut* out, TOut* tile_ws, TOut* grand_total,
                    hipStream_t stream) {
     const int64_t ntiles = ceil_div(n > 0 ? n : 1, kScanTile);
+    if (n <= kScanOne) {
+        hipLaunchKernelGGL((k_scan_one<TIn, TOut>), dim3(1), dim3(1024), 0, stream, in, int(n), out, grand_total);
+        MNX_CHECK_LAUNCH();
+        return MNX_OK;
+    }
     if (ntiles > kScanMaxTiles) return set_error(MNX_ERR_INVALID, "scan length %lld too large", (long long)n);
     hipLaunchKernelGGL((k_scan_tile_sums<TIn, TOut>), dim3(ntiles), dim3(kScanThreads), 0, stream, in, n, tile_ws);
     MNX_CHECK_LAUNCH();

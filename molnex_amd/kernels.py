@@ -1016,6 +1016,123 @@ def _pme_spec_bwd(ctx, grad, _grad_spec):
 pme_reciprocal_spectrum.register_autograd(_pme_spec_bwd, setup_context=_pme_spec_setup)
 
 
+@torch.library.custom_op("molix::pme_energy", mutates_args=(), device_types="cuda")
+def pme_energy(positions: Tensor, charges: Tensor, box_vectors: Tensor, xmoduli: Tensor, ymoduli: Tensor,
+               zmoduli: Tensor, gridx: int, gridy: int, gridz: int, order: int, alpha: float, cutoff: float,
+               coulomb: float, gradients: bool) -> tuple[Tensor, Tensor, Tensor, Tensor]:
+    """The whole PME energy of a periodic system: the real-space sum over the pairs within ``cutoff``
+    (minimum image) and the self term straight from the cell scan (no pair list, no host read of its
+    length), plus the reciprocal sum of ``molix::pme_reciprocal``.
+
+    Returns ``(energy, spectrum, dpos, dq)``: the convolved half spectrum and, with ``gradients``, the
+    derivatives of the real-space and self terms (else empty), which the backward uses; those three
+    carry no gradient."""
+    _require_gpu("pme_energy", positions, charges, box_vectors)
+    lib = _lib.load()
+    sfx = _fsuffix(positions)
+    dt, dev, n = positions.dtype, positions.device, positions.shape[0]
+    pos = positions.detach().contiguous()
+    q = charges.detach().to(dt).contiguous()
+    b = box_vectors.detach().to(device=dev, dtype=dt).contiguous()
+    if tuple(b.shape) != (3, 3) or tuple(pos.shape) != (n, 3) or tuple(q.shape) != (n,):
+        raise ValueError("pme_energy: positions must be (n, 3), charges (n,) and box_vectors (3, 3)")
+    mods = [m.detach().to(device=dev, dtype=dt).contiguous() for m in (xmoduli, ymoduli, zmoduli)]
+    if any(m.numel() < g for m, g in zip(mods, (gridx, gridy, gridz))):
+        raise ValueError("moduli shorter than the grid")
+    stream = _stream(pos)
+    # scratch of the three stages in turn, behind the energy's partial sums and the neighbour flag
+    nparts = lib.mnx_pme_real_partials(n)
+    head = (8 * nparts + 8 + 255) // 256 * 256
+    ws = _ws(head + max(lib.mnx_nlist_workspace_bytes(n), lib.mnx_pme_spread_workspace_bytes(n, gridx, gridy, gridz),
+                        lib.mnx_pme_convolve_workspace_bytes(gridx, gridy, gridz)), dev)
+    parts, flag, scratch, size = ptr(ws), ptr(ws) + 8 * nparts, ptr(ws) + head, ws.numel() - head
+    dpos = torch.empty_like(pos) if gradients else pos.new_empty((0, 3))
+    dq = torch.empty_like(q) if gradients else q.new_empty((0,))
+    check(getattr(lib, f"mnx_pme_real_{sfx}")(ptr(pos), ptr(q), n, ptr(b), float(cutoff), float(alpha), float(coulomb),
+                                              ptr(dpos) if gradients else None, ptr(dq) if gradients else None, parts,
+                                              flag, scratch, size, stream), "pme real-space sum")
+    many = None
+    if n > 2048:  # the count of too many neighbours: read below, when it has long arrived
+        many = torch.empty(4, dtype=torch.uint8, pin_memory=True)
+        many.copy_(ws[8 * nparts:8 * nparts + 4], non_blocking=True)
+        arrived = torch.cuda.Event()
+        arrived.record()
+    grid = torch.empty((gridx, gridy, gridz), dtype=dt, device=dev)
+    check(getattr(lib, f"mnx_pme_spread_{sfx}")(ptr(pos), ptr(q), ptr(b), n, gridx, gridy, gridz, order, float(coulomb),
+                                                ptr(grid), scratch, size, stream), "pme spread")
+    spec = torch.fft.rfftn(grid).contiguous()
+    energy = torch.empty((), dtype=dt, device=dev)
+    check(getattr(lib, f"mnx_pme_convolve_add_{sfx}")(
+        ptr(torch.view_as_real(spec)), ptr(b), gridx, gridy, gridz, float(alpha), ptr(mods[0]), ptr(mods[1]),
+        ptr(mods[2]), parts, nparts, ptr(energy), scratch, size, stream), "pme convolve")
+    if many is not None:
+        arrived.synchronize()
+        if int(many.view(torch.int32)[0]):
+            raise _lib.MolnexError("neighbor list: an atom has more than 4096 neighbours within the cutoff")
+    return energy, spec, dpos, dq
+
+
+@pme_energy.register_fake
+def _(positions, charges, box_vectors, xmoduli, ymoduli, zmoduli, gridx, gridy, gridz, order, alpha, cutoff, coulomb,
+      gradients):
+    cdt = torch.complex128 if positions.dtype == torch.float64 else torch.complex64
+    n = positions.shape[0] if gradients else 0
+    return (positions.new_empty(()), positions.new_empty((gridx, gridy, gridz // 2 + 1), dtype=cdt),
+            positions.new_empty((n, 3)), positions.new_empty((n,)))
+
+
+@torch.library.custom_op("molix::pme_energy_backward", mutates_args=(), device_types="cuda")
+def pme_energy_backward(grad: Tensor, positions: Tensor, charges: Tensor, box_vectors: Tensor, spectrum: Tensor,
+                        dpos: Tensor, dq: Tensor, gridx: int, gridy: int, gridz: int, order: int, alpha: float,
+                        cutoff: float, coulomb: float) -> tuple[Tensor, Tensor]:
+    """``grad`` times (dE/dpos, dE/dq) of ``molix::pme_energy`` from its other outputs."""
+    _require_gpu("pme_energy_backward", grad, positions, charges, box_vectors, spectrum)
+    lib = _lib.load()
+    sfx = _fsuffix(positions)
+    dt, dev, n = positions.dtype, positions.device, positions.shape[0]
+    pos = positions.detach().contiguous()
+    q = charges.detach().to(dt).contiguous()
+    b = box_vectors.detach().to(device=dev, dtype=dt).contiguous()
+    if spectrum.shape != (gridx, gridy, gridz // 2 + 1) or not spectrum.is_complex():
+        raise ValueError("pme_energy_backward: spectrum must be complex (gridx, gridy, gridz // 2 + 1)")
+    if dpos.shape[0] != n:  # the forward was told that no gradient is wanted
+        dpos, dq = torch.empty_like(pos), torch.empty_like(q)
+        parts = torch.empty(lib.mnx_pme_real_partials(n) + 1, dtype=torch.float64, device=dev)
+        ws = _ws(lib.mnx_nlist_workspace_bytes(n), dev)
+        check(getattr(lib, f"mnx_pme_real_{sfx}")(ptr(pos), ptr(q), n, ptr(b), float(cutoff), float(alpha),
+                                                  float(coulomb), ptr(dpos), ptr(dq), ptr(parts),
+                                                  ptr(parts) + 8 * (parts.numel() - 1), ptr(ws), ws.numel(),
+                                                  _stream(pos)), "pme real-space sum")
+    real = torch.fft.irfftn(spectrum, s=(gridx, gridy, gridz), norm="forward").contiguous()
+    gpos, gq = torch.empty_like(pos), torch.empty_like(q)
+    check(getattr(lib, f"mnx_pme_gather_add_{sfx}")(
+        ptr(pos), ptr(q), ptr(b), n, ptr(real), gridx, gridy, gridz, order, float(coulomb), ptr(grad.to(dt).contiguous()),
+        ptr(dpos.contiguous()), ptr(dq.contiguous()), ptr(gpos), ptr(gq), _stream(pos)), "pme gather")
+    return gpos, gq
+
+
+@pme_energy_backward.register_fake
+def _(grad, positions, charges, box_vectors, spectrum, dpos, dq, gridx, gridy, gridz, order, alpha, cutoff, coulomb):
+    return torch.empty_like(positions), torch.empty_like(charges)
+
+
+def _pme_energy_setup(ctx, inputs, output):
+    ctx.set_materialize_grads(False)
+    ctx.mark_non_differentiable(*output[1:])
+    ctx.save_for_backward(*inputs[:3], *output[1:])
+    ctx.args = tuple(inputs[6:13])
+
+
+def _pme_energy_bwd(ctx, grad, *_):
+    if grad is None:
+        return (None,) * 14
+    gpos, gq = pme_energy_backward(grad, *ctx.saved_tensors, *ctx.args)
+    return (gpos, gq) + (None,) * 12
+
+
+pme_energy.register_autograd(_pme_energy_bwd, setup_context=_pme_energy_setup)
+
+
 def _pme_direct_run(positions, charges, neighbors, deltas, distances, exclusions, alpha, coulomb, grads=True):
     """Energy, and (dE/dpos, dE/dq) when ``grads`` (else None, None: no derivative atomics)."""
     lib = _lib.load()

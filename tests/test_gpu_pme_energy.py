@@ -1,0 +1,119 @@
+"""molix::pme_energy (the whole PME term in one op) against the ops it stands for: the neighbor list's pairs
+through molix::pme_direct, molix::pme_reciprocal and the self term, in float64, over the paths of its pair
+scan (all pairs, cells, crowded cells, all-pairs grids) and the mesh kernels' orders and edges."""
+
+import math
+
+import pytest
+import torch
+
+import molnex_amd.kernels  # noqa: F401
+from molnex_amd.molpot import PMEPotential
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _composed(pme, pos, q, box):
+    """The module's form for given pairs, in float64."""
+    pos, q, box = (t.detach().double() for t in (pos, q, box))
+    pos.requires_grad_(True), q.requires_grad_(True)
+    i, j, _, d, r = torch.ops.molix.neighbor_list(pos.detach(), pme.cutoff, box, False)
+    e = pme(pos, q, box, pairs=(torch.stack([i, j]), d, r))
+    gp, gq = torch.autograd.grad(e, (pos, q))
+    return e.detach(), gp, gq
+
+
+def _run(pme, pos, q, box):
+    p, c = pos.clone().requires_grad_(True), q.clone().requires_grad_(True)
+    e = pme(p, c, box)
+    gp, gq = torch.autograd.grad(e, (p, c))
+    return e.detach(), gp, gq
+
+
+def _close(got, want, tol, terms=0.0):
+    """``terms``: the size of the terms a result is the difference of.  The mesh force of an atom on itself,
+    for one, is order^3 terms of size k q^2 alpha that cancel to the spline's error; their rounding stays."""
+    for a, b in zip(got, want):
+        assert a.shape == b.shape
+        bound = tol * b.norm().item() + torch.finfo(a.dtype).eps / 2 * terms
+        assert (a.double() - b).norm() <= bound, ((a.double() - b).norm(), b.norm())
+
+
+def _system(n, edge, seed, box=None):
+    g = torch.Generator().manual_seed(seed)
+    box = torch.eye(3, dtype=torch.float64) * edge if box is None else box
+    k = math.ceil(n ** (1 / 3))
+    grid = torch.stack(torch.meshgrid(*[torch.arange(k)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    sites = grid[torch.randperm(k ** 3, generator=g)[:n]].double()
+    # jittered lattice: pairs stay apart, so no single 1/r term decides the result
+    pos = ((sites + 0.25 + 0.5 * torch.rand(n, 3, generator=g, dtype=torch.float64)) / k) @ box
+    q = torch.randn(n, generator=g, dtype=torch.float64)
+    return pos.to(DEV), (q - q.mean() if n > 1 else q).to(DEV), box.to(DEV)
+
+
+# float64: both sides sum the same terms in other orders.  float32: positions and charges are rounded
+# identically for both sides (the oracle gets the rounded values); mesh sums of ~order^3 terms at 2^-24.
+@pytest.mark.parametrize("dtype,tol", [(torch.float64, 1e-11), (torch.float32, 2e-5)])
+@pytest.mark.parametrize("n,edge,cut,mesh,order,kind", [
+    (1, 9.0, 3.0, (16, 16, 16), 4, "cubic"),
+    (2, 9.0, 4.0, (12, 16, 20), 5, "cubic"),
+    (130, 11.0, 5.0, (16, 17, 18), 6, "cubic"),         # under three cutoffs: exact images only
+    (700, 19.0, 5.0, (9, 11, 8), 8, "cubic"),           # a mesh of one brick and a bit
+    (2047, 27.0, 4.0, (24, 24, 24), 3, "cubic"),
+    (2049, 27.0, 4.0, (26, 30, 28), 7, "triclinic"),    # the cell scan
+    (4000, 22.0, 5.0, (32, 32, 32), 4, "cubic"),        # about 200 neighbours
+    (3000, 30.0, 4.0, (16, 64, 16), 5, "thin"),         # two cells along one axis: an all-pairs grid
+])
+def test_energy_and_gradients(n, edge, cut, mesh, order, kind, dtype, tol):
+    box = None
+    if kind == "triclinic":
+        box = torch.tensor([[edge, 0, 0], [0.2 * edge, edge, 0], [-0.1 * edge, 0.3 * edge, edge]], dtype=torch.float64)
+    if kind == "thin":
+        box = torch.diag(torch.tensor([edge, 3 * edge, 9.0], dtype=torch.float64))
+    pos, q, box = (t.to(dtype) for t in _system(n, edge, n + order, box))
+    pme = PMEPotential(alpha=0.4, grid=mesh, order=order, cutoff=cut).to(DEV)
+    want = _composed(pme, pos, q, box)
+    got = _run(pme, pos, q, box)
+    _close(got, want, tol, pme.coulomb * pme.alpha * float((q.double() ** 2).sum()))
+    # bitwise the same again where the sums have a fixed order (all pairs); the cell scan's lists arrive in
+    # any order, and its fp64 sums differ in their last bits
+    again = _run(pme, pos, q, box)
+    if n <= 2048:
+        assert all(torch.equal(a, b) for a, b in zip(got, again))
+    else:
+        _close(again, [t.double() for t in got], tol)
+
+
+def test_single_gradients_scaling_and_no_grad():
+    pos, q, box = (t.float() for t in _system(600, 18.0, 1))
+    pme = PMEPotential(alpha=0.35, grid=(20, 20, 20), order=5, cutoff=4.5).to(DEV)
+    e, gp, gq = _run(pme, pos, q, box)
+    with torch.no_grad():
+        assert torch.equal(pme(pos, q, box), e)
+    p = pos.clone().requires_grad_(True)
+    (only,) = torch.autograd.grad(3.0 * pme(p, q, box), p)
+    torch.testing.assert_close(only, 3.0 * gp, rtol=1e-6, atol=1e-6)
+    c = q.clone().requires_grad_(True)
+    (only,) = torch.autograd.grad(pme(pos, c, box), c)
+    torch.testing.assert_close(only, gq, rtol=1e-6, atol=1e-6)
+    # the forward told that no gradient is wanted: the backward forms the real-space part itself
+    spec = torch.ops.molix.pme_energy(pos, q, box, *pme._moduli(torch.float32), 20, 20, 20, 5, 0.35, 4.5, pme.coulomb, False)
+    got = torch.ops.molix.pme_energy_backward(torch.ones((), device=DEV), pos, q, box, *spec[1:], 20, 20, 20, 5, 0.35, 4.5,
+                                              pme.coulomb)
+    assert torch.equal(got[0], gp) and torch.equal(got[1], gq)
+
+
+def test_too_many_neighbours_is_refused():
+    pos = torch.rand(4300, 3, device=DEV) * 2.0
+    pme = PMEPotential(alpha=0.3, grid=(16, 16, 16), order=4, cutoff=4.0).to(DEV)
+    with pytest.raises(RuntimeError, match="4096"):
+        pme(pos, torch.zeros(4300, device=DEV), torch.eye(3, device=DEV) * 20.0)
+
+
+def test_opcheck():
+    pos, q, box = _system(150, 12.0, 5)
+    pme = PMEPotential(alpha=0.4, grid=(16, 16, 16), order=4, cutoff=3.5).to(DEV)
+    pos.requires_grad_(True), q.requires_grad_(True)
+    torch.library.opcheck(torch.ops.molix.pme_energy.default,
+                          (pos, q, box, *pme._moduli(torch.float64), 16, 16, 16, 4, 0.4, 3.5, 1.0, True))
