@@ -39,6 +39,7 @@ from torch import Tensor
 
 from . import _lib
 from ._lib import check, ptr
+from ._ops import op as _op
 from .config import config as _settings
 
 MNX_NLIST_HALF, MNX_NLIST_FULL = 0, 1
@@ -101,10 +102,8 @@ def _prep_positions(positions: Tensor, box_vectors: Tensor):
     return pos, box
 
 
-@torch.library.custom_op(
+@_op(
     "molix::get_neighbor_pairs",
-    mutates_args=(),
-    device_types="cuda",
     schema="(Tensor positions, Scalar cutoff, Scalar max_num_pairs, Tensor box_vectors) -> "
     "(Tensor neighbors, Tensor deltas, Tensor distances, Tensor num_pairs)",
 )
@@ -151,7 +150,7 @@ def _(positions, cutoff, max_num_pairs, box_vectors):
     )
 
 
-@torch.library.custom_op("molix::get_neighbor_pairs_backward", mutates_args=(), device_types="cuda")
+@_op("molix::get_neighbor_pairs_backward")
 def get_neighbor_pairs_backward(neighbors: Tensor, deltas: Tensor, distances: Tensor, grad_deltas: Tensor,
                                 grad_distances: Tensor, num_atoms: int) -> Tensor:
     """d/d positions of <g_deltas, deltas> + <g_dist, distances> (``get_neighbor_pairs.cu:81-102``)."""
@@ -191,7 +190,7 @@ def _gnp_backward(ctx, g_neighbors, g_deltas, g_distances, g_num):
 get_neighbor_pairs.register_autograd(_gnp_backward, setup_context=_gnp_setup)
 
 
-@torch.library.custom_op("molix::neighbor_list", mutates_args=(), device_types="cuda")
+@_op("molix::neighbor_list")
 def neighbor_list(positions: Tensor, cutoff: float, box_vectors: Tensor, full: bool) -> tuple[
         Tensor, Tensor, Tensor, Tensor, Tensor]:
     """Exact-size cell list sorted by (i, j): ``full`` gives all ordered pairs i != j,
@@ -234,7 +233,7 @@ def _f32_rows(t: Tensor, width: int, what: str) -> Tensor:
     return t.reshape(-1, width).contiguous()
 
 
-@torch.library.custom_op("molix::spherical_harmonics", mutates_args=(), device_types="cuda")
+@_op("molix::spherical_harmonics")
 def spherical_harmonics(vectors: Tensor, l_max: int) -> Tensor:
     """Real harmonics ``[Y^0 .. Y^l_max]`` of normalised ``vectors`` (..., 3)."""
     _require_gpu("spherical_harmonics", vectors)
@@ -250,7 +249,7 @@ def _(vectors, l_max):
     return vectors.new_empty((*vectors.shape[:-1], (l_max + 1) ** 2))
 
 
-@torch.library.custom_op("molix::spherical_harmonics_backward", mutates_args=(), device_types="cuda")
+@_op("molix::spherical_harmonics_backward")
 def spherical_harmonics_backward(vectors: Tensor, grad: Tensor, l_max: int) -> Tensor:
     v = _f32_rows(vectors, 3, "vectors")
     d = (l_max + 1) ** 2
@@ -284,7 +283,7 @@ spherical_harmonics.register_autograd(_sh_backward, setup_context=_sh_setup)
 # ---------------------------------------------------------------------------
 
 
-@torch.library.custom_op("molix::edge_csr", mutates_args=(), device_types="cuda")
+@_op("molix::edge_csr")
 def edge_csr(edge_index: Tensor, num_nodes: int, validate: bool = True) -> tuple[Tensor, Tensor, Tensor]:
     """Receiver CSR of ``edge_index`` (E, 2) = [sender, receiver]: ``(row_ptr, perm, senders)``.
 
@@ -339,7 +338,7 @@ def _check_wrow(wrow: Tensor | None, E: int, Ew: int, what: str) -> None:
         raise ValueError(f"{what}: wrow must be a contiguous int32 ({E},) tensor")
 
 
-@torch.library.custom_op("molix::tp_scatter", mutates_args=(), device_types="cuda")
+@_op("molix::tp_scatter")
 def tp_scatter(x: Tensor, Y: Tensor, w: Tensor, row_ptr: Tensor, perm: Tensor, senders: Tensor, config: int,
                channels: int, s_row_ptr: Tensor | None = None, s_perm: Tensor | None = None,
                s_receivers: Tensor | None = None, wrow: Tensor | None = None) -> Tensor:
@@ -374,7 +373,7 @@ def _(x, Y, w, row_ptr, perm, senders, config, channels, s_row_ptr=None, s_perm=
     return x.new_empty((row_ptr.shape[0] - 1, no * channels))
 
 
-@torch.library.custom_op("molix::tp_scatter_backward", mutates_args=(), device_types="cuda")
+@_op("molix::tp_scatter_backward")
 def tp_scatter_backward(grad_out: Tensor, x: Tensor, Y: Tensor, w: Tensor, row_ptr: Tensor, perm: Tensor,
                         senders: Tensor, config: int, channels: int, need_x: bool, need_Y: bool,
                         need_w: bool, s_row_ptr: Tensor | None = None, s_perm: Tensor | None = None,
@@ -470,7 +469,7 @@ def _any_ctable(table: list[int]):
     return (C.c_int32 * len(table))(*table), len(table)
 
 
-@torch.library.custom_op("molix::tp_any", mutates_args=(), device_types="cuda")
+@_op("molix::tp_any")
 def tp_any(x: Tensor, Y: Tensor, w: Tensor, row_ptr: Tensor, perm: Tensor, senders: Tensor,
            table: list[int]) -> Tensor:
     """``out[r] = sum_{e -> r} TP(x[send(e)], Y[e]; w[e])`` for any irreps with l <= 3, driven by the
@@ -499,7 +498,7 @@ def _(x, Y, w, row_ptr, perm, senders, table):
     return x.new_empty((row_ptr.shape[0] - 1, table[3]))
 
 
-@torch.library.custom_op("molix::tp_any_backward", mutates_args=(), device_types="cuda")
+@_op("molix::tp_any_backward")
 def tp_any_backward(grad_out: Tensor, x: Tensor, Y: Tensor, w: Tensor, row_ptr: Tensor, perm: Tensor,
                     senders: Tensor, table: list[int], need_x: bool, need_Y: bool,
                     need_w: bool) -> tuple[Tensor, Tensor, Tensor]:
@@ -582,7 +581,7 @@ def edge_tp_out_rows(ls: list[int]) -> list[int]:
     return rows
 
 
-@torch.library.custom_op("molix::edge_tp", mutates_args=(), device_types="cuda")
+@_op("molix::edge_tp")
 def edge_tp(x: Tensor, Y: Tensor, w: Tensor, config: int, channels: int, x_scale: Tensor | None = None) -> Tensor:
     """``out[e] = TP(s[e] * x[e], Y[e]; w)``: per-edge channelwise product with weights shared by
     all edges (``w`` is ``(num_paths, C)``), no scatter -- Allegro's layer product
@@ -612,7 +611,7 @@ def _(x, Y, w, config, channels, x_scale=None):
     return x.new_empty((Y.shape[0], no * channels))
 
 
-@torch.library.custom_op("molix::edge_tp_backward", mutates_args=(), device_types="cuda")
+@_op("molix::edge_tp_backward")
 def edge_tp_backward(grad_out: Tensor, x: Tensor, Y: Tensor, w: Tensor, config: int, channels: int,
                      need_x: bool, need_Y: bool, need_w: bool, x_scale: Tensor | None = None,
                      need_scale: bool = False) -> tuple[Tensor, Tensor, Tensor, Tensor]:
@@ -725,7 +724,7 @@ def _proj_args(x, Y, w, config, proj, x_scale, x_scale2=None):
     return blocks, xs, int(shared), Ys, ws_, pj, sc, sc2, ni
 
 
-@torch.library.custom_op("molix::edge_tp_proj", mutates_args=(), device_types="cuda")
+@_op("molix::edge_tp_proj")
 def edge_tp_proj(x: Tensor, Y: Tensor, w: Tensor, config: int, proj: Tensor,
                  x_scale: Tensor | None = None, x_scale2: Tensor | None = None) -> Tensor:
     """``molix::edge_tp`` with 16 channels followed by the projection back to the input irreps
@@ -755,7 +754,7 @@ def _(x, Y, w, config, proj, x_scale=None, x_scale2=None):
     return x.new_empty((Y.shape[0], ni * 16))
 
 
-@torch.library.custom_op("molix::edge_tp_proj_backward", mutates_args=(), device_types="cuda")
+@_op("molix::edge_tp_proj_backward")
 def edge_tp_proj_backward(grad_out: Tensor, x: Tensor, Y: Tensor, w: Tensor, config: int, proj: Tensor,
                           need_x: bool, need_Y: bool, need_w: bool, x_scale: Tensor | None = None,
                           need_scale: bool = False, x_scale2: Tensor | None = None,
@@ -897,7 +896,7 @@ def _pme_recip_energy(positions, charges, box, gx, gy, gz, order, alpha, coulomb
     return energy, spec, pos, q, b
 
 
-@torch.library.custom_op("molix::pme_reciprocal", mutates_args=(), device_types="cuda", schema=_PME_RECIP_SCHEMA)
+@_op("molix::pme_reciprocal", schema=_PME_RECIP_SCHEMA)
 def pme_reciprocal(positions, charges, box_vectors, gridx, gridy, gridz, order, alpha, coulomb, xmoduli, ymoduli,
                    zmoduli):
     """Reciprocal-space PME energy (reference ``pme_cpu.cpp:220-296,378``): B-spline spread on the GPU,
@@ -913,7 +912,7 @@ def _(positions, charges, box_vectors, gridx, gridy, gridz, order, alpha, coulom
     return positions.new_empty(())
 
 
-@torch.library.custom_op("molix::pme_reciprocal_backward", mutates_args=(), device_types="cuda")
+@_op("molix::pme_reciprocal_backward")
 def pme_reciprocal_backward(positions: Tensor, charges: Tensor, box_vectors: Tensor, gridx: int, gridy: int,
                             gridz: int, order: int, alpha: float, coulomb: float, xmoduli: Tensor, ymoduli: Tensor,
                             zmoduli: Tensor) -> tuple[Tensor, Tensor]:
@@ -959,7 +958,7 @@ def _pme_recip_bwd(ctx, grad):
 pme_reciprocal.register_autograd(_pme_recip_bwd, setup_context=_pme_recip_setup)
 
 
-@torch.library.custom_op("molix::pme_reciprocal_spectrum", mutates_args=(), device_types="cuda")
+@_op("molix::pme_reciprocal_spectrum")
 def pme_reciprocal_spectrum(positions: Tensor, charges: Tensor, box_vectors: Tensor, gridx: int, gridy: int,
                             gridz: int, order: int, alpha: float, coulomb: float, xmoduli: Tensor, ymoduli: Tensor,
                             zmoduli: Tensor) -> tuple[Tensor, Tensor]:
@@ -979,7 +978,7 @@ def _(positions, charges, box_vectors, gridx, gridy, gridz, order, alpha, coulom
     return positions.new_empty(()), positions.new_empty((gridx, gridy, gridz // 2 + 1), dtype=cdt)
 
 
-@torch.library.custom_op("molix::pme_reciprocal_gather", mutates_args=(), device_types="cuda")
+@_op("molix::pme_reciprocal_gather")
 def pme_reciprocal_gather(positions: Tensor, charges: Tensor, box_vectors: Tensor, spectrum: Tensor, gridx: int,
                           gridy: int, gridz: int, order: int, coulomb: float) -> tuple[Tensor, Tensor]:
     """(dE/dpos, dE/dq) of ``molix::pme_reciprocal_spectrum`` from its spectrum output."""
@@ -1016,7 +1015,7 @@ def _pme_spec_bwd(ctx, grad, _grad_spec):
 pme_reciprocal_spectrum.register_autograd(_pme_spec_bwd, setup_context=_pme_spec_setup)
 
 
-@torch.library.custom_op("molix::pme_energy", mutates_args=(), device_types="cuda")
+@_op("molix::pme_energy")
 def pme_energy(positions: Tensor, charges: Tensor, box_vectors: Tensor, xmoduli: Tensor, ymoduli: Tensor,
                zmoduli: Tensor, gridx: int, gridy: int, gridz: int, order: int, alpha: float, cutoff: float,
                coulomb: float, gradients: bool) -> tuple[Tensor, Tensor, Tensor, Tensor]:
@@ -1081,7 +1080,7 @@ def _(positions, charges, box_vectors, xmoduli, ymoduli, zmoduli, gridx, gridy, 
             positions.new_empty((n, 3)), positions.new_empty((n,)))
 
 
-@torch.library.custom_op("molix::pme_energy_backward", mutates_args=(), device_types="cuda")
+@_op("molix::pme_energy_backward")
 def pme_energy_backward(grad: Tensor, positions: Tensor, charges: Tensor, box_vectors: Tensor, spectrum: Tensor,
                         dpos: Tensor, dq: Tensor, gridx: int, gridy: int, gridz: int, order: int, alpha: float,
                         cutoff: float, coulomb: float) -> tuple[Tensor, Tensor]:
@@ -1159,7 +1158,7 @@ def _pme_direct_run(positions, charges, neighbors, deltas, distances, exclusions
     return energy, dpos, dq
 
 
-@torch.library.custom_op("molix::pme_direct", mutates_args=(), device_types="cuda", schema=_PME_DIRECT_SCHEMA)
+@_op("molix::pme_direct", schema=_PME_DIRECT_SCHEMA)
 def pme_direct(positions, charges, neighbors, deltas, distances, exclusions, alpha, coulomb):
     """Real-space PME energy over a pair list minus excluded pairs (reference ``pme_cpu.cpp:95-216``).
     Like the reference, the gradient w.r.t. positions is the analytic one through the pair
@@ -1175,7 +1174,7 @@ def _(positions, charges, neighbors, deltas, distances, exclusions, alpha, coulo
     return positions.new_empty(())
 
 
-@torch.library.custom_op("molix::pme_direct_backward", mutates_args=(), device_types="cuda")
+@_op("molix::pme_direct_backward")
 def pme_direct_backward(positions: Tensor, charges: Tensor, neighbors: Tensor, deltas: Tensor, distances: Tensor,
                         exclusions: Tensor, alpha: float, coulomb: float) -> tuple[Tensor, Tensor]:
     _, dpos, dq = _pme_direct_run(positions, charges, neighbors, deltas, distances, exclusions, alpha, coulomb)
@@ -1206,7 +1205,7 @@ pme_direct.register_autograd(_pme_direct_bwd, setup_context=_pme_direct_setup)
 # ---------------------------------------------------------------------------
 
 
-@torch.library.custom_op("molix::symmetric_contraction_scalar", mutates_args=(), device_types="cuda")
+@_op("molix::symmetric_contraction_scalar")
 def symmetric_contraction_scalar(x: Tensor, atom_types: Tensor, weight: Tensor) -> Tensor:
     """``out[n, c] = sum_k weight[z_n, k, c] x[n, c]^(k+1)``; weight ``(S, degree, D)``."""
     _require_gpu("symmetric_contraction_scalar", x, atom_types, weight)
@@ -1225,7 +1224,7 @@ def _(x, atom_types, weight):
     return torch.empty_like(x)
 
 
-@torch.library.custom_op("molix::symmetric_contraction_scalar_backward", mutates_args=(), device_types="cuda")
+@_op("molix::symmetric_contraction_scalar_backward")
 def symmetric_contraction_scalar_backward(grad: Tensor, x: Tensor, atom_types: Tensor, weight: Tensor,
                                           need_x: bool, need_w: bool) -> tuple[Tensor, Tensor]:
     S, nu, D = weight.shape
@@ -1291,7 +1290,7 @@ def _sc_shapes(x, weight, l_in, l_out, correlation):
     return cfg, ni, no, S, Cc
 
 
-@torch.library.custom_op("molix::symmetric_contraction", mutates_args=(), device_types="cuda")
+@_op("molix::symmetric_contraction")
 def symmetric_contraction(x: Tensor, atom_types: Tensor, weight: Tensor, l_in: int, l_out: int,
                           correlation: int) -> Tensor:
     """B = sum_{nu<=correlation} U_nu . W[z] (x^{(x)nu}); x (N, (l_in+1)^2 C) ir_mul, weight
@@ -1312,7 +1311,7 @@ def _(x, atom_types, weight, l_in, l_out, correlation):
     return x.new_empty(*x.shape[:-1], (l_out + 1) ** 2 * weight.shape[-1])
 
 
-@torch.library.custom_op("molix::symmetric_contraction_backward", mutates_args=(), device_types="cuda")
+@_op("molix::symmetric_contraction_backward")
 def symmetric_contraction_backward(grad: Tensor, x: Tensor, atom_types: Tensor, weight: Tensor, l_in: int,
                                    l_out: int, correlation: int, need_x: bool,
                                    need_w: bool) -> tuple[Tensor, Tensor]:
@@ -1337,7 +1336,7 @@ def _(grad, x, atom_types, weight, l_in, l_out, correlation, need_x, need_w):
             torch.empty_like(weight) if need_w else weight.new_empty(0))
 
 
-@torch.library.custom_op("molix::symmetric_contraction_backward2", mutates_args=(), device_types="cuda")
+@_op("molix::symmetric_contraction_backward2")
 def symmetric_contraction_backward2(grad: Tensor, x: Tensor, atom_types: Tensor, weight: Tensor,
                                     seed_x: Tensor | None, seed_w: Tensor | None, l_in: int, l_out: int,
                                     correlation: int, need_grad: bool, need_x: bool,
@@ -1412,7 +1411,7 @@ def _radial_frag(params: Tensor, kin: int, hidden: int, layers: int) -> Tensor:
     return frag
 
 
-@torch.library.custom_op("molix::radial_hidden", mutates_args=(), device_types="cuda")
+@_op("molix::radial_hidden")
 def radial_hidden(feats: Tensor, params: Tensor, kin: int, hidden: int, layers: int) -> Tensor:
     """``mlp[:-1](feats)`` of ``RadialWeightMLP`` (``radial_mlp.py:38-93``: [Linear -> SiLU] x layers)
     in one HIP kernel.  ``params`` = concatenated ``W_j.flatten(), b_j`` of the hidden Linears."""
@@ -1432,7 +1431,7 @@ def _(feats, params, kin, hidden, layers):
     return feats.new_empty(feats.shape[0], hidden)
 
 
-@torch.library.custom_op("molix::radial_hidden_backward", mutates_args=(), device_types="cuda")
+@_op("molix::radial_hidden_backward")
 def radial_hidden_backward(grad: Tensor, feats: Tensor, params: Tensor, kin: int, hidden: int,
                            layers: int) -> Tensor:
     """dL/dfeats of ``radial_hidden`` (forward recomputed in registers)."""
@@ -1510,7 +1509,7 @@ def _ew_frag(weight: Tensor, backward: bool) -> Tensor:
     return frag
 
 
-@torch.library.custom_op("molix::edge_weights", mutates_args=(), device_types="cuda")
+@_op("molix::edge_weights")
 def edge_weights(h: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     """``h @ weight.T + bias``: the last Linear of ``RadialWeightMLP`` (``radial_mlp.py:38-93``) mapping
     the (E, K) hidden activations to the (E, N) per-edge tensor-product weights.  Near-fp32: rows of
@@ -1551,7 +1550,7 @@ def _edge_weights_rows(h: Tensor, rows: Tensor, weight: Tensor, bias: Tensor | N
     return out
 
 
-@torch.library.custom_op("molix::edge_weights_backward", mutates_args=(), device_types="cuda")
+@_op("molix::edge_weights_backward")
 def edge_weights_backward(grad: Tensor, weight: Tensor) -> Tensor:
     """``grad @ weight``: dL/dh of ``edge_weights`` (same split-fp16 arithmetic)."""
     N, K = weight.shape
@@ -1619,7 +1618,7 @@ def _rows_f32(t: Tensor, what: str) -> Tensor:
     return t if ok else t.contiguous()
 
 
-@torch.library.custom_op("molix::tall_tn", mutates_args=(), device_types="cuda")
+@_op("molix::tall_tn")
 def tall_tn(a: Tensor, b: Tensor) -> Tensor:
     """``a.T @ b`` for tall float32 ``a`` (K, M) and ``b`` (K, N), K >> M, N: a layer's weight
     gradient summed over all edges, fp32-accurate on the bf16 matrix cores (split operands),
@@ -1655,7 +1654,7 @@ def _tall_bwd(ctx, g):
 tall_tn.register_autograd(_tall_bwd, setup_context=_tall_setup)
 
 
-@torch.library.custom_op("molix::tall_tn_colsum", mutates_args=(), device_types="cuda")
+@_op("molix::tall_tn_colsum")
 def tall_tn_colsum(a: Tensor, b: Tensor) -> tuple[Tensor, Tensor]:
     """``(a.T @ b, a.sum(0))`` from one pass over ``a`` (``tall_tn`` with the column sums of ``a``:
     a layer's weight and bias gradients)."""
@@ -1744,7 +1743,7 @@ def tp_weight_grad_supported(config: int, channels: int, hidden: int) -> bool:
     return config >= 0 and channels % 16 == 0 and hidden in (16, 32, 64, 128)
 
 
-@torch.library.custom_op("molix::tp_weight_grad", mutates_args=(), device_types="cuda")
+@_op("molix::tp_weight_grad")
 def tp_weight_grad(x: Tensor, Y: Tensor, grad_out: Tensor, edge_index: Tensor, weight: Tensor, config: int,
                    channels: int) -> Tensor:
     """``grad_h = gw @ weight`` for the per-edge weights ``w = h @ weight.T + b`` of a
@@ -1774,7 +1773,7 @@ def _(x, Y, grad_out, edge_index, weight, config, channels):
     return x.new_empty(Y.shape[0], weight.shape[1])
 
 
-@torch.library.custom_op("molix::radial_tp", mutates_args=(), device_types="cuda")
+@_op("molix::radial_tp")
 def radial_tp(x: Tensor, Y: Tensor, h: Tensor, weight: Tensor, bias: Tensor | None, row_ptr: Tensor, perm: Tensor,
               senders: Tensor, edge_index: Tensor, config: int, channels: int) -> tuple[Tensor, Tensor]:
     """``tp_scatter(x, Y, w)`` with ``w = h @ weight.T + bias`` (the radial MLP's output layer,
@@ -1830,7 +1829,7 @@ radial_tp.register_autograd(_rtp_backward, setup_context=_rtp_setup)
 # ---------------------------------------------------------------------------
 
 
-@torch.library.custom_op("molix::edge_reverse", mutates_args=(), device_types="cuda")
+@_op("molix::edge_reverse")
 def edge_reverse(edge_index: Tensor, num_nodes: int, row_ptr: Tensor, perm: Tensor, senders: Tensor,
                  feats: Tensor) -> tuple[Tensor, Tensor]:
     """``(rev, bad)``: ``rev[e]`` (int32) is the edge that runs opposite to e (sender and receiver
@@ -1898,7 +1897,7 @@ class EdgePairs:
         return int(bad.item()) == 0
 
 
-@torch.library.custom_op("molix::gather_rows", mutates_args=(), device_types="cuda")
+@_op("molix::gather_rows")
 def gather_rows(src: Tensor, idx: Tensor) -> Tensor:
     """``src[idx]`` for a float32 (R, F) ``src`` and int64 indices (the radial features of the lead
     edge of each undirected pair; Allegro's type-pair embedding rows).  Its backward scatters the
@@ -1920,7 +1919,7 @@ def _(src, idx):
     return src.new_empty(idx.shape[0], src.shape[1])
 
 
-@torch.library.custom_op("molix::scatter_rows", mutates_args=(), device_types="cuda")
+@_op("molix::scatter_rows")
 def scatter_rows(grad: Tensor, idx: Tensor, num_rows: int) -> Tensor:
     """The adjoint of ``gather_rows``: a (num_rows, F) tensor with ``grad[i]`` at row ``idx[i]``, zero
     elsewhere (indices distinct)."""
@@ -1963,7 +1962,7 @@ def _sr_backward(ctx, grad):
 scatter_rows.register_autograd(_sr_backward, setup_context=_sr_setup)
 
 
-@torch.library.custom_op("molix::edge_weights_backward_pairs", mutates_args=(), device_types="cuda")
+@_op("molix::edge_weights_backward_pairs")
 def edge_weights_backward_pairs(grad: Tensor, pairs: Tensor, weight: Tensor) -> Tensor:
     """``(grad[pairs[:, 0]] + grad[pairs[:, 1]]) @ weight``: dL/dh of an output layer applied once per
     undirected pair, from the per-edge weight gradient (same split-fp16 arithmetic as
@@ -1986,7 +1985,7 @@ def _(grad, pairs, weight):
     return grad.new_empty(pairs.shape[0], weight.shape[1])
 
 
-@torch.library.custom_op("molix::pair_sum_rows", mutates_args=(), device_types="cuda")
+@_op("molix::pair_sum_rows")
 def pair_sum_rows(src: Tensor, pairs: Tensor) -> Tensor:
     """``src[pairs[:, 0]] + src[pairs[:, 1]]`` for int32 (P, 2) pairs and rows of a multiple of 4 floats
     (one kernel)."""
@@ -2037,7 +2036,7 @@ def _gh2_frag(weight: Tensor, config: int, channels: int) -> Tensor:
     return _ew_frag(weight.detach().index_select(0, rows), True)
 
 
-@torch.library.custom_op("molix::tp_weight_grad_batched", mutates_args=(), device_types="cuda")
+@_op("molix::tp_weight_grad_batched")
 def tp_weight_grad_batched(x: Tensor, Y: Tensor, grad_out: Tensor, row_ptr: Tensor, perm: Tensor, senders: Tensor,
                            batches: Tensor, weight: Tensor, config: int, channels: int) -> Tensor:
     """``grad_h = gw @ weight`` per directed edge (as ``tp_weight_grad``) over the receiver CSR, one
@@ -2153,7 +2152,7 @@ def tp_backward_gh_supported(config: int, channels: int, K: int) -> bool:
     return config >= 0 and bool(_lib.load().mnx_tp_bwd_gh_supported(config, channels, K))
 
 
-@torch.library.custom_op("molix::tp_scatter_backward_gh", mutates_args=(), device_types="cuda")
+@_op("molix::tp_scatter_backward_gh")
 def tp_scatter_backward_gh(grad_out: Tensor, x: Tensor, Y: Tensor, w: Tensor, row_ptr: Tensor, perm: Tensor,
                            senders: Tensor, wrow: Tensor | None, weight: Tensor, config: int, channels: int,
                            need_x: bool, need_Y: bool) -> tuple[Tensor, Tensor, Tensor]:
@@ -2193,7 +2192,7 @@ def _(grad_out, x, Y, w, row_ptr, perm, senders, wrow, weight, config, channels,
             x.new_empty(Y.shape[0], weight.shape[1]))
 
 
-@torch.library.custom_op("molix::radial_tp_pairs", mutates_args=(), device_types="cuda")
+@_op("molix::radial_tp_pairs")
 def radial_tp_pairs(x: Tensor, Y: Tensor, h: Tensor, weight: Tensor, bias: Tensor | None, row_ptr: Tensor,
                     perm: Tensor, senders: Tensor, wrow: Tensor, pairs: Tensor, config: int,
                     channels: int, batches: Tensor | None = None) -> tuple[Tensor, Tensor]:
@@ -2344,7 +2343,7 @@ def _parse_blocks(blocks: list[int]):
         yield off, mul, d, woff, [tuple(segs[3 * s:3 * s + 3]) for s in range(n)]
 
 
-@torch.library.custom_op("molix::block_linear", mutates_args=(), device_types="cuda")
+@_op("molix::block_linear")
 def block_linear(a: Tensor, weights: Tensor, blocks: list[int], out_dim: int) -> Tensor:
     """One ``mnx_block_linear_f32`` launch per output block of an ir_mul linear
     (``src/molrep/interaction/linear.py:43-105``): ``blocks`` as built by ``block_linear_desc``,
@@ -2385,7 +2384,7 @@ def _(a, weights, blocks, out_dim):
     return a.new_empty(a.shape[0], out_dim)
 
 
-@torch.library.custom_op("molix::block_linear_weights", mutates_args=(), device_types="cuda")
+@_op("molix::block_linear_weights")
 def block_linear_weights(a: Tensor, weight: Tensor, blocks: list[int], scales: list[float], out_dim: int,
                          transposed: bool, order: Tensor | None = None, class_start: Tensor | None = None) -> Tensor:
     """Every output block of an ir_mul linear in one launch, with the weights in the module's own
@@ -2435,7 +2434,7 @@ def _(a, weight, blocks, scales, out_dim, transposed, order=None, class_start=No
     return a.new_empty(a.shape[0], out_dim)
 
 
-@torch.library.custom_op("molix::block_linear_weight_grad", mutates_args=(), device_types="cuda")
+@_op("molix::block_linear_weight_grad")
 def block_linear_weight_grad(x: Tensor, g: Tensor, pairs: list[int], scales: list[float], numel: int) -> Tensor:
     """The weight gradient of an ir_mul linear (``src/molrep/interaction/linear.py:43-105``), flat
     ``(numel,)``: 8 integers per pair of an input and an output block (column, component step and
@@ -2464,7 +2463,7 @@ def _(x, g, pairs, scales, numel):
     return x.new_empty(numel)
 
 
-@torch.library.custom_op("molix::class_groups", mutates_args=(), device_types="cuda")
+@_op("molix::class_groups")
 def _class_groups_op(classes: Tensor, num_classes: int) -> tuple[Tensor, Tensor]:
     lib = _lib.load()
     c = classes.reshape(-1).to(torch.int64).contiguous()
@@ -2493,7 +2492,7 @@ def class_groups(classes: Tensor, num_classes: int) -> tuple[Tensor, Tensor]:
     return _class_groups_op(classes, int(num_classes))
 
 
-@torch.library.custom_op("molix::indexed_block_linear", mutates_args=(), device_types="cuda")
+@_op("molix::indexed_block_linear")
 def indexed_block_linear(a: Tensor, weights: Tensor, order: Tensor, class_start: Tensor, blocks: list[int],
                          out_dim: int) -> Tensor:
     """``block_linear`` with one weight set per node class (``cuet.Linear(weight_classes=S,
@@ -2547,7 +2546,7 @@ def _(a, weights, order, class_start, blocks, out_dim):
 # Bond vectors
 # ---------------------------------------------------------------------------
 
-@torch.library.custom_op("molix::bond_vectors", mutates_args=(), device_types="cuda")
+@_op("molix::bond_vectors")
 def bond_vectors(positions: Tensor, edge_index: Tensor, shifts: Tensor | None = None) -> Tensor:
     """``positions[edge_index[:, 1]] - positions[edge_index[:, 0]] - shifts`` for an (E, 2) edge list of
     [sender, receiver] rows: the reference's ``bond_diff = pos[target] - pos[source]``
@@ -2574,7 +2573,7 @@ def _(positions, edge_index, shifts=None):
     return positions.new_empty(edge_index.shape[0], 3)
 
 
-@torch.library.custom_op("molix::bond_vectors_backward", mutates_args=(), device_types="cuda")
+@_op("molix::bond_vectors_backward")
 def bond_vectors_backward(grad: Tensor, edge_index: Tensor, num_atoms: int) -> Tensor:
     ei = edge_index.to(torch.int64).contiguous()
     g = grad.to(torch.float32).contiguous()
@@ -2616,7 +2615,7 @@ def _cs_rows(t: Tensor, width: int, what: str) -> Tensor:
     return _aligned16(t)
 
 
-@torch.library.custom_op("molix::channel_scale", mutates_args=(), device_types="cuda")
+@_op("molix::channel_scale")
 def channel_scale(t: Tensor, s: Tensor, components: int) -> Tensor:
     """``out[e][d][c] = t[e][d][c] * s[e][c]`` for an (E, D*F) ir_mul tensor and (E, F) scales: the
     reference's ``_scale_by_channel`` (src/molzoo/allegro.py:95-128); one HIP pass each way (the
@@ -2638,7 +2637,7 @@ def _(t, s, components):
     return t.new_empty(t.shape)
 
 
-@torch.library.custom_op("molix::channel_scale_backward", mutates_args=(), device_types="cuda")
+@_op("molix::channel_scale_backward")
 def channel_scale_backward(grad: Tensor, t: Tensor, s: Tensor, components: int, need_t: bool,
                            need_s: bool) -> tuple[Tensor, Tensor]:
     """(grad * s, sum_d grad * t) of ``channel_scale`` in one pass; an empty tensor for a gradient
@@ -2715,7 +2714,7 @@ channel_scale_backward.register_autograd(_cs2_bwd, setup_context=_cs2_setup)
 CHANNEL_PRODUCT_COMPONENTS = (1, 4, 9, 16)
 
 
-@torch.library.custom_op("molix::channel_outer", mutates_args=(), device_types="cuda")
+@_op("molix::channel_outer")
 def channel_outer(y: Tensor, s: Tensor) -> Tensor:
     """``out[e][d][c] = y[e][d] * s[e][c]`` as an (E, D*F) ir_mul tensor: the env-weighted harmonics
     of Allegro's pair embedding (src/molzoo/allegro.py:55-92); the backward forms both gradients in
@@ -2739,7 +2738,7 @@ def _(y, s):
     return y.new_empty(y.shape[0], y.shape[1] * s.shape[1])
 
 
-@torch.library.custom_op("molix::channel_outer_backward", mutates_args=(), device_types="cuda")
+@_op("molix::channel_outer_backward")
 def channel_outer_backward(grad: Tensor, y: Tensor, s: Tensor, need_y: bool, need_s: bool) -> tuple[Tensor, Tensor]:
     """(sum_c grad * s, sum_d grad * y) of ``channel_outer`` in one pass; an empty tensor for a
     gradient not requested."""
@@ -2825,7 +2824,7 @@ def _ptr_array(ts) -> C.c_void_p:
     return C.cast((C.c_void_p * len(ts))(*[t.data_ptr() for t in ts]), C.c_void_p)
 
 
-@torch.library.custom_op("molix::channel_outer_stack", mutates_args=(), device_types="cuda")
+@_op("molix::channel_outer_stack")
 def channel_outer_stack(y: Tensor, s: list[Tensor]) -> Tensor:
     """``stack([y * s_l for s_l in s], 1)`` for a per-edge factor ``y`` (E rows of one entry) and
     L (E, F) inputs, (E, L, F) in one pass: the cutoff envelope on Allegro's per-layer scalar
@@ -2844,7 +2843,7 @@ def _(y, s):
     return y.new_empty(s[0].shape[0], len(s), s[0].shape[1])
 
 
-@torch.library.custom_op("molix::channel_outer_stack_backward", mutates_args=(), device_types="cuda")
+@_op("molix::channel_outer_stack_backward")
 def channel_outer_stack_backward(grad: Tensor, y: Tensor, s: list[Tensor], need_y: bool,
                                  need_s: bool) -> list[Tensor]:
     """``[grad y, grad s_0, ..., grad s_{L-1}]`` of ``channel_outer_stack`` in one pass: grad y
@@ -2887,7 +2886,7 @@ def _basis_args(r, mu, sigma, num_radial):
     return rr, m, s
 
 
-@torch.library.custom_op("molix::bessel_cutoff", mutates_args=(), device_types="cuda")
+@_op("molix::bessel_cutoff")
 def bessel_cutoff(r: Tensor, num_radial: int, r_cut: float, eps: float, mu: Tensor | None, sigma: Tensor | None,
                   cutoff: int, exponent: int) -> Tensor:
     """``BesselRBF(r) * cutoff(r)[..., None]`` in one kernel (``radial.py:36-148``, ``cutoff.py:23-161``,
@@ -2906,7 +2905,7 @@ def _(r, num_radial, r_cut, eps, mu, sigma, cutoff, exponent):
     return r.new_empty(*r.shape, num_radial, dtype=torch.float32)
 
 
-@torch.library.custom_op("molix::bessel_cutoff_backward", mutates_args=(), device_types="cuda")
+@_op("molix::bessel_cutoff_backward")
 def bessel_cutoff_backward(grad: Tensor, r: Tensor, num_radial: int, r_cut: float, eps: float, mu: Tensor | None,
                            sigma: Tensor | None, cutoff: int, exponent: int) -> Tensor:
     rr, m, sg = _basis_args(r, mu, sigma, num_radial)
@@ -2955,7 +2954,7 @@ def _segment_csr(index: Tensor, num_segments: int, validate: bool) -> tuple[Tens
     return row_ptr, perm
 
 
-@torch.library.custom_op("molix::segment_sum", mutates_args=(), device_types="cuda")
+@_op("molix::segment_sum")
 def segment_sum(values: Tensor, index: Tensor, num_segments: int, weights: Tensor | None = None,
                 validate: bool = True) -> Tensor:
     """``out[n] = sum_{r: index[r] = n} weights[r] * values[r]`` for ``values`` (R, D), ``index`` (R,)
@@ -2983,7 +2982,7 @@ def _(values, index, num_segments, weights=None, validate=True):
     return values.new_empty(num_segments, values.shape[1])
 
 
-@torch.library.custom_op("molix::segment_sum_backward", mutates_args=(), device_types="cuda")
+@_op("molix::segment_sum_backward")
 def segment_sum_backward(grad: Tensor, index: Tensor, values: Tensor, weights: Tensor | None, need_values: bool,
                          need_weights: bool) -> tuple[Tensor, Tensor]:
     g = _f32_rows(grad, grad.shape[-1], "grad")
