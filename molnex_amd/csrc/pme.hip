@@ -341,9 +341,9 @@ constexpr int kConvThreads = 256;
 // per-block energy partial sums (pme_cpu.cpp:263-294).
 template <typename T>
 __global__ void __launch_bounds__(kConvThreads) k_convolve(T* __restrict__ cgrid, const T* __restrict__ box, int gx,
-                                                           int gy, int gz, T alpha, const T* __restrict__ xm,
-                                                           const T* __restrict__ ym, const T* __restrict__ zm,
-                                                           double* __restrict__ partials) {
+                                                           int gy, int gz, T alpha, const void* __restrict__ xm,
+                                                           const void* __restrict__ ym, const void* __restrict__ zm,
+                                                           bool mods64, double* __restrict__ partials) {
     __shared__ double red[kConvThreads];
     const int zs = gz / 2 + 1;
     const int64_t total = int64_t(gx) * gy * zs;
@@ -365,7 +365,11 @@ __global__ void __launch_bounds__(kConvThreads) k_convolve(T* __restrict__ cgrid
         const T mhz = mx * R.r[2][0] + my * R.r[2][1] + mz * R.r[2][2];
         const T m2 = mhx * mhx + mhy * mhy + mhz * mhz;
         const T scale_f = T(M_PI) * box[0] * box[4] * box[8];
-        const T denom = m2 * (scale_f * xm[kx] * ym[ky]) * zm[kz];
+        // the moduli in T or (mods64) in double, rounded to T
+        auto mod = [&](const void* m, int k) {
+            return mods64 ? T(static_cast<const double*>(m)[k]) : static_cast<const T*>(m)[k];
+        };
+        const T denom = m2 * (scale_f * mod(xm, kx) * mod(ym, ky)) * mod(zm, kz);
         const T rexp = T(M_PI * M_PI) / (alpha * alpha);
         const T eterm = idx == 0 ? T(0) : exp(-rexp * m2) / denom;
         const T s = (kz > 0 && kz <= (gz - 1) / 2) ? T(2) : T(1);
@@ -696,8 +700,8 @@ int spread(const T* pos, const T* q, const T* box, int64_t n, int gx, int gy, in
 int64_t conv_blocks(int gx, int gy, int gz) { return ceil_div(int64_t(gx) * gy * (gz / 2 + 1), kConvThreads); }
 
 template <typename T>
-int convolve(T* cgrid, const T* box, int gx, int gy, int gz, double alpha, const T* xm, const T* ym, const T* zm,
-             const double* more, int64_t nmore, T* energy, void* ws, size_t ws_bytes, hipStream_t s) {
+int convolve(T* cgrid, const T* box, int gx, int gy, int gz, double alpha, const void* xm, const void* ym, const void* zm,
+             bool mods64, const double* more, int64_t nmore, T* energy, void* ws, size_t ws_bytes, hipStream_t s) {
     clear_error();
     int rc = check_grid(gx, gy, gz, 3);
     MNX_REQUIRE(rc || nmore == 0 || more, "null pointer argument");
@@ -708,7 +712,7 @@ int convolve(T* cgrid, const T* box, int gx, int gy, int gz, double alpha, const
         return set_error(MNX_ERR_WORKSPACE, "workspace %zu < %zu bytes", ws_bytes, size_t(nb) * sizeof(double));
     double* part = static_cast<double*>(ws);
     hipLaunchKernelGGL((k_convolve<T>), dim3(nb), dim3(kConvThreads), 0, s, cgrid, box, gx, gy, gz, T(alpha), xm, ym,
-                       zm, part);
+                       zm, mods64, part);
     MNX_CHECK_LAUNCH();
     hipLaunchKernelGGL((k_sum_partials<T>), dim3(1), dim3(1024), 0, s, part, nb, 0.5, more, nmore, energy);
     MNX_CHECK_LAUNCH();
@@ -808,12 +812,12 @@ size_t mnx_pme_convolve_workspace_bytes(int32_t gx, int32_t gy, int32_t gz) {
 int mnx_pme_convolve_f32(float* cgrid, const float* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
                          const float* xm, const float* ym, const float* zm, float* energy, void* ws, size_t ws_bytes,
                          mnx_stream_t s) {
-    return convolve<float>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, nullptr, 0, energy, ws, ws_bytes, (hipStream_t)s);
+    return convolve<float>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, false, nullptr, 0, energy, ws, ws_bytes, (hipStream_t)s);
 }
 int mnx_pme_convolve_f64(double* cgrid, const double* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
                          const double* xm, const double* ym, const double* zm, double* energy, void* ws,
                          size_t ws_bytes, mnx_stream_t s) {
-    return convolve<double>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, nullptr, 0, energy, ws, ws_bytes, (hipStream_t)s);
+    return convolve<double>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, false, nullptr, 0, energy, ws, ws_bytes, (hipStream_t)s);
 }
 int mnx_pme_gather_f32(const float* pos, const float* q, const float* box, int64_t n, const float* grid, int32_t gx,
                        int32_t gy, int32_t gz, int32_t order, double coulomb, float* dpos, float* dq, mnx_stream_t s) {
@@ -841,9 +845,9 @@ int mnx_pme_direct_f64(const double* pos, const double* q, int64_t n, const int3
 }
 
 int mnx_pme_convolve_add_f32(float* cgrid, const float* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
-                             const float* xm, const float* ym, const float* zm, const double* more, int64_t nmore,
-                             float* energy, void* ws, size_t ws_bytes, mnx_stream_t s) {
-    return convolve<float>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, more, nmore, energy, ws, ws_bytes, (hipStream_t)s);
+                             const void* xm, const void* ym, const void* zm, int32_t mods64, const double* more,
+                             int64_t nmore, float* energy, void* ws, size_t ws_bytes, mnx_stream_t s) {
+    return convolve<float>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, mods64 != 0, more, nmore, energy, ws, ws_bytes, (hipStream_t)s);
 }
 int mnx_pme_gather_add_f32(const float* pos, const float* q, const float* box, int64_t n, const float* grid, int32_t gx,
                            int32_t gy, int32_t gz, int32_t order, double coulomb, const float* grad, const float* dpos_add,
@@ -851,9 +855,9 @@ int mnx_pme_gather_add_f32(const float* pos, const float* q, const float* box, i
     return gather<float>(pos, q, box, n, grid, gx, gy, gz, order, coulomb, grad, dpos_add, dq_add, dpos, dq, (hipStream_t)s);
 }
 int mnx_pme_convolve_add_f64(double* cgrid, const double* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
-                             const double* xm, const double* ym, const double* zm, const double* more, int64_t nmore,
-                             double* energy, void* ws, size_t ws_bytes, mnx_stream_t s) {
-    return convolve<double>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, more, nmore, energy, ws, ws_bytes, (hipStream_t)s);
+                             const void* xm, const void* ym, const void* zm, int32_t mods64, const double* more,
+                             int64_t nmore, double* energy, void* ws, size_t ws_bytes, mnx_stream_t s) {
+    return convolve<double>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, mods64 != 0, more, nmore, energy, ws, ws_bytes, (hipStream_t)s);
 }
 int mnx_pme_gather_add_f64(const double* pos, const double* q, const double* box, int64_t n, const double* grid, int32_t gx,
                            int32_t gy, int32_t gz, int32_t order, double coulomb, const double* grad, const double* dpos_add,

@@ -1035,7 +1035,9 @@ def pme_energy(positions: Tensor, charges: Tensor, box_vectors: Tensor, xmoduli:
     b = box_vectors.detach().to(device=dev, dtype=dt).contiguous()
     if tuple(b.shape) != (3, 3) or tuple(pos.shape) != (n, 3) or tuple(q.shape) != (n,):
         raise ValueError("pme_energy: positions must be (n, 3), charges (n,) and box_vectors (3, 3)")
-    mods = [m.detach().to(device=dev, dtype=dt).contiguous() for m in (xmoduli, ymoduli, zmoduli)]
+    # moduli in float64 (as the module keeps them) are used as they are, rounded by the kernel
+    mdt = torch.float64 if xmoduli.dtype == ymoduli.dtype == zmoduli.dtype == torch.float64 else dt
+    mods = [m.detach().to(device=dev, dtype=mdt).contiguous() for m in (xmoduli, ymoduli, zmoduli)]
     if any(m.numel() < g for m, g in zip(mods, (gridx, gridy, gridz))):
         raise ValueError("moduli shorter than the grid")
     stream = _stream(pos)
@@ -1063,7 +1065,7 @@ def pme_energy(positions: Tensor, charges: Tensor, box_vectors: Tensor, xmoduli:
     energy = torch.empty((), dtype=dt, device=dev)
     check(getattr(lib, f"mnx_pme_convolve_add_{sfx}")(
         ptr(torch.view_as_real(spec)), ptr(b), gridx, gridy, gridz, float(alpha), ptr(mods[0]), ptr(mods[1]),
-        ptr(mods[2]), parts, nparts, ptr(energy), scratch, size, stream), "pme convolve")
+        ptr(mods[2]), int(mdt == torch.float64), parts, nparts, ptr(energy), scratch, size, stream), "pme convolve")
     if many is not None:
         arrived.synchronize()
         if int(many.view(torch.int32)[0]):

@@ -51,17 +51,8 @@ class PMEPotential(nn.Module):
         super().__init__()
         self.alpha, self.grid, self.order, self.cutoff, self.coulomb = alpha, tuple(grid), order, cutoff, coulomb
         for name, g in zip(("xmoduli", "ymoduli", "zmoduli"), self.grid):
-            mod = torch.tensor(bspline_moduli(g, order), dtype=torch.float64)
-            self.register_buffer(name, mod, persistent=False)
-            self.register_buffer(name + "_f32", mod.float(), persistent=False)
-
-    def _moduli(self, dt: torch.dtype):
-        """The three axes' moduli in ``dt``, from the buffers where one has it."""
-        out = []
-        for name in ("xmoduli", "ymoduli", "zmoduli"):
-            full, half = getattr(self, name), getattr(self, name + "_f32")
-            out.append(full.to(dt) if full.dtype == dt or half.dtype != dt else half)
-        return out
+            self.register_buffer(name, torch.tensor(bspline_moduli(g, order), dtype=torch.float64),
+                                 persistent=False)
 
     def forward(self, positions: torch.Tensor, charges: torch.Tensor, box: torch.Tensor,
                 exclusions: torch.Tensor | None = None, pairs=None) -> torch.Tensor:
@@ -71,7 +62,7 @@ class PMEPotential(nn.Module):
                 and dt in (torch.float32, torch.float64) and charges.dtype == dt):
             # all three terms as one op each way, the real-space pairs never listed
             want = torch.is_grad_enabled() and (positions.requires_grad or charges.requires_grad)
-            return ops.pme_energy(positions, charges, box, *self._moduli(dt), *self.grid, self.order, self.alpha,
+            return ops.pme_energy(positions, charges, box, self.xmoduli, self.ymoduli, self.zmoduli, *self.grid, self.order, self.alpha,
                                   self.cutoff, self.coulomb, want)[0]
         if pairs is None:
             i, j, _, d, r = ops.neighbor_list(positions.detach(), self.cutoff, box.detach(), False)
@@ -81,7 +72,7 @@ class PMEPotential(nn.Module):
         if exclusions is None:
             exclusions = torch.full((positions.shape[0], 1), -1, dtype=torch.int32, device=positions.device)
         e_dir = ops.pme_direct(positions, charges, nb, d, r, exclusions, self.alpha, self.coulomb)
-        mods = self._moduli(dt)
+        mods = [m.to(dt) for m in (self.xmoduli, self.ymoduli, self.zmoduli)]
         # the spectrum variant of molix::pme_reciprocal keeps the convolved spectrum for the
         # backward, which then skips the second spread and forward transform
         e_rec, _ = ops.pme_reciprocal_spectrum(positions, charges, box.to(dt), *self.grid, self.order, self.alpha,

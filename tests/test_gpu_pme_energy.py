@@ -98,7 +98,7 @@ def test_single_gradients_scaling_and_no_grad():
     (only,) = torch.autograd.grad(pme(pos, c, box), c)
     torch.testing.assert_close(only, gq, rtol=1e-6, atol=1e-6)
     # the forward told that no gradient is wanted: the backward forms the real-space part itself
-    spec = torch.ops.molix.pme_energy(pos, q, box, *pme._moduli(torch.float32), 20, 20, 20, 5, 0.35, 4.5, pme.coulomb, False)
+    spec = torch.ops.molix.pme_energy(pos, q, box, pme.xmoduli, pme.ymoduli, pme.zmoduli, 20, 20, 20, 5, 0.35, 4.5, pme.coulomb, False)
     got = torch.ops.molix.pme_energy_backward(torch.ones((), device=DEV), pos, q, box, *spec[1:], 20, 20, 20, 5, 0.35, 4.5,
                                               pme.coulomb)
     assert torch.equal(got[0], gp) and torch.equal(got[1], gq)
@@ -116,4 +116,4 @@ def test_opcheck():
     pme = PMEPotential(alpha=0.4, grid=(16, 16, 16), order=4, cutoff=3.5).to(DEV)
     pos.requires_grad_(True), q.requires_grad_(True)
     torch.library.opcheck(torch.ops.molix.pme_energy.default,
-                          (pos, q, box, *pme._moduli(torch.float64), 16, 16, 16, 4, 0.4, 3.5, 1.0, True))
+                          (pos, q, box, pme.xmoduli, pme.ymoduli, pme.zmoduli, 16, 16, 16, 4, 0.4, 3.5, 1.0, True))
