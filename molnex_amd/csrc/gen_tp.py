@@ -209,16 +209,11 @@ def gen_fwd(cfg: Cfg, g: int) -> str:
     L = []
     a = L.append
     name = f"tp_fwd_c{cfg.idx}_g{g}"
-    a(f"template <int CPL, bool FULL>\n__global__ void __launch_bounds__(64) {name}(const float* __restrict__ x, "
-      "const float* __restrict__ Y, const float* __restrict__ w, const int32_t* __restrict__ row_ptr, "
-      "const int32_t* __restrict__ perm, const int32_t* __restrict__ snd, const int32_t* __restrict__ wrow, "
-      "int64_t N, int C, float* __restrict__ out) {")
-    a("  const int64_t n = xcd_node(blockIdx.x, gridDim.x);")
+    a(f"template <int CPL, bool FULL, int LW>\n__device__ __forceinline__ void {name}_body({FWD_PARAMS}, {BODY_PARAMS}) {{")
     a("  if (n >= N) return;")
-    a("  const int lane = threadIdx.x;")
     a("  int cc[CPL]; bool ok[CPL];")
     a("#pragma unroll")
-    a("  for (int k = 0; k < CPL; ++k) { cc[k] = blockIdx.y * (64 * CPL) + 64 * k + lane; ok[k] = FULL || cc[k] < C; }")
+    a("  for (int k = 0; k < CPL; ++k) { cc[k] = cblock * (LW * CPL) + LW * k + lane; ok[k] = FULL || cc[k] < C; }")
     a(f"  float acc[CPL][{len(outs)}];")
     a("#pragma unroll")
     a(f"  for (int k = 0; k < CPL; ++k)\n#pragma unroll\n    for (int i = 0; i < {len(outs)}; ++i) acc[k][i] = 0.f;")
@@ -262,6 +257,45 @@ def gen_fwd(cfg: Cfg, g: int) -> str:
         a(f"    on[{c} * C + cc[k]] = acc[k][{oi[c]}];")
     a("  }")
     a("}")
+    a(f"template <int CPL, bool FULL>\n__global__ void __launch_bounds__(64) {name}({FWD_PARAMS}) {{")
+    a(f"  {name}_body<CPL, FULL, 64>({FWD_ARGS}, xcd_node(blockIdx.x, gridDim.x), threadIdx.x, blockIdx.y);")
+    a("}")
+    return "\n".join(L)
+
+
+# Parameters of the receiver-walked kernels and of their bodies.  A body works for LW lanes of a wavefront
+# on one receiver: 64, or 32 / 16 with two / four receivers per wavefront for as many channels.
+FWD_PARAMS = ("const float* __restrict__ x, const float* __restrict__ Y, const float* __restrict__ w, "
+              "const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ perm, "
+              "const int32_t* __restrict__ snd, const int32_t* __restrict__ wrow, int64_t N, int C, "
+              "float* __restrict__ out")
+FWD_ARGS = "x, Y, w, row_ptr, perm, snd, wrow, N, C, out"
+BWD_PARAMS = ("const float* __restrict__ x, const float* __restrict__ Y, const float* __restrict__ w, "
+              "const float* __restrict__ gout, const int32_t* __restrict__ row_ptr, "
+              "const int32_t* __restrict__ perm, const int32_t* __restrict__ snd, "
+              "const int32_t* __restrict__ wrow, int64_t N, int C, float* __restrict__ gx, "
+              "float* __restrict__ gw, float* __restrict__ gyp, int npart, int pbase")
+BWD_ARGS = "x, Y, w, gout, row_ptr, perm, snd, wrow, N, C, gx, gw, gyp, npart"
+BODY_PARAMS = "const int64_t n, const int lane, const int cblock"
+
+
+def gen_all(cfg: Cfg) -> str:
+    """Every path group of a configuration in one launch (blockIdx.z), one channel per lane."""
+    L = []
+    a = L.append
+    for d, params in (("fwd", FWD_PARAMS), ("bwd", BWD_PARAMS)):
+        a(f"template <int LW>\n__global__ void __launch_bounds__(64) tp_{d}_c{cfg.idx}_all({params}) {{")
+        a("  const int64_t b = xcd_node(blockIdx.x, gridDim.x);")
+        a("  const int64_t n = LW == 64 ? b : b * (64 / LW) + threadIdx.x / LW;")
+        a("  const int lane = threadIdx.x % LW;")
+        a("  switch (blockIdx.z) {")
+        for g in range(len(cfg.groups)):
+            args = FWD_ARGS if d == "fwd" else f"{BWD_ARGS}, pbase + {g} * int(gridDim.y)"
+            last = g == len(cfg.groups) - 1
+            a(f"    {'default' if last else f'case {g}'}: tp_{d}_c{cfg.idx}_g{g}_body<1, false, LW>({args}, n, lane, "
+              "blockIdx.y); break;")
+        a("  }")
+        a("}")
     return "\n".join(L)
 
 
@@ -276,19 +310,12 @@ def gen_bwd(cfg: Cfg, g: int) -> str:
     L = []
     a = L.append
     name = f"tp_bwd_c{cfg.idx}_g{g}"
-    a(f"template <int CPL, bool FULL>\n__global__ void __launch_bounds__(64) {name}(const float* __restrict__ x, "
-      "const float* __restrict__ Y, const float* __restrict__ w, const float* __restrict__ gout, "
-      "const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ perm, const int32_t* __restrict__ snd, "
-      "const int32_t* __restrict__ wrow, "
-      "int64_t N, int C, float* __restrict__ gx, float* __restrict__ gw, float* __restrict__ gyp, int npart, "
-      "int pbase) {")
-    a("  const int64_t n = xcd_node(blockIdx.x, gridDim.x);")
+    a(f"template <int CPL, bool FULL, int LW>\n__device__ __forceinline__ void {name}_body({BWD_PARAMS}, {BODY_PARAMS}) {{")
     a("  if (n >= N) return;")
-    a("  const int lane = threadIdx.x;")
     a("  int cc[CPL]; bool ok[CPL];")
     a("#pragma unroll")
-    a("  for (int k = 0; k < CPL; ++k) { cc[k] = blockIdx.y * (64 * CPL) + 64 * k + lane; ok[k] = FULL || cc[k] < C; }")
-    a("  const int pidx = pbase + blockIdx.y;")
+    a("  for (int k = 0; k < CPL; ++k) { cc[k] = cblock * (LW * CPL) + LW * k + lane; ok[k] = FULL || cc[k] < C; }")
+    a("  const int pidx = pbase + cblock;")
     a(f"  const int64_t XS = int64_t({cfg.NX}) * C, WS = int64_t({cfg.NP}) * C;")
     a(f"  const float* __restrict__ gn = gout + n * int64_t({cfg.NO}) * C;")
     vnames = {}
@@ -334,11 +361,12 @@ def gen_bwd(cfg: Cfg, g: int) -> str:
         f(f"          atomicAdd(gxs + {c} * C + cc[k], dgx[k][{xi[c]}]);")
     f("        }")
     f("      }")
-    f(f"      if (gyp && (lane & (64 / {V} - 1)) == 0 && dcomp < {cfg.NY}) "
+    f(f"      if (gyp && (lane & (LW / {V} - 1)) == 0 && dcomp < {cfg.NY}) "
       f"gyp[(int64_t(de) * npart + pidx) * {cfg.NY} + dcomp] = dgy;")
     f("    }")
     a(f"  float dgw[CPL][{len(ps)}], dgx[CPL][{len(xs)}], dgy = 0.f;")
-    a(f"  const int dcomp = reduce_scatter_index<{V}>(lane);")
+    a(f"  static_assert({V} <= LW, \"one lane per component\");")
+    a(f"  const int dcomp = reduce_scatter_index<{V}, LW>(lane);")
     a("  int de = 0, ds = 0;")
     a("  bool pend = false;")
     _emit_edge_loop_head(a, cfg, ps, xs, ys, xi, flush)
@@ -382,11 +410,14 @@ def gen_bwd(cfg: Cfg, g: int) -> str:
     for c in xs:
         a(f"      dgx[k][{xi[c]}] = gxl[{xi[c]}];")
     a("    }")
-    a(f"    if (gyp) dgy = wave_reduce_scatter<{V}>(gy, lane);")
+    a(f"    if (gyp) dgy = wave_reduce_scatter<{V}, LW>(gy, lane);")
     a("    de = e; ds = s; pend = true;")
     a("  }")
     for line in flush:
         a(line[2:] if line.startswith("  ") else line)
+    a("}")
+    a(f"template <int CPL, bool FULL>\n__global__ void __launch_bounds__(64) {name}({BWD_PARAMS}) {{")
+    a(f"  {name}_body<CPL, FULL, 64>({BWD_ARGS}, pbase, xcd_node(blockIdx.x, gridDim.x), threadIdx.x, blockIdx.y);")
     a("}")
     return "\n".join(L)
 
@@ -901,6 +932,8 @@ def generate() -> str:
             out.append("")
             out.append(gen_bwd(cfg, g))
             out.append("")
+        out.append(gen_all(cfg))
+        out.append("")
         for sg, (ps, first) in enumerate(sender_subgroups(cfg)):
             out.append(gen_bwd_sender(cfg, sg, ps, first))
             out.append("")
@@ -927,6 +960,19 @@ def generate() -> str:
             fns = [f"tp_bwd_c{cfg.idx}_g{g}<{bwd_cpl(ps)}, {fl}>" for g, ps in enumerate(cfg.groups)]
             fns += ["nullptr"] * (4 - len(fns))
             out.append("  {" + ", ".join(fns) + "},")
+        out.append("};")
+        # ... and with one channel per lane, for at most 64 channels
+        out.append(f"static const TPBwdFn kTPBwd{tag}1[][4] = {{")
+        for cfg in cfgs:
+            fns = [f"tp_bwd_c{cfg.idx}_g{g}<1, {fl}>" for g in range(len(cfg.groups))]
+            fns += ["nullptr"] * (4 - len(fns))
+            out.append("  {" + ", ".join(fns) + "},")
+        out.append("};")
+    # all groups in one launch: 16, 32 or 64 lanes per receiver
+    for d, typ in (("fwd", "TPFwdFn"), ("bwd", "TPBwdFn")):
+        out.append(f"static const {typ} kTP{d.capitalize()}All[][3] = {{")
+        for cfg in cfgs:
+            out.append("  {" + ", ".join(f"tp_{d}_c{cfg.idx}_all<{lw}>" for lw in (16, 32, 64)) + "},")
         out.append("};")
     out.append("static const int kTPBwdCPL[][4] = {")
     for cfg in cfgs:

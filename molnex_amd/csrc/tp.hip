@@ -72,6 +72,34 @@ int64_t bwd_partials(int config, int C) {
     return np;
 }
 
+// Lanes per receiver of the launch that takes all path groups at once, or 0 for one launch per group.
+//
+// With at most 32 (16) channels, two (four) receivers share a wavefront: with one, half (three
+// quarters) of its lanes carry no channel.  Periodic boxes, l <= 2, forward + backward: 16 channels,
+// 20k receivers 1751 -> 1175 us, 8k 794 -> 488, 2k 383 -> 219; 32 channels, 8k 890 -> 693 us (all
+// groups in one launch but one receiver per wavefront: 1486, 630, 216; 755).  Molecules of degree 8,
+// 2048 receivers, 16 channels: forward kernels 43 -> 19 us, backward 66 -> 30.
+//
+// With more channels, graphs of at most kTPSmallWaves wavefronts per group (3.4 per SIMD) are bound by
+// the latency of each wavefront's edge walk, one group after the other, so their groups go together:
+// 64 channels, 0e+1o, 2k receivers 292 -> 235 us, 3k 369 -> 319; 128 channels, l <= 3, 1k receivers
+// 757 -> 639.  From 4k wavefronts on the two are even, and the forward alone loses (64 channels, 6k
+// receivers: 166 us by group, 175 together).
+constexpr int64_t kTPSmallWaves = 3500;
+
+int all_lanes(int64_t N, int C) {
+    if (C <= 32) return C <= 16 ? 16 : 32;
+    return N * ceil_div(C, 64) <= kTPSmallWaves ? 64 : 0;
+}
+
+int lanes_index(int lw) { return lw == 16 ? 0 : (lw == 32 ? 1 : 2); }
+
+dim3 all_grid(int64_t N, int C, int lw, int groups) {
+    dim3 g = node_grid(ceil_div(N, 64 / lw), int(ceil_div(C, lw)));
+    g.z = unsigned(groups);
+    return g;
+}
+
 }  // namespace
 }  // namespace mnx
 
@@ -112,6 +140,12 @@ int mnx_tp_fwd_rows_f32(int32_t config, int32_t C, const float* x, const float* 
     if (N == 0) return MNX_OK;
     MNX_REQUIRE(out && row_ptr && (E == 0 || (x && Y && w && perm && snd)), "null pointer argument");
     const TPConfigInfo& cfg = kTPConfigs[config];
+    if (const int lw = all_lanes(N, C)) {
+        hipLaunchKernelGGL(kTPFwdAll[config][lanes_index(lw)], all_grid(N, C, lw, cfg.ngroups), dim3(64), 0,
+                           (hipStream_t)stream, x, Y, w, row_ptr, perm, snd, wrow, N, C, out);
+        MNX_CHECK_LAUNCH();
+        return MNX_OK;
+    }
     const int cpl = C > 64 ? 2 : 1;
     const int cblocks = int(ceil_div(C, 64 * cpl));
     const dim3 grid = node_grid(N, cblocks);
@@ -127,7 +161,9 @@ int mnx_tp_fwd_rows_f32(int32_t config, int32_t C, const float* x, const float* 
 size_t mnx_tp_bwd_workspace_bytes(int32_t config, int32_t C, int64_t E) {
     if (config < 0 || config >= kNumTPConfigs || C <= 0 || E < 0) return 0;
     const TPConfigInfo& cfg = kTPConfigs[config];
-    return size_t(E > 0 ? E : 1) * size_t(bwd_partials(config, C)) * size_t(cfg.ny) * sizeof(float) + 256;
+    // the launch of all groups takes one channel per lane
+    const int64_t np = std::max<int64_t>(bwd_partials(config, C), cfg.ngroups * ceil_div(C, 64));
+    return size_t(E > 0 ? E : 1) * size_t(np) * size_t(cfg.ny) * sizeof(float) + 256;
 }
 
 int mnx_tp_bwd_f32(int32_t config, int32_t C, const float* x, const float* Y, const float* w, const float* gout,
@@ -147,7 +183,8 @@ int mnx_tp_bwd_rows_f32(int32_t config, int32_t C, const float* x, const float* 
     if (N == 0 || E == 0) return MNX_OK;
     MNX_REQUIRE(x && Y && w && gout && row_ptr && perm && snd, "null pointer argument");
     const TPConfigInfo& cfg = kTPConfigs[config];
-    const int npart = int(bwd_partials(config, C));
+    const int lw = all_lanes(N, C);
+    const int npart = lw ? int(cfg.ngroups * ceil_div(C, lw)) : int(bwd_partials(config, C));
     float* part = nullptr;
     if (gY) {
         const size_t need = mnx_tp_bwd_workspace_bytes(config, C, E);
@@ -157,12 +194,20 @@ int mnx_tp_bwd_rows_f32(int32_t config, int32_t C, const float* x, const float* 
         // out-of-range indices), so the buffer needs no clearing.
         part = static_cast<float*>(ws);
     }
+    if (lw) {
+        hipLaunchKernelGGL(kTPBwdAll[config][lanes_index(lw)], all_grid(N, C, lw, cfg.ngroups), dim3(64), 0,
+                           (hipStream_t)stream, x, Y, w, gout, row_ptr, perm, snd, wrow, N, C, gx, gw, part, npart, 0);
+        MNX_CHECK_LAUNCH();
+    }
     int pbase = 0;
-    for (int g = 0; g < cfg.ngroups; ++g) {
-        const int cblocks = int(ceil_div(C, 64 * kTPBwdCPL[config][g]));
-        const bool full = C % (64 * kTPBwdCPL[config][g]) == 0;
-        hipLaunchKernelGGL((full ? kTPBwdF : kTPBwd)[config][g], node_grid(N, cblocks), dim3(64), 0,
-                           (hipStream_t)stream, x, Y, w, gout,
+    for (int g = 0; !lw && g < cfg.ngroups; ++g) {
+        // two channels per lane where a group's register budget allows, but not for channels that
+        // one per lane already covers (half the lanes would idle)
+        const int cpl = C <= 64 ? 1 : kTPBwdCPL[config][g];
+        const int cblocks = int(ceil_div(C, 64 * cpl));
+        const bool full = C % (64 * cpl) == 0;
+        const TPBwdFn fn = C <= 64 ? (full ? kTPBwdF1 : kTPBwd1)[config][g] : (full ? kTPBwdF : kTPBwd)[config][g];
+        hipLaunchKernelGGL(fn, node_grid(N, cblocks), dim3(64), 0, (hipStream_t)stream, x, Y, w, gout,
                            row_ptr, perm, snd, wrow, N, C, gx, gw, part, npart, pbase);
         MNX_CHECK_LAUNCH();
         pbase += cblocks;

@@ -83,17 +83,18 @@ __device__ __forceinline__ void rs_step(float (&a)[V], int lane) {
     }
 }
 
-// Sum V per-lane values over the 64 lanes; returns one of the V sums, which one
-// given by reduce_scatter_index (lanes sharing an index hold the same sum).
-template <int V>
+// Sum V per-lane values over the wavefront's lanes, or over each aligned group of
+// LW of them; returns one of the V sums, which one given by reduce_scatter_index
+// (lanes sharing an index hold the same sum).
+template <int V, int LW = 64>
 __device__ __forceinline__ float wave_reduce_scatter(float (&a)[V], int lane) {
-    rs_step<32, V, V>(a, lane);
+    rs_step<LW / 2, V, V>(a, lane);
     return a[0];
 }
 
-template <int V>
+template <int V, int LW = 64>
 __device__ __forceinline__ int reduce_scatter_index(int lane) {
-    int idx = 0, off = 32;
+    int idx = 0, off = LW / 2;
 #pragma unroll
     for (int cnt = V; cnt > 1; cnt >>= 1) {
         if (lane & off) idx += cnt >> 1;
