@@ -535,6 +535,16 @@ int mnx_bessel_cutoff_f32(const float* r, int64_t num_edges, int32_t num_radial,
 int mnx_bessel_cutoff_bwd_f32(const float* r, int64_t num_edges, int32_t num_radial, double r_cut, double eps,
                               const float* mu, const float* sigma, int32_t cutoff, int32_t exponent,
                               const float* grad, float* grad_r, mnx_stream_t stream);
+/* Rows [num_radial features of mnx_bessel_cutoff | table[ti] | table[tj]] of num_radial + 2 dim floats, and
+ * the envelope u (all 1 without a cutoff); table [num_types][dim], a type outside it gives NaN.  Backward:
+ * dL/dr from the first num_radial columns of grad [num_edges][row] and from grad_u. */
+int mnx_pair_features_f32(const float* r, const int64_t* ti, const int64_t* tj, int64_t num_edges, int32_t num_radial,
+                          double r_cut, double eps, const float* mu, const float* sigma, int32_t cutoff,
+                          int32_t exponent, const float* table, int64_t num_types, int32_t dim, float* out, float* u,
+                          mnx_stream_t stream);
+int mnx_pair_features_bwd_f32(const float* r, int64_t num_edges, int32_t num_radial, double r_cut, double eps,
+                              const float* mu, const float* sigma, int32_t cutoff, int32_t exponent, const float* grad,
+                              int32_t row, const float* grad_u, float* grad_r, mnx_stream_t stream);
 
 /* ------------------------------------------------------------------------ */
 /* Hidden stack of the radial weight MLP (replaces mlp[:-1] of               */

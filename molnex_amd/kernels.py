@@ -2942,6 +2942,68 @@ def _bc_bwd(ctx, grad):
 bessel_cutoff.register_autograd(_bc_bwd, setup_context=_bc_setup)
 
 
+@_op("molix::pair_features")
+def pair_features(r: Tensor, ti: Tensor, tj: Tensor, table: Tensor, num_radial: int, r_cut: float, eps: float,
+                  mu: Tensor | None, sigma: Tensor | None, cutoff: int, exponent: int) -> tuple[Tensor, Tensor]:
+    """``(cat([bessel_cutoff(r), table[ti], table[tj]], -1), cutoff(r))`` of (E,) float32 distances and int64
+    types in one kernel each way (``allegro.py:137-249``); the (types, dim) table takes no gradient."""
+    _require_gpu("pair_features", r, ti, tj, table, mu, sigma)
+    if (r.dim() != 1 or ti.shape != r.shape or tj.shape != r.shape or ti.dtype != torch.int64
+            or tj.dtype != torch.int64 or table.dim() != 2 or table.dtype != torch.float32):
+        raise ValueError("pair_features: r (E,), ti and tj int64 (E,), table float32 (types, dim)")
+    rr, m, sg = _basis_args(r, mu, sigma, num_radial)
+    i, j, tab = ti.contiguous(), tj.contiguous(), table.detach().contiguous()
+    out = rr.new_empty(rr.shape[0], num_radial + 2 * tab.shape[1])
+    u = rr.new_empty(rr.shape[0])
+    check(_lib.load().mnx_pair_features_f32(ptr(rr), ptr(i), ptr(j), rr.shape[0], num_radial, float(r_cut), float(eps),
+                                            ptr(m), ptr(sg), cutoff, exponent, ptr(tab), tab.shape[0], tab.shape[1],
+                                            ptr(out), ptr(u), _stream(rr)), "pair_features")
+    return out, u
+
+
+@pair_features.register_fake
+def _(r, ti, tj, table, num_radial, r_cut, eps, mu, sigma, cutoff, exponent):
+    return (r.new_empty(r.shape[0], num_radial + 2 * table.shape[1], dtype=torch.float32),
+            r.new_empty(r.shape[0], dtype=torch.float32))
+
+
+@_op("molix::pair_features_backward")
+def pair_features_backward(grad: Tensor, grad_u: Tensor, r: Tensor, num_radial: int, r_cut: float, eps: float,
+                           mu: Tensor | None, sigma: Tensor | None, cutoff: int, exponent: int) -> Tensor:
+    rr, m, sg = _basis_args(r, mu, sigma, num_radial)
+    g, gu = grad.to(torch.float32).contiguous(), grad_u.to(torch.float32).contiguous()
+    if g.dim() != 2 or g.shape[0] != rr.shape[0] or g.shape[1] < num_radial or gu.shape != rr.shape:
+        raise ValueError("pair_features_backward: grad (E, >= num_radial), grad_u (E,)")
+    gr = rr.new_empty(rr.shape[0])
+    check(_lib.load().mnx_pair_features_bwd_f32(ptr(rr), rr.shape[0], num_radial, float(r_cut), float(eps), ptr(m),
+                                                ptr(sg), cutoff, exponent, ptr(g), g.shape[1], ptr(gu), ptr(gr),
+                                                _stream(rr)), "pair_features backward")
+    return gr
+
+
+@pair_features_backward.register_fake
+def _(grad, grad_u, r, num_radial, r_cut, eps, mu, sigma, cutoff, exponent):
+    return r.new_empty(r.shape, dtype=torch.float32)
+
+
+def _pf_setup(ctx, inputs, output):
+    r, _, _, _, num_radial, r_cut, eps, mu, sigma, cutoff, exponent = inputs
+    ctx.save_for_backward(r, mu, sigma)
+    ctx.args = (num_radial, r_cut, eps, cutoff, exponent)
+
+
+def _pf_bwd(ctx, grad, grad_u):
+    r, mu, sigma = ctx.saved_tensors
+    n, r_cut, eps, cutoff, exponent = ctx.args
+    gr = None
+    if ctx.needs_input_grad[0]:
+        gr = pair_features_backward(grad, grad_u, r, n, r_cut, eps, mu, sigma, cutoff, exponent).to(r.dtype)
+    return gr, None, None, None, None, None, None, None, None, None, None
+
+
+pair_features.register_autograd(_pf_bwd, setup_context=_pf_setup)
+
+
 
 
 # ---------------------------------------------------------------------------

@@ -32,7 +32,7 @@ from .. import kernels as K
 from ..config import config
 from ..irreps import Irreps
 from ..molrep.embedding.angular import SphericalHarmonics
-from ..molrep.embedding.cutoff import PolynomialCutoff
+from ..molrep.embedding.cutoff import CosineCutoff, PolynomialCutoff
 from ..molrep.embedding.radial import BesselRBF
 from ..molrep.interaction.linear import Linear
 from ..molrep.interaction.tensor_product import irreps_from_l_max, sh_irreps_from_l_max
@@ -126,6 +126,25 @@ def _envelope_stack(per_layer, u):
         return _EnvelopeStack.apply(u, *per_layer)
     stacked = torch.stack(per_layer, dim=1)
     return _times_envelope(stacked.reshape(stacked.shape[0], -1), u).reshape(stacked.shape)
+
+
+def _pair_features(rbf, cutoff_fn, emb: nn.Embedding, r: torch.Tensor, zs: torch.Tensor, zd: torch.Tensor):
+    """``(cat([rbf(r) * cutoff_fn(r), emb(zs), emb(zd)], -1), cutoff_fn(r))``: one kernel each way
+    (``molix::pair_features``) for a Bessel basis and a cosine or polynomial cutoff of one radius on
+    (E,) float32 GPU distances with the embedding frozen, else the modules."""
+    w = emb.weight
+    kind = 1 if type(cutoff_fn) is CosineCutoff else 2 if type(cutoff_fn) is PolynomialCutoff else 0
+    if (kind and type(rbf) is BesselRBF and r.is_cuda and r.dtype == torch.float32 and r.dim() == 1
+            and rbf.config.num_radial <= 32 and float(cutoff_fn.config.r_cut) == rbf.r_cut
+            and (kind == 1 or cutoff_fn.exponent <= 64) and zs.shape == zd.shape == r.shape
+            and w.dtype == torch.float32 and not (torch.is_grad_enabled() and w.requires_grad)
+            and emb.padding_idx is None and emb.max_norm is None and w.shape[1] <= 4096
+            and not zs.is_floating_point()):
+        mu, sigma = (rbf.mu, rbf.sigma) if rbf.normalize else (None, None)
+        return K.pair_features(r, zs.long(), zd.long(), w, int(rbf.config.num_radial), rbf.r_cut, rbf.eps, mu, sigma,
+                               kind, cutoff_fn.exponent if kind == 2 else 0)
+    cut = cutoff_fn(r)
+    return torch.cat([rbf(r) * cut.unsqueeze(-1), _type_pair_embedding(emb, zs, zd)], dim=-1), cut
 
 
 def _type_pair_embedding(emb: nn.Embedding, zs: torch.Tensor, zd: torch.Tensor) -> torch.Tensor:
@@ -556,11 +575,10 @@ class PairEmbedding(nn.Module):
         tensor track ``harmonics x env weights`` is formed (env weights None with ``env=False``:
         ``tensor_env`` of the scalar features, left to the caller)."""
         src, dst = edge_index[:, 0], edge_index[:, 1]
-        edge_cutoff = self.cutoff_fn(bond_dist)
-        edge_radial = self.radial_basis(bond_dist) * edge_cutoff.unsqueeze(-1)
         edge_angular = self.spherical_harmonics(bond_diff / (bond_dist.unsqueeze(-1) + 1e-8))
-        type_embed = _type_pair_embedding(self.type_embedding, Z[src], Z[dst])
-        scalar_features = _silu_stack(self.scalar_mlp, torch.cat([edge_radial, type_embed], dim=-1))
+        pair, edge_cutoff = _pair_features(self.radial_basis, self.cutoff_fn, self.type_embedding, bond_dist, Z[src],
+                                           Z[dst])
+        scalar_features = _silu_stack(self.scalar_mlp, pair)
         return scalar_features, self.tensor_env(scalar_features) if env else None, edge_angular, edge_cutoff
 
     def forward(self, Z, bond_dist, bond_diff, edge_index):

@@ -113,6 +113,13 @@ def bessel_cutoff_torch(r: Tensor, num_radial: int, r_cut: float, eps: float, mu
         phi = (phi - mu.to(r.dtype)) / sigma.to(r.dtype)
     if cutoff == 0:
         return phi
+    return phi * envelope_torch(r, r_cut, cutoff, exponent).unsqueeze(-1)
+
+
+def envelope_torch(r: Tensor, r_cut: float, cutoff: int, exponent: int) -> Tensor:
+    """The cutoff envelope of ``molix::bessel_cutoff`` and ``molix::pair_features`` in torch."""
+    if cutoff == 0:
+        return torch.ones_like(r)
     if cutoff == 1:
         c = 0.5 * (torch.cos(math.pi * (r / r_cut)) + 1.0)
     else:
@@ -121,8 +128,7 @@ def bessel_cutoff_torch(r: Tensor, num_radial: int, r_cut: float, eps: float, mu
         for k in range(exponent - 2, -1, -1):
             g = g * x + float((k + 2) * (k + 1) // 2)
         c = (1.0 - x) ** 3 * g
-    c = torch.where(r < r_cut, c, torch.zeros_like(c))
-    return phi * c.unsqueeze(-1)
+    return torch.where(r < r_cut, c, torch.zeros_like(c))
 
 
 def _bc2_setup(ctx, inputs, output):
@@ -145,6 +151,35 @@ def _bc2_bwd(ctx, ggr):
 
 
 K.bessel_cutoff_backward.register_autograd(_bc2_bwd, setup_context=_bc2_setup)
+
+
+def _pf2_setup(ctx, inputs, output):
+    grad, grad_u, r, num_radial, r_cut, eps, mu, sigma, cutoff, exponent = inputs
+    ctx.save_for_backward(grad, grad_u, r, mu, sigma)
+    ctx.args = (num_radial, r_cut, eps, cutoff, exponent)
+
+
+def _pf2_bwd(ctx, ggr):
+    g, gu, r, mu, sigma = ctx.saved_tensors
+    n, r_cut, eps, cutoff, exponent = ctx.args
+    ng, nu, nr = ctx.needs_input_grad[:3]
+
+    def both(rr):
+        return torch.cat([bessel_cutoff_torch(rr, n, r_cut, eps, mu, sigma, cutoff, exponent),
+                          envelope_torch(rr, r_cut, cutoff, exponent).unsqueeze(-1)], dim=-1)
+
+    # in fp64, as _bc2_bwd; the columns past the radial features do not depend on r
+    seed = None if ggr is None else ggr.double()
+    dg, dr = _vjp_second(both, [r.double()], torch.cat([g[:, :n], gu.unsqueeze(-1)], dim=-1).double(), [seed],
+                         [ng or nu, nr])
+    dgrad = dgu = None
+    if dg is not None:
+        dgrad = torch.nn.functional.pad(dg[:, :n].to(g.dtype), (0, g.shape[1] - n)) if ng else None
+        dgu = dg[:, n].to(gu.dtype) if nu else None
+    return dgrad, dgu, None if dr is None else dr.to(r.dtype), None, None, None, None, None, None, None
+
+
+K.pair_features_backward.register_autograd(_pf2_bwd, setup_context=_pf2_setup)
 
 
 # ---------------------------------------------------------------------------
