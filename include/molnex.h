@@ -535,6 +535,10 @@ int mnx_bessel_cutoff_f32(const float* r, int64_t num_edges, int32_t num_radial,
 int mnx_bessel_cutoff_bwd_f32(const float* r, int64_t num_edges, int32_t num_radial, double r_cut, double eps,
                               const float* mu, const float* sigma, int32_t cutoff, int32_t exponent,
                               const float* grad, float* grad_r, mnx_stream_t stream);
+/* Blocks of updated = a s + b (W [s, t] + c), W (S, S + F): ws = a I + b W[:, :S], wt = b W[:, S:], its
+ * transpose wt_t (F, S), bc = b c. */
+int mnx_residual_blocks_f32(const float* weight, const float* bias, int32_t S, int32_t F, double a, double b, float* ws,
+                            float* wt, float* wt_t, float* bc, mnx_stream_t stream);
 /* Rows [num_radial features of mnx_bessel_cutoff | table[ti] | table[tj]] of num_radial + 2 dim floats, and
  * the envelope u (all 1 without a cutoff); table [num_types][dim], a type outside it gives NaN.  Backward:
  * dL/dr from the first num_radial columns of grad [num_edges][row] and from grad_u. */

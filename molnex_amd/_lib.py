@@ -108,6 +108,7 @@ SIGNATURES = {
     "mnx_bond_vectors_bwd_f32": (C.c_int, [vp, vp, c_i64, c_i64, vp, vp]),
     "mnx_bessel_cutoff_f32": (C.c_int, [vp, c_i64, c_i32, c_f64, c_f64, vp, vp, c_i32, c_i32, vp, vp]),
     "mnx_bessel_cutoff_bwd_f32": (C.c_int, [vp, c_i64, c_i32, c_f64, c_f64, vp, vp, c_i32, c_i32, vp, vp, vp]),
+    "mnx_residual_blocks_f32": (C.c_int, [vp, vp, c_i32, c_i32, c_f64, c_f64, vp, vp, vp, vp, vp]),
     "mnx_pair_features_f32": (C.c_int, [vp, vp, vp, c_i64, c_i32, c_f64, c_f64, vp, vp, c_i32, c_i32, vp, c_i64, c_i32, vp,
                                         vp, vp]),
     "mnx_pair_features_bwd_f32": (C.c_int, [vp, c_i64, c_i32, c_f64, c_f64, vp, vp, c_i32, c_i32, vp, c_i32, vp, vp, vp]),

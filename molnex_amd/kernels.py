@@ -2872,6 +2872,28 @@ def _(grad, y, s, need_y, need_s):
             + [t.new_empty(t.shape) if need_s else t.new_empty(0) for t in s])
 
 
+@_op("molix::residual_blocks")
+def residual_blocks(weight: Tensor, bias: Tensor, a: float, b: float) -> tuple[Tensor, Tensor, Tensor, Tensor]:
+    """``(a I + b W_s, b W_t, (b W_t)^T, b c)`` of a linear layer with the (S, S + F) weight
+    ``[W_s | W_t]`` and bias ``c``: the blocks of ``a s + b (W [s, t] + c)`` (no gradient)."""
+    _require_gpu("residual_blocks", weight, bias)
+    if (weight.dim() != 2 or weight.dtype != torch.float32 or bias.dtype != torch.float32
+            or bias.shape != weight.shape[:1] or weight.shape[1] < weight.shape[0]):
+        raise ValueError("residual_blocks: weight float32 (S, S + F), bias float32 (S,)")
+    w, c = weight.detach().contiguous(), bias.detach().contiguous()
+    S, F = w.shape[0], w.shape[1] - w.shape[0]
+    ws, wt, wtt, bc = w.new_empty(S, S), w.new_empty(S, F), w.new_empty(F, S), w.new_empty(S)
+    check(_lib.load().mnx_residual_blocks_f32(ptr(w), ptr(c), S, F, float(a), float(b), ptr(ws), ptr(wt), ptr(wtt),
+                                              ptr(bc), _stream(w)), "residual_blocks")
+    return ws, wt, wtt, bc
+
+
+@residual_blocks.register_fake
+def _(weight, bias, a, b):
+    S, F = weight.shape[0], weight.shape[1] - weight.shape[0]
+    return weight.new_empty(S, S), weight.new_empty(S, F), weight.new_empty(F, S), weight.new_empty(S)
+
+
 # ---------------------------------------------------------------------------
 # Radial edge embedding (Bessel basis x cutoff envelope)
 # ---------------------------------------------------------------------------

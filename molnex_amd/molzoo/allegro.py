@@ -169,14 +169,12 @@ def _tail_torch(s, nt, lat, tenv, a, b, F):
     return updated, _scale_by_channel(nt, tenv(updated), None, F)
 
 
-def _tail_weights(layer, S):
-    """(W_s, W_t, b c) of the frozen tail: ``updated = s W_s^T + nt[:, :F] W_t^T + b c`` with the
+def _tail_weights(layer):
+    """(W_s, W_t, W_t^T, b c) of the frozen tail: ``updated = s W_s^T + nt[:, :F] W_t^T + b c`` with the
     residual folded into the square block (``W_s = b W[:, :S] + a I``: ``a s`` needs no pass of its
     own, forward or backward)."""
     lat = layer.latent_mlp[0]
-    a, b = layer.residual_a, layer.residual_b
-    ws = torch.eye(S, dtype=lat.weight.dtype, device=lat.weight.device).mul_(a).add_(lat.weight[:, :S], alpha=b)
-    return ws, lat.weight[:, S:] * b, lat.bias * b
+    return K.residual_blocks(lat.weight, lat.bias, layer.residual_a, layer.residual_b)
 
 
 def _row_linear(h, weight, bias=None):
@@ -240,12 +238,12 @@ class _LayerTail(torch.autograd.Function):
     def forward(ctx, s, nt, layer):
         tenv = layer.tensor_env
         F = layer.num_tensor_features
-        ws, wt, bc = _tail_weights(layer, s.shape[1])
+        ws, wt, _, bc = _tail_weights(layer)
         upd = _row_linear(s, ws, bc)
         upd.addmm_(nt[:, :F], wt.t())
         tv = torch.addmm(tenv.bias, upd, tenv.weight.t())
         out = K.channel_scale(nt, tv, nt.shape[1] // F)
-        ctx.save_for_backward(s, nt, tv)
+        ctx.save_for_backward(s, nt, tv, ws, wt)
         ctx.layer = layer
         # an output nothing uses (the last layer's tensor track) arrives as None, not as zeros
         ctx.set_materialize_grads(False)
@@ -253,7 +251,7 @@ class _LayerTail(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g_upd, g_out):
-        s, nt, tv = ctx.saved_tensors
+        s, nt, tv, ws, wt = ctx.saved_tensors
         layer = ctx.layer
         lat, tenv = layer.latent_mlp[0], layer.tensor_env
         a, b, F = layer.residual_a, layer.residual_b, layer.num_tensor_features
@@ -262,11 +260,11 @@ class _LayerTail(torch.autograd.Function):
             # differentiated again (create_graph): the same gradient formulas in tracked ops
             g_s, g_nt = _tail_grads_tracked(layer, s, nt, g_upd, g_out, need_s, need_nt)
             return g_s, g_nt, None
-        g_s, g_nt = _tail_grads(layer, s, nt, tv, g_upd, g_out, need_s, need_nt)
+        g_s, g_nt = _tail_grads(layer, s, nt, tv, ws, wt, g_upd, g_out, need_s, need_nt)
         return g_s, g_nt, None
 
 
-def _tail_grads(layer, s, nt, tv, g_upd, g_out, need_s, need_nt):
+def _tail_grads(layer, s, nt, tv, ws, wt, g_upd, g_out, need_s, need_nt):
     """(grad s, grad nt) of the frozen tail: with ``g_lat = g_upd + g_tv T`` (T the env layer's
     weight), ``g_s = g_upd W_s + g_tv (T W_s)`` and the scalar columns of nt get
     ``g_upd W_t + g_tv (T W_t)``: two products each, the second accumulated in the same pass, and the
@@ -279,7 +277,6 @@ def _tail_grads(layer, s, nt, tv, g_upd, g_out, need_s, need_nt):
         g_nt = torch.zeros_like(nt) if need_nt else None
     if g_upd is None and g_tv is None:
         return None, (g_nt if need_nt else None)
-    ws, wt, _ = _tail_weights(layer, s.shape[1])
     g_upd = g_upd.contiguous() if g_upd is not None else None
 
     def through(w):
@@ -322,18 +319,18 @@ class _LayerChain(torch.autograd.Function):
             tvp = torch.addmm(tvp_lin.bias, s, tvp_lin.weight.t())
         xs = _row_linear(s, ee.weight, ee.bias)
         nt = K.edge_tp_proj(V, eY, w, layer.tp.config_id, proj, xs, tvp)  # the product scales by xs tvp
-        ws, wt, bc = _tail_weights(layer, s.shape[1])
-        upd = _row_grad(nt[:, :F], wt.t().contiguous(), _row_linear(s, ws, bc))
+        ws, wt, wtt, bc = _tail_weights(layer)
+        upd = _row_grad(nt[:, :F], wtt, _row_linear(s, ws, bc))
         # the last layer's env weights scale only its tensor output, which an encoder does not return
         tv = torch.addmm(tenv.bias, upd, tenv.weight.t()) if need_tv else None
-        ctx.save_for_backward(s, V, tvp, eY, w, proj, xs)
+        ctx.save_for_backward(s, V, tvp, eY, w, proj, xs, ws, wt)
         ctx.layer, ctx.tvp_lin = layer, tvp_lin
         ctx.set_materialize_grads(False)
         return upd, nt, tv, s
 
     @staticmethod
     def backward(ctx, g_upd, g_nt, g_tv, g_pass):
-        s, V, tvp, eY, w, proj, xs = ctx.saved_tensors
+        s, V, tvp, eY, w, proj, xs, ws, wt = ctx.saved_tensors
         layer, tl = ctx.layer, ctx.tvp_lin
         ee, tenv, cfg = layer.env_embed, layer.tensor_env, layer.tp.config_id
         a, b, F = layer.residual_a, layer.residual_b, layer.num_tensor_features
@@ -377,9 +374,7 @@ class _LayerChain(torch.autograd.Function):
                         g_s = g_s + g_pass
             return (g_s, gV.reshape(V.shape) if need_V else None, g_tvp if need_tvp else None,
                     geY.reshape(eY.shape) if need_eY else None, None, None, None, None, None)
-        ws = None
         if g_upd is not None or g_tv is not None:
-            ws, wt, _ = _tail_weights(layer, s.shape[1])
             # g_upd may be a strided slice of the stacked features' gradient: the row kernel reads it
             # in place
             g_tv = g_tv.contiguous() if g_tv is not None else None
