@@ -921,8 +921,8 @@ __device__ __forceinline__ void scan_cells(const T* __restrict__ pos, const T* _
                             s_y[base + lane] = p.y + sy;
                             s_z[base + lane] = p.z + sz;
                             s_id[base + lane] = atoms_sorted[slot];
-                        } else {  // past the end (of the last 64): too far from everything
-                            s_x[base + lane] = s_y[base + lane] = s_z[base + lane] = T(1e30);
+                        } else {  // past the end (of the last 64): NaN passes no test, whatever the cutoff
+                            s_x[base + lane] = s_y[base + lane] = s_z[base + lane] = T(__builtin_nan(""));
                             s_id[base + lane] = INT32_MAX;
                         }
                     }

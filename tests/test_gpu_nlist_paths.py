@@ -94,3 +94,16 @@ def test_duplicates_and_another_stream():
     want = [neighbor_list(t, 4.0, None, True) for t in (a, a.flip(0).contiguous())]
     for got, ref in zip(outs, want):
         assert all(torch.equal(x, y) for x, y in zip(got, ref))
+
+
+@pytest.mark.parametrize("dtype,cut", [(np.float32, 1e20), (np.float64, 1e200)])
+def test_cutoff_whose_square_overflows(dtype, cut):
+    """Every pair of an open system that takes the cell scan (lanes past its candidates match nothing)."""
+    pos = np.random.default_rng(5).uniform(0, 30, (2100, 3)).astype(dtype)
+    empty = torch.empty((0, 0), dtype=torch.from_numpy(pos).dtype, device=DEV)
+    for full in (False, True):
+        i, j, _, _, r = (t.cpu().numpy() for t in ops.neighbor_list(torch.from_numpy(pos).to(DEV), cut, empty, full))
+        wi, wj = np.nonzero(~np.eye(len(pos), dtype=bool) if full else np.tri(len(pos), k=-1, dtype=bool))
+        assert np.array_equal(i, wi) and np.array_equal(j, wj)
+        want = np.linalg.norm((pos[wi] - pos[wj]).astype(np.float64), axis=1)
+        np.testing.assert_allclose(r, want, rtol=8 * np.finfo(dtype).eps)
