@@ -349,7 +349,7 @@ int mnx_pme_gather_f64(const double* pos, const double* charges, const double* b
  * (both or neither) its derivatives.  *overflow (device) becomes non-zero when an atom has more than
  * 4096 neighbours; it is written only for more than 2048 atoms.  Workspace: mnx_nlist_workspace_bytes.
  * convolve_add: mnx_pme_convolve whose energy also includes sum(more[0..nmore)); with mods64 the moduli
- * are doubles (used in the entry point's precision), else of its type.  gather_add:
+ * are doubles, else of the entry point's type.  gather_add:
  * mnx_pme_gather whose derivatives are (reciprocal + dpos_add / dq_add) * *grad, where these device
  * pointers are not NULL. */
 int64_t mnx_pme_real_partials(int64_t num_atoms);

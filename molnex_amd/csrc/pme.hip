@@ -341,7 +341,7 @@ constexpr int kConvThreads = 256;
 // per-block energy partial sums (pme_cpu.cpp:263-294).
 template <typename T>
 __global__ void __launch_bounds__(kConvThreads) k_convolve(T* __restrict__ cgrid, const T* __restrict__ box, int gx,
-                                                           int gy, int gz, T alpha, const void* __restrict__ xm,
+                                                           int gy, int gz, double alpha, const void* __restrict__ xm,
                                                            const void* __restrict__ ym, const void* __restrict__ zm,
                                                            bool mods64, double* __restrict__ partials) {
     __shared__ double red[kConvThreads];
@@ -350,7 +350,11 @@ __global__ void __launch_bounds__(kConvThreads) k_convolve(T* __restrict__ cgrid
     const int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     double e = 0.0;
     if (idx < total) {
-        const Recip<T> R = invert_box<T>(box);
+        // the influence function and the energy's terms in fp64, rounded once: the energy is a small
+        // difference from the self term, where a factor common to all terms, rounded in T, shows
+        double b64[9];
+        for (int k = 0; k < 9; ++k) b64[k] = double(box[k]);
+        const Recip<double> R = invert_box<double>(b64);
         // the mesh has fewer than 2^31 points
         const uint32_t i32 = uint32_t(idx), plane = uint32_t(gy) * zs;
         const int kx = int(i32 / plane);
@@ -360,24 +364,24 @@ __global__ void __launch_bounds__(kConvThreads) k_convolve(T* __restrict__ cgrid
         const int mx = kx < (gx + 1) / 2 ? kx : kx - gx;
         const int my = ky < (gy + 1) / 2 ? ky : ky - gy;
         const int mz = kz < (gz + 1) / 2 ? kz : kz - gz;
-        const T mhx = mx * R.r[0][0];
-        const T mhy = mx * R.r[1][0] + my * R.r[1][1];
-        const T mhz = mx * R.r[2][0] + my * R.r[2][1] + mz * R.r[2][2];
-        const T m2 = mhx * mhx + mhy * mhy + mhz * mhz;
-        const T scale_f = T(M_PI) * box[0] * box[4] * box[8];
-        // the moduli in T or (mods64) in double, rounded to T
+        const double mhx = mx * R.r[0][0];
+        const double mhy = mx * R.r[1][0] + my * R.r[1][1];
+        const double mhz = mx * R.r[2][0] + my * R.r[2][1] + mz * R.r[2][2];
+        const double m2 = mhx * mhx + mhy * mhy + mhz * mhz;
+        const double scale_f = M_PI * b64[0] * b64[4] * b64[8];
+        // the moduli in T or (mods64) in double
         auto mod = [&](const void* m, int k) {
-            return mods64 ? T(static_cast<const double*>(m)[k]) : static_cast<const T*>(m)[k];
+            return mods64 ? static_cast<const double*>(m)[k] : double(static_cast<const T*>(m)[k]);
         };
-        const T denom = m2 * (scale_f * mod(xm, kx) * mod(ym, ky)) * mod(zm, kz);
-        const T rexp = T(M_PI * M_PI) / (alpha * alpha);
-        const T eterm = idx == 0 ? T(0) : exp(-rexp * m2) / denom;
-        const T s = (kz > 0 && kz <= (gz - 1) / 2) ? T(2) : T(1);
+        const double denom = m2 * (scale_f * mod(xm, kx) * mod(ym, ky)) * mod(zm, kz);
+        const double rexp = M_PI * M_PI / (alpha * alpha);
+        const double eterm = idx == 0 ? 0.0 : exp(-rexp * m2) / denom;
+        const double s = (kz > 0 && kz <= (gz - 1) / 2) ? 2.0 : 1.0;
         T* c = cgrid + 2 * idx;
-        const T re = c[0], im = c[1];
-        e = double(s * eterm * (re * re + im * im));
-        c[0] = re * eterm;
-        c[1] = im * eterm;
+        const double re = c[0], im = c[1];
+        e = s * eterm * (re * re + im * im);
+        c[0] = T(re * eterm);
+        c[1] = T(im * eterm);
     }
     red[threadIdx.x] = e;
     __syncthreads();
@@ -711,7 +715,7 @@ int convolve(T* cgrid, const T* box, int gx, int gy, int gz, double alpha, const
     if (!ws || ws_bytes < size_t(nb) * sizeof(double))
         return set_error(MNX_ERR_WORKSPACE, "workspace %zu < %zu bytes", ws_bytes, size_t(nb) * sizeof(double));
     double* part = static_cast<double*>(ws);
-    hipLaunchKernelGGL((k_convolve<T>), dim3(nb), dim3(kConvThreads), 0, s, cgrid, box, gx, gy, gz, T(alpha), xm, ym,
+    hipLaunchKernelGGL((k_convolve<T>), dim3(nb), dim3(kConvThreads), 0, s, cgrid, box, gx, gy, gz, alpha, xm, ym,
                        zm, mods64, part);
     MNX_CHECK_LAUNCH();
     hipLaunchKernelGGL((k_sum_partials<T>), dim3(1), dim3(1024), 0, s, part, nb, 0.5, more, nmore, energy);
