@@ -1035,7 +1035,7 @@ def pme_energy(positions: Tensor, charges: Tensor, box_vectors: Tensor, xmoduli:
     b = box_vectors.detach().to(device=dev, dtype=dt).contiguous()
     if tuple(b.shape) != (3, 3) or tuple(pos.shape) != (n, 3) or tuple(q.shape) != (n,):
         raise ValueError("pme_energy: positions must be (n, 3), charges (n,) and box_vectors (3, 3)")
-    # moduli in float64 (as the module keeps them) are used as they are, rounded by the kernel
+    # moduli in float64 (as the module keeps them) are used as they are by the kernel
     mdt = torch.float64 if xmoduli.dtype == ymoduli.dtype == zmoduli.dtype == torch.float64 else dt
     mods = [m.detach().to(device=dev, dtype=mdt).contiguous() for m in (xmoduli, ymoduli, zmoduli)]
     if any(m.numel() < g for m, g in zip(mods, (gridx, gridy, gridz))):
@@ -1127,6 +1127,10 @@ def _pme_energy_setup(ctx, inputs, output):
 def _pme_energy_bwd(ctx, grad, *_):
     if grad is None:
         return (None,) * 14
+    if torch.is_grad_enabled():
+        # differentiated again: linear in grad, tracked (the derivatives themselves have no formula)
+        gpos, gq = pme_energy_backward(torch.ones_like(grad), *ctx.saved_tensors, *ctx.args)
+        return (gpos * grad, gq * grad) + (None,) * 12
     gpos, gq = pme_energy_backward(grad, *ctx.saved_tensors, *ctx.args)
     return (gpos, gq) + (None,) * 12
 

@@ -117,3 +117,17 @@ def test_opcheck():
     pos.requires_grad_(True), q.requires_grad_(True)
     torch.library.opcheck(torch.ops.molix.pme_energy.default,
                           (pos, q, box, pme.xmoduli, pme.ymoduli, pme.zmoduli, 16, 16, 16, 4, 0.4, 3.5, 1.0, True))
+
+
+def test_scaled_forces_differentiated_by_the_scale():
+    """The gradient is linear in its upstream gradient, also under create_graph: |w F|^2 by w."""
+    pos, q, box = _system(300, 15.0, 3)
+    pme = PMEPotential(alpha=0.4, grid=(16, 16, 16), order=4, cutoff=4.5).to(DEV)
+    _, gp, gq = _run(pme, pos, q, box)
+    w = torch.tensor(1.5, dtype=pos.dtype, device=DEV, requires_grad=True)
+    p, c = pos.clone().requires_grad_(True), q.clone().requires_grad_(True)
+    fp, fq = torch.autograd.grad(w * pme(p, c, box), (p, c), create_graph=True)
+    (gw,) = torch.autograd.grad(fp.square().sum() + fq.square().sum(), w, retain_graph=True)
+    torch.testing.assert_close(gw, 2 * 1.5 * (gp.square().sum() + gq.square().sum()), rtol=1e-11, atol=0.0)
+    with pytest.raises(RuntimeError, match="no autograd formula"):
+        torch.autograd.grad(fp.square().sum(), p)
