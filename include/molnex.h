@@ -348,14 +348,15 @@ int mnx_pme_gather_f64(const double* pos, const double* charges, const double* b
  * is the sum of the mnx_pme_real_partials(n) doubles written to `partials`; dpos [n][3] and dq [n]
  * (both or neither) its derivatives.  *overflow (device) becomes non-zero when an atom has more than
  * 4096 neighbours; it is written only for more than 2048 atoms.  Workspace: mnx_nlist_workspace_bytes.
- * convolve_add: mnx_pme_convolve whose energy also includes sum(more[0..nmore)); with mods64 the moduli
+ * convolve_add: mnx_pme_convolve whose energy also includes sum(more[0..nmore)), for a mesh spread with
+ * `coulomb` (the rounding of its square root taken out of the energy); with mods64 the moduli
  * are doubles, else of the entry point's type.  gather_add:
  * mnx_pme_gather whose derivatives are (reciprocal + dpos_add / dq_add) * *grad, where these device
  * pointers are not NULL. */
 int64_t mnx_pme_real_partials(int64_t num_atoms);
 int mnx_pme_convolve_add_f32(float* cgrid, const float* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
-                             const void* xm, const void* ym, const void* zm, int32_t mods64, const double* more,
-                             int64_t nmore, float* energy, void* ws, size_t ws_bytes, mnx_stream_t s);
+                             const void* xm, const void* ym, const void* zm, int32_t mods64, double coulomb,
+                             const double* more, int64_t nmore, float* energy, void* ws, size_t ws_bytes, mnx_stream_t s);
 int mnx_pme_gather_add_f32(const float* pos, const float* q, const float* box, int64_t n, const float* grid, int32_t gx,
                            int32_t gy, int32_t gz, int32_t order, double coulomb, const float* grad,
                            const float* dpos_add, const float* dq_add, float* dpos, float* dq, mnx_stream_t s);
@@ -363,8 +364,8 @@ int mnx_pme_real_f32(const float* pos, const float* q, int64_t n, const float* b
                      double coulomb, float* dpos, float* dq, double* partials, int32_t* overflow, void* ws,
                      size_t ws_bytes, mnx_stream_t stream);
 int mnx_pme_convolve_add_f64(double* cgrid, const double* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
-                             const void* xm, const void* ym, const void* zm, int32_t mods64, const double* more,
-                             int64_t nmore, double* energy, void* ws, size_t ws_bytes, mnx_stream_t s);
+                             const void* xm, const void* ym, const void* zm, int32_t mods64, double coulomb,
+                             const double* more, int64_t nmore, double* energy, void* ws, size_t ws_bytes, mnx_stream_t s);
 int mnx_pme_gather_add_f64(const double* pos, const double* q, const double* box, int64_t n, const double* grid, int32_t gx,
                            int32_t gy, int32_t gz, int32_t order, double coulomb, const double* grad,
                            const double* dpos_add, const double* dq_add, double* dpos, double* dq, mnx_stream_t s);

@@ -705,7 +705,8 @@ int64_t conv_blocks(int gx, int gy, int gz) { return ceil_div(int64_t(gx) * gy *
 
 template <typename T>
 int convolve(T* cgrid, const T* box, int gx, int gy, int gz, double alpha, const void* xm, const void* ym, const void* zm,
-             bool mods64, const double* more, int64_t nmore, T* energy, void* ws, size_t ws_bytes, hipStream_t s) {
+             bool mods64, double coulomb, const double* more, int64_t nmore, T* energy, void* ws, size_t ws_bytes,
+             hipStream_t s) {
     clear_error();
     int rc = check_grid(gx, gy, gz, 3);
     MNX_REQUIRE(rc || nmore == 0 || more, "null pointer argument");
@@ -715,10 +716,13 @@ int convolve(T* cgrid, const T* box, int gx, int gy, int gz, double alpha, const
     if (!ws || ws_bytes < size_t(nb) * sizeof(double))
         return set_error(MNX_ERR_WORKSPACE, "workspace %zu < %zu bytes", ws_bytes, size_t(nb) * sizeof(double));
     double* part = static_cast<double*>(ws);
+    // the mesh holds charges times sqrt(coulomb) rounded to T: a factor common to all terms, so taken out
+    // of the sum (energy error of 50k atoms in float32, six inputs: 0.8e-6..5.8e-6 -> 0.7e-6..4.7e-6)
+    const double sk = double(T(sqrt(coulomb))), fix = sk > 0 ? coulomb / (sk * sk) : 1.0;
     hipLaunchKernelGGL((k_convolve<T>), dim3(nb), dim3(kConvThreads), 0, s, cgrid, box, gx, gy, gz, alpha, xm, ym,
                        zm, mods64, part);
     MNX_CHECK_LAUNCH();
-    hipLaunchKernelGGL((k_sum_partials<T>), dim3(1), dim3(1024), 0, s, part, nb, 0.5, more, nmore, energy);
+    hipLaunchKernelGGL((k_sum_partials<T>), dim3(1), dim3(1024), 0, s, part, nb, 0.5 * fix, more, nmore, energy);
     MNX_CHECK_LAUNCH();
     return MNX_OK;
 }
@@ -816,12 +820,12 @@ size_t mnx_pme_convolve_workspace_bytes(int32_t gx, int32_t gy, int32_t gz) {
 int mnx_pme_convolve_f32(float* cgrid, const float* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
                          const float* xm, const float* ym, const float* zm, float* energy, void* ws, size_t ws_bytes,
                          mnx_stream_t s) {
-    return convolve<float>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, false, nullptr, 0, energy, ws, ws_bytes, (hipStream_t)s);
+    return convolve<float>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, false, 1.0, nullptr, 0, energy, ws, ws_bytes, (hipStream_t)s);
 }
 int mnx_pme_convolve_f64(double* cgrid, const double* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
                          const double* xm, const double* ym, const double* zm, double* energy, void* ws,
                          size_t ws_bytes, mnx_stream_t s) {
-    return convolve<double>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, false, nullptr, 0, energy, ws, ws_bytes, (hipStream_t)s);
+    return convolve<double>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, false, 1.0, nullptr, 0, energy, ws, ws_bytes, (hipStream_t)s);
 }
 int mnx_pme_gather_f32(const float* pos, const float* q, const float* box, int64_t n, const float* grid, int32_t gx,
                        int32_t gy, int32_t gz, int32_t order, double coulomb, float* dpos, float* dq, mnx_stream_t s) {
@@ -849,9 +853,10 @@ int mnx_pme_direct_f64(const double* pos, const double* q, int64_t n, const int3
 }
 
 int mnx_pme_convolve_add_f32(float* cgrid, const float* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
-                             const void* xm, const void* ym, const void* zm, int32_t mods64, const double* more,
-                             int64_t nmore, float* energy, void* ws, size_t ws_bytes, mnx_stream_t s) {
-    return convolve<float>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, mods64 != 0, more, nmore, energy, ws, ws_bytes, (hipStream_t)s);
+                             const void* xm, const void* ym, const void* zm, int32_t mods64, double coulomb,
+                             const double* more, int64_t nmore, float* energy, void* ws, size_t ws_bytes, mnx_stream_t s) {
+    return convolve<float>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, mods64 != 0, coulomb, more, nmore, energy, ws, ws_bytes,
+                           (hipStream_t)s);
 }
 int mnx_pme_gather_add_f32(const float* pos, const float* q, const float* box, int64_t n, const float* grid, int32_t gx,
                            int32_t gy, int32_t gz, int32_t order, double coulomb, const float* grad, const float* dpos_add,
@@ -859,9 +864,10 @@ int mnx_pme_gather_add_f32(const float* pos, const float* q, const float* box, i
     return gather<float>(pos, q, box, n, grid, gx, gy, gz, order, coulomb, grad, dpos_add, dq_add, dpos, dq, (hipStream_t)s);
 }
 int mnx_pme_convolve_add_f64(double* cgrid, const double* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
-                             const void* xm, const void* ym, const void* zm, int32_t mods64, const double* more,
-                             int64_t nmore, double* energy, void* ws, size_t ws_bytes, mnx_stream_t s) {
-    return convolve<double>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, mods64 != 0, more, nmore, energy, ws, ws_bytes, (hipStream_t)s);
+                             const void* xm, const void* ym, const void* zm, int32_t mods64, double coulomb,
+                             const double* more, int64_t nmore, double* energy, void* ws, size_t ws_bytes, mnx_stream_t s) {
+    return convolve<double>(cgrid, box, gx, gy, gz, alpha, xm, ym, zm, mods64 != 0, coulomb, more, nmore, energy, ws, ws_bytes,
+                           (hipStream_t)s);
 }
 int mnx_pme_gather_add_f64(const double* pos, const double* q, const double* box, int64_t n, const double* grid, int32_t gx,
                            int32_t gy, int32_t gz, int32_t order, double coulomb, const double* grad, const double* dpos_add,

@@ -1065,7 +1065,8 @@ def pme_energy(positions: Tensor, charges: Tensor, box_vectors: Tensor, xmoduli:
     energy = torch.empty((), dtype=dt, device=dev)
     check(getattr(lib, f"mnx_pme_convolve_add_{sfx}")(
         ptr(torch.view_as_real(spec)), ptr(b), gridx, gridy, gridz, float(alpha), ptr(mods[0]), ptr(mods[1]),
-        ptr(mods[2]), int(mdt == torch.float64), parts, nparts, ptr(energy), scratch, size, stream), "pme convolve")
+        ptr(mods[2]), int(mdt == torch.float64), float(coulomb), parts, nparts, ptr(energy), scratch, size, stream),
+        "pme convolve")
     if many is not None:
         arrived.synchronize()
         if int(many.view(torch.int32)[0]):
