@@ -47,6 +47,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "nlist_run.h"
 #include "scan.h"
 
 namespace mnx {
@@ -1112,7 +1113,7 @@ __global__ void __launch_bounds__(256) k_emit_slots(const T* __restrict__ pos, i
                 }
                 wave_lds_fence();
                 const int64_t first = 3 * (off + first_k);
-                const int here = int(min(int64_t(3 * min(32, cnt - first_k)), 3 * capacity - first));
+                const int here = run_components(off + first_k, min(32, cnt - first_k), capacity);
 #pragma unroll
                 for (int x = l; x < 96; x += 32) {
                     if (x < here) {
