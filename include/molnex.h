@@ -347,7 +347,7 @@ int mnx_pme_gather_f64(const double* pos, const double* charges, const double* b
  * erfc(alpha r) / r, minus coulomb alpha / sqrt(pi) sum q^2 (pme_cpu.cpp:95-135,195-215).  The energy
  * is the sum of the mnx_pme_real_partials(n) doubles written to `partials`; dpos [n][3] and dq [n]
  * (both or neither) its derivatives.  *overflow (device) becomes non-zero when an atom has more than
- * 4096 neighbours; it is written only for more than 2048 atoms.  Workspace: mnx_nlist_workspace_bytes.
+ * 4096 neighbours of lower index (the half list's limit); it is written only for more than 2048 atoms.  Workspace: mnx_nlist_workspace_bytes.
  * convolve_add: mnx_pme_convolve whose energy also includes sum(more[0..nmore)), for a mesh spread with
  * `coulomb` (the rounding of its square root taken out of the energy); with mods64 the moduli
  * are doubles, else of the entry point's type.  gather_add:

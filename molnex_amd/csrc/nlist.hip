@@ -1334,15 +1334,18 @@ struct RealSink {
     RealArgs<T> a;
     double energy = 0.0;  // this lane's share over all centres
     double c1[kCentres], dq[kCentres], g[kCentres][3];
+    int lower[kCentres];  // neighbours of lower index: the half list's count, which is what is limited
 
     __device__ __forceinline__ void begin(int q, int i) {
         c1[q] = double(a.q[i]);
+        lower[q] = 0;
         dq[q] = g[q][0] = g[q][1] = g[q][2] = 0.0;
     }
     __device__ __forceinline__ void take(int q, int i, const int32_t* list, int count) {
         const int lane = threadIdx.x & (kWave - 1);
-        if (lane >= count) return;
         const int j = list[lane];
+        lower[q] += __popcll(__ballot(lane < count && j < i));
+        if (lane >= count) return;
         Geo<T> gg;
         const bool flip = i < j;
         pair_geo<T>(pos, box, flip ? j : i, flip ? i : j, box != nullptr, false, gg);
@@ -1361,13 +1364,13 @@ struct RealSink {
             for (int k = 0; k < 3; ++k) g[q][k] += f * double(gg.d[k]);
         }
     }
-    __device__ __forceinline__ void finish(int q, int i, const int32_t* list, int count, int held) {
+    __device__ __forceinline__ void finish(int q, int i, const int32_t* list, int, int held) {
         const int lane = threadIdx.x & (kWave - 1);
         take(q, i, list, held);
         const double self = a.coulomb * a.alpha * (0.5 * M_2_SQRTPI);
         if (lane == 0) {
             energy -= self * c1[q] * c1[q];
-            if (count > kNlCap) atomicExch(a.overflow, 1);
+            if (lower[q] > kNlCap) atomicExch(a.overflow, 1);
         }
         if (!a.dpos) return;
 #pragma unroll

@@ -111,6 +111,21 @@ def test_too_many_neighbours_is_refused():
         pme(pos, torch.zeros(4300, device=DEV), torch.eye(3, device=DEV) * 20.0)
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.float64, 1e-11), (torch.float32, 2e-5)])
+@pytest.mark.parametrize("box", [(30.0, 12.0, 12.0), (30.0, 8.0, 8.0)])  # the cell scan, an all-pairs grid
+def test_dense_sorted_systems_within_the_half_lists_limit(box, dtype, tol):
+    """Up to 6000 neighbours an atom, at most 3000 of lower index: the limit of 4096 is the half list's, so such
+    a system is taken (tolerances as above)."""
+    n, g = 12000, torch.Generator().manual_seed(1)
+    pos = 1.0 + 0.5 * torch.rand(n, 3, generator=g, dtype=torch.float64)
+    pos[:, 0] = 0.001 * torch.arange(n)
+    q = torch.randn(n, generator=g, dtype=torch.float64)
+    pos, q, box = (t.to(DEV, dtype) for t in (pos, q - q.mean(), torch.diag(torch.tensor(box, dtype=torch.float64))))
+    pme = PMEPotential(alpha=0.4, grid=(32, 32, 32), order=4, cutoff=3.0).to(DEV)
+    want = _composed(pme, pos, q, box)
+    _close(_run(pme, pos, q, box), want, tol, pme.coulomb * pme.alpha * float((q.double() ** 2).sum()))
+
+
 def test_opcheck():
     pos, q, box = _system(150, 12.0, 5)
     pme = PMEPotential(alpha=0.4, grid=(16, 16, 16), order=4, cutoff=3.5).to(DEV)
