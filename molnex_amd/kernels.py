@@ -1057,7 +1057,7 @@ def pme_energy(positions: Tensor, charges: Tensor, box_vectors: Tensor, xmoduli:
         many = torch.empty(4, dtype=torch.uint8, pin_memory=True)
         many.copy_(ws[8 * nparts:8 * nparts + 4], non_blocking=True)
         arrived = torch.cuda.Event()
-        arrived.record()
+        arrived.record(torch.cuda.current_stream(dev))  # the copy's; the current device may be another one
     grid = torch.empty((gridx, gridy, gridz), dtype=dt, device=dev)
     check(getattr(lib, f"mnx_pme_spread_{sfx}")(ptr(pos), ptr(q), ptr(b), n, gridx, gridy, gridz, order, float(coulomb),
                                                 ptr(grid), scratch, size, stream), "pme spread")

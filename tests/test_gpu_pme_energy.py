@@ -126,6 +126,26 @@ def test_dense_sorted_systems_within_the_half_lists_limit(box, dtype, tol):
     _close(_run(pme, pos, q, box), want, tol, pme.coulomb * pme.alpha * float((q.double() ** 2).sum()))
 
 
+def test_the_neighbour_flag_is_awaited_on_the_tensors_stream(monkeypatch):
+    """The flag's event is recorded on the stream of the positions' device, which need not be the current one."""
+    seen = []
+
+    class Event(torch.cuda.Event):
+        def record(self, stream=None):
+            seen.append(stream)
+            super().record(torch.cuda.current_stream() if stream is None else stream)
+
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    pos, q, box = _system(4200, 35.0, 2)
+    pme = PMEPotential(alpha=0.4, grid=(32, 32, 32), order=4, cutoff=4.0).to(DEV)
+    side = torch.cuda.Stream(pos.device)
+    side.wait_stream(torch.cuda.current_stream(pos.device))
+    with torch.cuda.stream(side):
+        pme(pos, q, box)
+    torch.cuda.synchronize()
+    assert seen == [side]
+
+
 def test_opcheck():
     pos, q, box = _system(150, 12.0, 5)
     pme = PMEPotential(alpha=0.4, grid=(16, 16, 16), order=4, cutoff=3.5).to(DEV)
