@@ -55,6 +55,7 @@ int mnx_abi_version(void);
 #define MNX_NLIST_TRIANGULAR 1 /* HALF only: pair (i, j) at slot i*(i-1)/2 + j
                                   (reference max_num_pairs == -1 layout) */
 #define MNX_NLIST_EXACT 2      /* COMPACT with capacity == total: nothing to pad */
+#define MNX_NLIST_MAX_NEIGHBORS 4096 /* of one atom, in the list asked for */
 
 size_t mnx_nlist_workspace_bytes(int64_t num_atoms);
 
@@ -347,7 +348,7 @@ int mnx_pme_gather_f64(const double* pos, const double* charges, const double* b
  * erfc(alpha r) / r, minus coulomb alpha / sqrt(pi) sum q^2 (pme_cpu.cpp:95-135,195-215).  The energy
  * is the sum of the mnx_pme_real_partials(n) doubles written to `partials`; dpos [n][3] and dq [n]
  * (both or neither) its derivatives.  *overflow (device) becomes non-zero when an atom has more than
- * 4096 neighbours of lower index (the half list's limit); it is written only for more than 2048 atoms.  Workspace: mnx_nlist_workspace_bytes.
+ * 4096 neighbours of lower index (the half list's limit), else zero.  Workspace: mnx_nlist_workspace_bytes.
  * convolve_add: mnx_pme_convolve whose energy also includes sum(more[0..nmore)), for a mesh spread with
  * `coulomb` (the rounding of its square root taken out of the energy); with mods64 the moduli
  * are doubles, else of the entry point's type.  gather_add:

@@ -55,7 +55,7 @@ namespace {
 
 constexpr int kNlSmall = 2048;  // atoms of the all-pairs path (its lists hold 16-bit ids; where both were
                                 // timed the cell list passes it at about this size)
-constexpr int kNlCap = 4096;   // max neighbours of one atom
+constexpr int kNlCap = MNX_NLIST_MAX_NEIGHBORS;  // of one atom
 constexpr int kSlots = 128;    // sorted neighbours kept per atom by the count pass
 constexpr int kMidCap = 1024;  // LDS list per wavefront of the emit for atoms with more
 constexpr int kCand = 512;     // candidates staged in LDS at once (394 on average at liquid density, cells of 5 A)
@@ -1432,6 +1432,7 @@ __global__ void __launch_bounds__(256) k_real_small(const T* __restrict__ pos, i
     const int wave = threadIdx.x >> 6;
     const int i = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * kParts + wave);
     RealSink<T> sink{pos, box, a};
+    if (blockIdx.x == 0 && threadIdx.x == 0) *a.overflow = 0;
     if (i < n) {
         const AcceptTest<T> at = accept_test<T>(box, box != nullptr, !wide_box<T>(box, double(cutoff)), cutoff);
         real_all_pairs<T>(pos, i, n, box, cutoff, at, lists[wave], sink);
@@ -1479,7 +1480,8 @@ int pme_real(const T* pos, const T* q, int64_t n, const T* box, double cutoff, d
     if (ws_bytes < need || !ws) return set_error(MNX_ERR_WORKSPACE, "workspace %zu < %zu bytes", ws_bytes, need);
     const RealArgs<T> a{q, alpha, coulomb, dpos, dq, partials, overflow};
     const unsigned blocks = unsigned(real_blocks(n));
-    if (n <= kNlSmall) {  // cannot exceed kNlCap neighbours
+    static_assert(kNlSmall <= kNlCap, "a small system cannot exceed the limit");
+    if (n <= kNlSmall) {
         hipLaunchKernelGGL((k_real_small<T>), dim3(blocks), dim3(256), 0, stream, pos, int(n), box, T(cutoff), a);
         MNX_CHECK_LAUNCH();
         return MNX_OK;

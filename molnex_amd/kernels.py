@@ -44,6 +44,7 @@ from .config import config as _settings
 
 MNX_NLIST_HALF, MNX_NLIST_FULL = 0, 1
 MNX_NLIST_COMPACT, MNX_NLIST_TRIANGULAR, MNX_NLIST_EXACT = 0, 1, 2
+MNX_NLIST_MAX_NEIGHBORS = 4096
 
 
 def _stream(t: Tensor) -> int:
@@ -65,6 +66,9 @@ def _ws(nbytes: int, device) -> Tensor:
 # ---------------------------------------------------------------------------
 
 
+_TOO_MANY = f"neighbor list: an atom has more than {MNX_NLIST_MAX_NEIGHBORS} neighbours within the cutoff"
+
+
 def _nlist_run(positions: Tensor, cutoff: float, box: Tensor | None, mode: int):
     """Stage 1 of the cell list; returns (workspace, total pair count on host)."""
     lib = _lib.load()
@@ -77,7 +81,7 @@ def _nlist_run(positions: Tensor, cutoff: float, box: Tensor | None, mode: int):
              _stream(positions)), "neighbor list count")
     t = int(total.item())
     if t < 0:
-        raise _lib.MolnexError("neighbor list: an atom has more than 4096 neighbours within the cutoff")
+        raise _lib.MolnexError(_TOO_MANY)
     return ws, t
 
 
@@ -1053,7 +1057,7 @@ def pme_energy(positions: Tensor, charges: Tensor, box_vectors: Tensor, xmoduli:
                                               ptr(dpos) if gradients else None, ptr(dq) if gradients else None, parts,
                                               flag, scratch, size, stream), "pme real-space sum")
     many = None
-    if n > 2048:  # the count of too many neighbours: read below, when it has long arrived
+    if n > MNX_NLIST_MAX_NEIGHBORS + 1:  # an atom may have more: read below, when it has long arrived
         many = torch.empty(4, dtype=torch.uint8, pin_memory=True)
         many.copy_(ws[8 * nparts:8 * nparts + 4], non_blocking=True)
         arrived = torch.cuda.Event()
@@ -1070,7 +1074,7 @@ def pme_energy(positions: Tensor, charges: Tensor, box_vectors: Tensor, xmoduli:
     if many is not None:
         arrived.synchronize()
         if int(many.view(torch.int32)[0]):
-            raise _lib.MolnexError("neighbor list: an atom has more than 4096 neighbours within the cutoff")
+            raise _lib.MolnexError(_TOO_MANY)
     return energy, spec, dpos, dq
 
 

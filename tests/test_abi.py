@@ -42,3 +42,10 @@ def test_host_only_queries():
     # error path: invalid config reports a message
     rc = lib.mnx_tp_fwd_f32(9999, 16, None, None, None, None, None, None, 1, 1, None, None)
     assert rc != 0 and b"invalid tp config" in lib.mnx_last_error()
+
+
+def test_neighbour_limit_is_one_value():
+    import molnex_amd.kernels as K
+
+    text = open(os.path.join(ROOT, "include", "molnex.h")).read()
+    assert int(re.search(r"#define MNX_NLIST_MAX_NEIGHBORS (\d+)", text).group(1)) == K.MNX_NLIST_MAX_NEIGHBORS

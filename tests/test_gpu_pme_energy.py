@@ -146,6 +146,20 @@ def test_the_neighbour_flag_is_awaited_on_the_tensors_stream(monkeypatch):
     assert seen == [side]
 
 
+@pytest.mark.parametrize("n", [1, 100, 2047, 2048, 2049])
+def test_the_neighbour_flag_is_always_written(n):
+    from molnex_amd import _lib
+
+    lib, ptr = _lib.load(), _lib.ptr
+    pos, q, box = _system(n, 28.0, 3)
+    parts = torch.zeros(lib.mnx_pme_real_partials(n), dtype=torch.float64, device=DEV)
+    flag = torch.full((1,), -1, dtype=torch.int32, device=DEV)
+    ws = torch.empty(lib.mnx_nlist_workspace_bytes(n), dtype=torch.uint8, device=DEV)
+    _lib.check(lib.mnx_pme_real_f64(ptr(pos), ptr(q), n, ptr(box), 4.0, 0.4, 1.0, None, None, ptr(parts), ptr(flag), ptr(ws),
+                                    ws.numel(), torch.cuda.current_stream().cuda_stream), "real")
+    assert flag.item() == 0
+
+
 def test_opcheck():
     pos, q, box = _system(150, 12.0, 5)
     pme = PMEPotential(alpha=0.4, grid=(16, 16, 16), order=4, cutoff=3.5).to(DEV)
