@@ -62,8 +62,10 @@ class PMEPotential(nn.Module):
                 and dt in (torch.float32, torch.float64) and charges.dtype == dt):
             # all three terms as one op each way, the real-space pairs never listed
             want = torch.is_grad_enabled() and (positions.requires_grad or charges.requires_grad)
-            return ops.pme_energy(positions, charges, box, self.xmoduli, self.ymoduli, self.zmoduli, *self.grid, self.order, self.alpha,
-                                  self.cutoff, self.coulomb, want)[0]
+            # (n, 1) as well as (n,)
+            q = charges.reshape(-1) if charges.dim() != 1 and charges.numel() == positions.shape[0] else charges
+            return ops.pme_energy(positions, q, box, self.xmoduli, self.ymoduli, self.zmoduli, *self.grid, self.order,
+                                  self.alpha, self.cutoff, self.coulomb, want)[0]
         if pairs is None:
             i, j, _, d, r = ops.neighbor_list(positions.detach(), self.cutoff, box.detach(), False)
             nb = torch.stack([i, j])

@@ -104,6 +104,18 @@ def test_single_gradients_scaling_and_no_grad():
     assert torch.equal(got[0], gp) and torch.equal(got[1], gq)
 
 
+@pytest.mark.parametrize("n", [1, 600])
+@pytest.mark.parametrize("shape", [(-1, 1), (1, -1)])
+def test_charges_in_a_column_or_a_row(n, shape):
+    pos, q, box = _system(n, 18.0, 1)
+    pme = PMEPotential(alpha=0.35, grid=(20, 20, 20), order=5, cutoff=4.5).to(DEV)
+    e, gp, gq = _run(pme, pos, q, box)
+    got = _run(pme, pos, q.reshape(shape), box)
+    assert torch.equal(got[0], e) and torch.equal(got[1], gp) and torch.equal(got[2], gq.reshape(shape))
+    with pytest.raises((ValueError, RuntimeError)):
+        pme(pos, torch.zeros(n + 1, device=DEV, dtype=pos.dtype), box)
+
+
 def test_too_many_neighbours_is_refused():
     pos = torch.rand(4300, 3, device=DEV) * 2.0
     pme = PMEPotential(alpha=0.3, grid=(16, 16, 16), order=4, cutoff=4.0).to(DEV)
