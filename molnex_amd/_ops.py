@@ -7,12 +7,14 @@ autograd kernel are registered directly, so a call passes through one Python fun
 ``custom_op`` also checks every result for aliasing with the arguments, at 16 us a call without and
 42 us with a gradient (9 and 18 us here; forward and backward of a small op 114 against 60 us), which
 is what bounds systems of a few thousand atoms.  The ops here return fresh tensors; one that writes
-into an argument stays a ``custom_op``.
+into an argument, or takes or returns a list of tensors (which an autograd function does not look
+into), stays a ``custom_op``.
 """
 
 from __future__ import annotations
 
 import inspect
+import re
 
 import torch
 
@@ -21,10 +23,7 @@ _lib = torch.library.Library("molix", "FRAGMENT")
 
 def _needs_grad(args) -> bool:
     for a in args:
-        if isinstance(a, torch.Tensor):
-            if a.requires_grad:
-                return True
-        elif isinstance(a, (list, tuple)) and any(isinstance(t, torch.Tensor) and t.requires_grad for t in a):
+        if isinstance(a, torch.Tensor) and a.requires_grad:
             return True
     return False
 
@@ -36,8 +35,10 @@ class Op:
         ns, name = qualname.split("::")
         if ns != "molix":
             raise ValueError(f"{qualname}: the namespace is molix")
-        _lib.define(name + (schema or torch.library.infer_schema(fn, mutates_args=())),
-                    tags=(torch.Tag.pt2_compliant_tag,))
+        schema = schema or torch.library.infer_schema(fn, mutates_args=())
+        if re.search(r"Tensor\??\[", schema):
+            raise TypeError(f"{qualname}{schema}: lists of tensors need torch.library.custom_op")
+        _lib.define(name + schema, tags=(torch.Tag.pt2_compliant_tag,))
         self.qualname, self.__doc__, self.__name__ = qualname, fn.__doc__, fn.__name__
         self._op = getattr(torch.ops.molix, name).default
         # a call through the dispatcher leaves out trailing arguments that have their default value

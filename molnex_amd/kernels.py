@@ -2835,7 +2835,7 @@ def _ptr_array(ts) -> C.c_void_p:
     return C.cast((C.c_void_p * len(ts))(*[t.data_ptr() for t in ts]), C.c_void_p)
 
 
-@_op("molix::channel_outer_stack")
+@torch.library.custom_op("molix::channel_outer_stack", mutates_args=(), device_types="cuda")
 def channel_outer_stack(y: Tensor, s: list[Tensor]) -> Tensor:
     """``stack([y * s_l for s_l in s], 1)`` for a per-edge factor ``y`` (E rows of one entry) and
     L (E, F) inputs, (E, L, F) in one pass: the cutoff envelope on Allegro's per-layer scalar
@@ -2854,7 +2854,7 @@ def _(y, s):
     return y.new_empty(s[0].shape[0], len(s), s[0].shape[1])
 
 
-@_op("molix::channel_outer_stack_backward")
+@torch.library.custom_op("molix::channel_outer_stack_backward", mutates_args=(), device_types="cuda")
 def channel_outer_stack_backward(grad: Tensor, y: Tensor, s: list[Tensor], need_y: bool,
                                  need_s: bool) -> list[Tensor]:
     """``[grad y, grad s_0, ..., grad s_{L-1}]`` of ``channel_outer_stack`` in one pass: grad y

@@ -257,6 +257,19 @@ def test_envelope_stack_opcheck_and_errors():
         K.channel_outer_stack(u, [xs[0], xs[1][:36]])
 
 
+def test_channel_outer_stack_does_not_lose_the_lists_gradients():
+    """The op has no autograd formula of its own: a gradient to its list of inputs is refused, not left out."""
+    u = torch.rand(5, 1, device=DEV)
+    xs = [torch.randn(5, 16, device=DEV) for _ in range(2)]
+    xs[1].requires_grad_(True)
+    out = torch.ops.molix.channel_outer_stack(u, xs)
+    assert out.requires_grad
+    with pytest.raises(RuntimeError, match="no autograd formula"):
+        torch.autograd.grad(out.sum(), xs[1])
+    for t in torch.ops.molix.channel_outer_stack_backward(out.detach(), u, xs, True, True):
+        assert t.requires_grad
+
+
 def test_allegro_rotation_invariant_and_contract():
     """Scalar edge features are invariant under a rotation of the positions (the reference checks
     rtol = atol = 1e-4; fp32 here stays far inside), and the GraphBatch contract writes

@@ -68,3 +68,23 @@ def test_hooks_vmap_tracing_and_opcheck():
     f = torch.compile(lambda a: scaled(a, Y)[0].sin(), backend="aot_eager", fullgraph=True)
     assert torch.allclose(torch.autograd.grad(f(x).sum(), x)[0], torch.cos(2 * X * Y) * 2 * Y)
     torch.library.opcheck(torch.ops.molix._test_scaled.default, (x, Y, 3))
+
+
+def test_lists_of_tensors_are_left_to_custom_op():
+    """An autograd function does not look into lists: such an op's gradients would be lost in silence."""
+
+    def takes(y: torch.Tensor, s: list[torch.Tensor]) -> torch.Tensor:
+        return y * s[0]
+
+    def gives(y: torch.Tensor) -> list[torch.Tensor]:
+        return [y + 1]
+
+    for fn in (takes, gives):
+        with pytest.raises(TypeError, match="custom_op"):
+            _ops.op(f"molix::_test_{fn.__name__}")(fn)
+    with pytest.raises(TypeError, match="custom_op"):
+        _ops.op("molix::_test_optional", schema="(Tensor y, Tensor?[] s) -> Tensor")(takes)
+    import molnex_amd.kernels as K
+
+    assert not any("Tensor[" in str(op._schema) or "Tensor?[" in str(op._schema)
+                   for op in (v._op for v in vars(K).values() if isinstance(v, _ops.Op)))
