@@ -19,6 +19,9 @@ import re
 import torch
 
 _lib = torch.library.Library("molix", "FRAGMENT")
+# Each op's own Library, kept across a reload of this module: defining an op again (importlib.reload,
+# a notebook's autoreload) replaces it, as with ``custom_op``
+_libs: dict[str, torch.library.Library] = globals().get("_libs", {})
 
 
 def _needs_grad(args) -> bool:
@@ -38,21 +41,24 @@ class Op:
         schema = schema or torch.library.infer_schema(fn, mutates_args=())
         if re.search(r"Tensor\??\[", schema):
             raise TypeError(f"{qualname}{schema}: lists of tensors need torch.library.custom_op")
-        _lib.define(name + schema, tags=(torch.Tag.pt2_compliant_tag,))
+        if name in _libs:
+            _libs.pop(name)._destroy()
+        self._lib = _libs[name] = torch.library.Library("molix", "FRAGMENT")
+        self._lib.define(name + schema, tags=(torch.Tag.pt2_compliant_tag,))
         self.qualname, self.__doc__, self.__name__ = qualname, fn.__doc__, fn.__name__
         self._op = getattr(torch.ops.molix, name).default
         # a call through the dispatcher leaves out trailing arguments that have their default value
         self._defaults = tuple(p.default for p in inspect.signature(fn).parameters.values())
         self._setup = self._backward = None
         self._function = self._make_function()
-        _lib.impl(name, fn, "CUDA")
-        _lib.impl(name, self._autograd, "Autograd")
+        self._lib.impl(name, fn, "CUDA")
+        self._lib.impl(name, self._autograd, "Autograd")
 
     def __call__(self, *args, **kwargs):
         return self._op(*args, **kwargs)
 
     def register_fake(self, fn):
-        torch.library.register_fake(self.qualname, fn, lib=_lib)
+        torch.library.register_fake(self.qualname, fn, lib=self._lib)
         return fn
 
     def register_autograd(self, backward, *, setup_context=None) -> None:

@@ -1,6 +1,10 @@
 """molnex_amd._ops: what the registration of an op gives its callers (on the CPU, with a stand-in kernel),
 as torch.library.custom_op gives it."""
 
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -88,3 +92,32 @@ def test_lists_of_tensors_are_left_to_custom_op():
 
     assert not any("Tensor[" in str(op._schema) or "Tensor?[" in str(op._schema)
                    for op in (v._op for v in vars(K).values() if isinstance(v, _ops.Op)))
+
+
+def test_an_op_defined_again_replaces_the_first():
+    """A module of ops can be reloaded (a notebook's autoreload)."""
+    def first(x: torch.Tensor) -> torch.Tensor:
+        return x + 1
+
+    def second(x: torch.Tensor, k: int) -> torch.Tensor:
+        return x + k
+
+    for fn, args, want in ((first, (), 1), (second, (5,), 5)):
+        op = _ops.op("molix::_test_again")(fn)
+        op._lib.impl("_test_again", fn, "CPU")
+        op.register_fake(lambda x, *a: torch.empty_like(x))
+        op.register_autograd(lambda ctx, g, n=len(args): (g, None)[:1 + n])
+        x = X.clone().requires_grad_(True)
+        out = torch.ops.molix._test_again(x, *args)
+        assert torch.equal(out, X + want) and torch.equal(torch.autograd.grad(out.sum(), x)[0], torch.ones(3))
+        f = torch.compile(lambda a, rest=args: torch.ops.molix._test_again(a, *rest).sin(), backend="aot_eager", fullgraph=True)
+        assert torch.allclose(f(x), torch.sin(X + want))
+
+
+def test_the_kernels_module_can_be_reloaded():
+    code = ("import importlib, torch, molnex_amd._ops as O, molnex_amd.kernels as K\n"
+            "old = K.tall_tn\n"
+            "for m in (K, O, K):\n"
+            "    importlib.reload(m)\n"
+            "assert K.tall_tn is not old and torch.ops.molix.tall_tn.default is K.tall_tn._op\n")
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=240, cwd=os.path.dirname(os.path.dirname(_ops.__file__)))
