@@ -499,7 +499,8 @@ int mnx_linear_blocks_f32(const float* a, int64_t a_stride, int64_t R, const flo
 /*       x[n*x_stride + xcol + i*xcomp + c] * g[n*g_stride + gcol + i*gcomp + p] */
 /* for c < M, p < N (overwritten; R = 0 gives zeros).  desc holds 8 integers  */
 /* per pair (xcol, xcomp, M, gcol, gcomp, N, d, wo), scale one factor per     */
-/* pair; both are host memory.  fp32-accurate products (three-way bf16 splits), */
+/* pair; both are host memory.  fp32-accurate products (three-way bf16 splits; */
+/* fp32 products where an entry is not finite or above 3.39e38, bf16's largest), */
 /* summed in a fixed order (deterministic).  Widths, columns, component steps  */
 /* and row strides even; x and g 8-byte aligned.                              */
 /* ------------------------------------------------------------------------ */

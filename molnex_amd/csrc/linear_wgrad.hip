@@ -185,6 +185,36 @@ __global__ void __launch_bounds__(kWgThreads) k_linear_wgrad(WgArgs p, const flo
         split(a, b, pl);
         products(pl);
     }
+    // The parts of a value that bf16 cannot hold (infinite, or above its largest, 3.39e38) are not
+    // finite, and their products are NaN: such a tile is formed again by fp32 products, whose infinities
+    // and finite results are those of the sum.  The test is once per slab (a linear of 20k nodes, 128
+    // channels, with its gradients: 659.2 us without, 660.6 with; runs differ by 0.6 %).
+    float odd = 0.f;
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int j = 0; j < T; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) odd = fmaf(acc[i][j][r], 0.f, odd);  // 0, or NaN of any infinity or NaN
+    if (__ballot(odd != 0.f)) {
+#pragma unroll
+        for (int i = 0; i < T; ++i)
+#pragma unroll
+            for (int j = 0; j < T; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        comp = oa = og = 0;
+        for (int r = 0; r < H; r += 8) {
+            load(kTail, r, a, b);
+#pragma unroll
+            for (int z = 0; z < 8; ++z)
+#pragma unroll
+                for (int i = 0; i < T; ++i)
+#pragma unroll
+                    for (int j = 0; j < T; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][z], b[j][z], acc[i][j], 0, 0, 0);
+        }
+    }
     float* dst = part + int64_t(unit) * (1024 * T * T) + lane;
 #pragma unroll
     for (int i = 0; i < T; ++i)
