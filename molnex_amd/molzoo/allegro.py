@@ -128,10 +128,17 @@ def _envelope_stack(per_layer, u):
     return _times_envelope(stacked.reshape(stacked.shape[0], -1), u).reshape(stacked.shape)
 
 
+def _plain(*modules: nn.Module) -> bool:
+    """Whether a call of each module is its class's forward and nothing more (no hooks, no forward of its own)."""
+    return not nn.modules.module._has_any_global_hook() and not any(
+        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__
+        for m in modules)
+
+
 def _pair_features(rbf, cutoff_fn, emb: nn.Embedding, r: torch.Tensor, zs: torch.Tensor, zd: torch.Tensor):
     """``(cat([rbf(r) * cutoff_fn(r), emb(zs), emb(zd)], -1), cutoff_fn(r))``: one kernel each way
-    (``molix::pair_features``) for a Bessel basis and a cosine or polynomial cutoff of one radius on
-    (E,) float32 GPU distances with the embedding frozen, else the modules."""
+    (``molix::pair_features``) for a Bessel basis and a cosine or polynomial cutoff of one radius, neither
+    with hooks, on (E,) float32 GPU distances with the embedding frozen, else the modules."""
     w = emb.weight
     kind = 1 if type(cutoff_fn) is CosineCutoff else 2 if type(cutoff_fn) is PolynomialCutoff else 0
     if (kind and type(rbf) is BesselRBF and r.is_cuda and r.dtype == torch.float32 and r.dim() == 1
@@ -139,7 +146,7 @@ def _pair_features(rbf, cutoff_fn, emb: nn.Embedding, r: torch.Tensor, zs: torch
             and (kind == 1 or cutoff_fn.exponent <= 64) and zs.shape == zd.shape == r.shape
             and w.dtype == torch.float32 and not (torch.is_grad_enabled() and w.requires_grad)
             and emb.padding_idx is None and emb.max_norm is None and w.shape[1] <= 4096
-            and not zs.is_floating_point()):
+            and not zs.is_floating_point() and _plain(rbf, cutoff_fn)):
         mu, sigma = (rbf.mu, rbf.sigma) if rbf.normalize else (None, None)
         return K.pair_features(r, zs.long(), zd.long(), w, int(rbf.config.num_radial), rbf.r_cut, rbf.eps, mu, sigma,
                                kind, cutoff_fn.exponent if kind == 2 else 0)

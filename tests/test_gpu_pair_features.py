@@ -64,3 +64,45 @@ def test_type_outside_the_table_and_no_edges():
     e = torch.empty(0, dtype=torch.int64, device=DEV)
     out, u = K.pair_features(torch.empty(0, device=DEV), e, e, table, 4, RC, 1e-8, None, None, 2, 6)
     assert out.shape == (0, 12) and u.shape == (0,)
+
+
+@pytest.mark.parametrize("kind", ["forward", "pre", "backward", "global", "own"])
+def test_hooks_of_the_basis_and_the_cutoff_run(kind):
+    """The embedding calls its modules where a hook (or a forward of the instance's own) waits on them."""
+    from molnex_amd.molzoo.allegro import PairEmbedding
+
+    torch.manual_seed(0)
+    emb = PairEmbedding(num_elements=4, num_scalar_features=16, num_tensor_features=16, r_max=RC, l_max=1).to(DEV)
+    for p in emb.parameters():
+        p.requires_grad_(False)
+    mods = (emb.radial_basis, emb.cutoff_fn)
+    ei, d = torch.randint(0, 10, (70, 2), device=DEV), torch.randn(70, 3, device=DEV)
+    z, r = torch.randint(0, 4, (10,), device=DEV), d.norm(dim=-1).requires_grad_(True)
+    plain = emb(z, r, d, ei)
+    seen = []
+
+    def note(m, *_):
+        if m in mods:
+            seen.append(m)
+
+    handles = []
+    if kind == "global":
+        handles.append(torch.nn.modules.module.register_module_forward_hook(note))
+    for m in mods:
+        if kind == "forward":
+            handles.append(m.register_forward_hook(note))
+        elif kind == "pre":
+            handles.append(m.register_forward_pre_hook(note))
+        elif kind == "backward":
+            handles.append(m.register_full_backward_hook(note))
+        elif kind == "own":
+            m.forward = lambda r, m=m, f=m.forward: (note(m), f(r))[1]
+    try:
+        out = emb(z, r, d, ei)
+        torch.autograd.grad(sum(t.sum() for t in out), r)
+    finally:
+        for h in handles:
+            h.remove()
+    assert set(seen) == set(mods)
+    for a, b in zip(out, plain):
+        _close(a, b.cpu())
