@@ -19,8 +19,8 @@
 //
 // Above that, a cell list.  Atoms are binned into cells whose slab widths exceed
 // the cutoff (fractional coordinates for periodic cells); a cell's atoms take a
-// run of the cell-ordered arrays in whatever order they arrive (nothing that is
-// written depends on it).  A workgroup takes a cell: its four wavefronts stage the
+// run of the cell-ordered arrays in whatever order they arrive (no list depends
+// on it; the real-space sum below, whose last bits would, takes them by id).  A workgroup takes a cell: its four wavefronts stage the
 // atoms of the 27 neighbour cells in LDS (wrapped next to the cell), then each
 // tests them against every fourth atom of the cell as a centre, whose position is
 // wave-uniform (a screening distance on positions moved into the primary cell, the
@@ -95,6 +95,7 @@ struct NlWs {
     int32_t* atoms_sorted;
     int32_t* counts;
     int32_t* big;
+    int32_t* ids;     // the real-space sum's: each cell's atoms in order of arrival
     int32_t* slots;   // [n][kSlots]: an atom's neighbours, ascending
     uint64_t* masks;  // small systems: [n][words] accept ballots
     void* posw;       // PosW<T> per cell-ordered slot
@@ -120,7 +121,7 @@ NlWs carve(void* base, size_t bytes, int64_t n, size_t* used) {
         w.cell_count = ws.take<int32_t>(w.max_cells);
         w.cell_start = ws.take<int32_t>(w.max_cells);
         w.atoms_sorted = ws.take<int32_t>(n);
-        w.big = ws.take<int32_t>(n);
+        w.big = w.ids = ws.take<int32_t>(n);
         w.slots = ws.take<int32_t>(size_t(n) * kSlots);
         w.posw = ws.take<PosW<double>>(n);
         w.tiles64 = ws.take<int64_t>(scan_workspace_elems(n));
@@ -469,17 +470,39 @@ __global__ void __launch_bounds__(kScanThreads) k_cell_runs(NlGrid* __restrict__
     }
 }
 
-// Each atom into its slot of the cell order, with its position moved into the primary cell (by
-// whole box vectors, from the fractional coordinates that binned it), which the count pass's
-// screening test reads.
-template <typename T>
-__global__ void k_place(int64_t n, const T* __restrict__ pos, const T* __restrict__ box,
-                        const NlGrid* __restrict__ gp, const int32_t* __restrict__ cell_of,
-                        const int32_t* __restrict__ rank, const int32_t* __restrict__ cell_start,
-                        int32_t* __restrict__ atoms_sorted, PosW<T>* __restrict__ posw) {
+// The slots of each cell's atoms in order of arrival, their ids alone.
+__global__ void __launch_bounds__(256) k_place_ids(int64_t n, const NlGrid* __restrict__ gp,
+                                                   const int32_t* __restrict__ cell_of,
+                                                   const int32_t* __restrict__ rank,
+                                                   const int32_t* __restrict__ cell_start, int32_t* __restrict__ ids) {
     const int64_t a = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (a >= n || gp->brute) return;
-    const int slot = cell_start[cell_of[a]] + rank[a];
+    ids[cell_start[cell_of[a]] + rank[a]] = int32_t(a);
+}
+
+// Each atom into its slot of the cell order, with its position moved into the primary cell (by
+// whole box vectors, from the fractional coordinates that binned it), which the count pass's
+// screening test reads.  Within a cell the atoms take their slots as they arrived (rank) or, ORDERED,
+// by id: a thread per slot of `ids` counts the smaller ids of its cell.
+template <typename T, bool ORDERED>
+__global__ void __launch_bounds__(256) k_place(int64_t n, const T* __restrict__ pos, const T* __restrict__ box,
+                                               const NlGrid* __restrict__ gp, const int32_t* __restrict__ cell_of,
+                                               const int32_t* __restrict__ rank,
+                                               const int32_t* __restrict__ cell_start,
+                                               const int32_t* __restrict__ cell_count, const int32_t* __restrict__ ids,
+                                               int32_t* __restrict__ atoms_sorted, PosW<T>* __restrict__ posw) {
+    const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (t >= n || gp->brute) return;
+    const int64_t a = ORDERED ? ids[t] : t;
+    const int c = cell_of[a], first = cell_start[c];
+    int r = 0;
+    if (ORDERED) {
+        const int m = cell_count[c];
+        for (int k = 0; k < m; ++k) r += ids[first + k] < a;
+    } else {
+        r = rank[a];
+    }
+    const int slot = first + r;
     atoms_sorted[slot] = int32_t(a);
     const double x = pos[3 * a], y = pos[3 * a + 1], z = pos[3 * a + 2];
     PosW<T> p;
@@ -1180,8 +1203,9 @@ __global__ void __launch_bounds__(kScanThreads) k_nl_offsets(const int32_t* __re
     }
 }
 
-// Cell grid and cell-ordered atoms of a system of more than kNlSmall atoms.
-template <typename T>
+// Cell grid and cell-ordered atoms of a system of more than kNlSmall atoms; ORDERED: by id within a
+// cell (w.ids), for a scan that sums in the order of its candidates.
+template <typename T, bool ORDERED>
 int bin_atoms(const T* pos, int64_t n, double cutoff, const T* box, const NlWs& w, hipStream_t stream,
               int32_t* flag = nullptr) {
     const int tb = 256;
@@ -1203,8 +1227,14 @@ int bin_atoms(const T* pos, int64_t n, double cutoff, const T* box, const NlWs& 
     hipLaunchKernelGGL(k_cell_runs, dim3(ceil_div(w.max_cells, kScanTile)), dim3(kScanThreads), 0, stream, w.grid,
                        w.cell_count, w.cell_start);
     MNX_CHECK_LAUNCH();
-    hipLaunchKernelGGL((k_place<T>), dim3(ceil_div(n, tb)), dim3(tb), 0, stream, n, pos, box, w.grid, w.cell_of, w.rank,
-                       w.cell_start, w.atoms_sorted, static_cast<PosW<T>*>(w.posw));
+    if (ORDERED) {
+        hipLaunchKernelGGL(k_place_ids, dim3(ceil_div(n, tb)), dim3(tb), 0, stream, n, w.grid, w.cell_of, w.rank,
+                           w.cell_start, w.ids);
+        MNX_CHECK_LAUNCH();
+    }
+    hipLaunchKernelGGL((k_place<T, ORDERED>), dim3(ceil_div(n, tb)), dim3(tb), 0, stream, n, pos, box, w.grid,
+                       w.cell_of, w.rank, w.cell_start, w.cell_count, w.ids, w.atoms_sorted,
+                       static_cast<PosW<T>*>(w.posw));
     MNX_CHECK_LAUNCH();
     return MNX_OK;
 }
@@ -1231,7 +1261,7 @@ int nlist_count(const T* pos, int64_t n, double cutoff, const T* box, int mode, 
         MNX_CHECK_LAUNCH();
         return MNX_OK;
     }
-    int rc = bin_atoms<T>(pos, n, cutoff, box, w, stream);
+    int rc = bin_atoms<T, false>(pos, n, cutoff, box, w, stream);
     if (rc) return rc;
     const PosW<T>* posw = static_cast<const PosW<T>*>(w.posw);
     const unsigned blocks = unsigned(std::min<int64_t>(w.max_cells, kNlBlocks));
@@ -1313,6 +1343,8 @@ __global__ void k_nl_backward(const int32_t* __restrict__ ii, const int32_t* __r
 // once -- no pair list in memory, no atomics and no read of a pair count on the host.
 // The pairs and their geometry are the neighbor list's, bit for bit; their terms are
 // evaluated and summed in fp64 whatever the storage type.
+// The cells' atoms are ordered by id, so the sums have a fixed order and the results the same bits every time
+// (one launch and 5 to 10 us of a 420 us term at 50k atoms; by arrival, 4 energies in 8 float64 runs).
 // Measured, 50k atoms (1.3 M pairs): 123 us and six launches, bound by the fp64 erfc and exp of both
 // ends; the list (150 us), the energy over it (12) and its derivatives with scattered atomics (147)
 // took over 300 us and 30 launches.
@@ -1486,7 +1518,7 @@ int pme_real(const T* pos, const T* q, int64_t n, const T* box, double cutoff, d
         MNX_CHECK_LAUNCH();
         return MNX_OK;
     }
-    int rc = bin_atoms<T>(pos, n, cutoff, box, w, stream, overflow);
+    int rc = bin_atoms<T, true>(pos, n, cutoff, box, w, stream, overflow);
     if (rc) return rc;
     hipLaunchKernelGGL((k_real_cells<T>), dim3(blocks), dim3(256), 0, stream, pos, n, box, T(cutoff), w.grid,
                        w.cell_start, w.cell_count, w.atoms_sorted, static_cast<const PosW<T>*>(w.posw), a);

@@ -85,6 +85,17 @@ def test_energy_and_gradients(n, edge, cut, mesh, order, kind, dtype, tol):
         _close(again, [t.double() for t in got], tol)
 
 
+@pytest.mark.parametrize("n,edge,cut", [(2049, 27.0, 4.0), (9000, 45.0, 5.0), (6000, 45.0, 14.9)])
+def test_the_same_bits_every_time(n, edge, cut):
+    """The cell scan sums in a fixed order: energy and gradients are reproducible in float64.  (The last size has
+    27 cells of 220 atoms.)"""
+    pos, q, box = _system(n, edge, 11)
+    pme = PMEPotential(alpha=0.4, grid=(32, 32, 32), order=4, cutoff=cut).to(DEV)
+    first = _run(pme, pos, q, box)
+    for _ in range(7):
+        assert all(torch.equal(a, b) for a, b in zip(_run(pme, pos, q, box), first))
+
+
 def test_single_gradients_scaling_and_no_grad():
     pos, q, box = (t.float() for t in _system(600, 18.0, 1))
     pme = PMEPotential(alpha=0.35, grid=(20, 20, 20), order=5, cutoff=4.5).to(DEV)
