@@ -348,12 +348,13 @@ int mnx_pme_gather_f64(const double* pos, const double* charges, const double* b
  * erfc(alpha r) / r, minus coulomb alpha / sqrt(pi) sum q^2 (pme_cpu.cpp:95-135,195-215).  The energy
  * is the sum of the mnx_pme_real_partials(n) doubles written to `partials`; dpos [n][3] and dq [n]
  * (both or neither) its derivatives.  *overflow (device) becomes non-zero when an atom has more than
- * 4096 neighbours of lower index (the half list's limit), else zero.  Workspace: mnx_nlist_workspace_bytes.
+ * 4096 neighbours of lower index (the half list's limit), else zero.
  * convolve_add: mnx_pme_convolve whose energy also includes sum(more[0..nmore)), for a mesh spread with
  * `coulomb` (the rounding of its square root taken out of the energy); with mods64 the moduli
  * are doubles, else of the entry point's type.  gather_add:
  * mnx_pme_gather whose derivatives are (reciprocal + dpos_add / dq_add) * *grad, where these device
  * pointers are not NULL. */
+size_t mnx_pme_real_workspace_bytes(int64_t num_atoms, int32_t f64);
 int64_t mnx_pme_real_partials(int64_t num_atoms);
 int mnx_pme_convolve_add_f32(float* cgrid, const float* box, int32_t gx, int32_t gy, int32_t gz, double alpha,
                              const void* xm, const void* ym, const void* zm, int32_t mods64, double coulomb,

@@ -72,6 +72,7 @@ SIGNATURES = {
     "mnx_pme_convolve_f64": (C.c_int, [vp, vp, c_i32, c_i32, c_i32, c_f64, vp, vp, vp, vp, vp, c_sz, vp]),
     "mnx_pme_gather_f32": (C.c_int, [vp, vp, vp, c_i64, vp, c_i32, c_i32, c_i32, c_i32, c_f64, vp, vp, vp]),
     "mnx_pme_gather_f64": (C.c_int, [vp, vp, vp, c_i64, vp, c_i32, c_i32, c_i32, c_i32, c_f64, vp, vp, vp]),
+    "mnx_pme_real_workspace_bytes": (c_sz, [c_i64, c_i32]),
     "mnx_pme_real_partials": (c_i64, [c_i64]),
     "mnx_pme_real_f32": (C.c_int, [vp, vp, c_i64, vp, c_f64, c_f64, c_f64, vp, vp, vp, vp, vp, c_sz, vp]),
     "mnx_pme_convolve_add_f32": (C.c_int, [vp, vp, c_i32, c_i32, c_i32, c_f64, vp, vp, vp, c_i32, c_f64, vp, c_i64, vp, vp,

@@ -106,25 +106,43 @@ struct NlWs {
 
 int64_t max_cells_for(int64_t n) { return 2 * n + 64; }
 
+// The cell grid and the atoms in cell order.
+void take_cells(Workspace& ws, int64_t n, size_t posw_bytes, NlWs& w) {
+    w.max_cells = max_cells_for(n);
+    w.grid = ws.take<NlGrid>(1);
+    w.cell_of = ws.take<int32_t>(n);
+    w.rank = ws.take<int32_t>(n);
+    w.cell_count = ws.take<int32_t>(w.max_cells);
+    w.cell_start = ws.take<int32_t>(w.max_cells);
+    w.atoms_sorted = ws.take<int32_t>(n);
+    w.posw = ws.take<char>(size_t(n) * posw_bytes);
+}
+
 NlWs carve(void* base, size_t bytes, int64_t n, size_t* used) {
     Workspace ws{static_cast<char*>(base), bytes};
     NlWs w{};
-    w.max_cells = max_cells_for(n);
     w.offsets = ws.take<int64_t>(n + 1);
     w.counts = ws.take<int32_t>(n > 0 ? n : 1);
     if (n <= kNlSmall) {
         w.masks = ws.take<uint64_t>(size_t(n > 0 ? n : 1) * ((n + kWave - 1) / kWave + 1));
     } else {
-        w.grid = ws.take<NlGrid>(1);
-        w.cell_of = ws.take<int32_t>(n);
-        w.rank = ws.take<int32_t>(n);
-        w.cell_count = ws.take<int32_t>(w.max_cells);
-        w.cell_start = ws.take<int32_t>(w.max_cells);
-        w.atoms_sorted = ws.take<int32_t>(n);
-        w.big = w.ids = ws.take<int32_t>(n);
+        take_cells(ws, n, sizeof(PosW<double>), w);
+        w.big = ws.take<int32_t>(n);
         w.slots = ws.take<int32_t>(size_t(n) * kSlots);
-        w.posw = ws.take<PosW<double>>(n);
         w.tiles64 = ws.take<int64_t>(scan_workspace_elems(n));
+    }
+    *used = ws.used;
+    return w;
+}
+
+// What the real-space sum needs of it: no rows, counts or offsets (48 bytes an atom, 64 in float64, instead
+// of 588), and nothing for small systems.
+NlWs carve_real(void* base, size_t bytes, int64_t n, size_t posw_bytes, size_t* used) {
+    Workspace ws{static_cast<char*>(base), bytes};
+    NlWs w{};
+    if (n > kNlSmall) {
+        take_cells(ws, n, posw_bytes, w);
+        w.ids = ws.take<int32_t>(n);
     }
     *used = ws.used;
     return w;
@@ -1508,8 +1526,9 @@ int pme_real(const T* pos, const T* q, int64_t n, const T* box, double cutoff, d
     MNX_REQUIRE(pos && q && box && partials && overflow, "null pointer argument");
     MNX_REQUIRE((dpos == nullptr) == (dq == nullptr), "dpos and dq must both be given or both be null");
     size_t need = 0;
-    NlWs w = carve(ws, ws_bytes, n, &need);
-    if (ws_bytes < need || !ws) return set_error(MNX_ERR_WORKSPACE, "workspace %zu < %zu bytes", ws_bytes, need);
+    NlWs w = carve_real(ws, ws_bytes, n, sizeof(PosW<T>), &need);
+    if (need && (ws_bytes < need || !ws))
+        return set_error(MNX_ERR_WORKSPACE, "workspace %zu < %zu bytes", ws_bytes, need);
     const RealArgs<T> a{q, alpha, coulomb, dpos, dq, partials, overflow};
     const unsigned blocks = unsigned(real_blocks(n));
     static_assert(kNlSmall <= kNlCap, "a small system cannot exceed the limit");
@@ -1586,6 +1605,11 @@ int mnx_nlist_backward_f64(const int32_t* idx_i, const int32_t* idx_j, const dou
     return MNX_OK;
 }
 
+size_t mnx_pme_real_workspace_bytes(int64_t num_atoms, int32_t f64) {
+    size_t used = 0;
+    carve_real(nullptr, 0, num_atoms, f64 ? sizeof(PosW<double>) : sizeof(PosW<float>), &used);
+    return used + 256;
+}
 int64_t mnx_pme_real_partials(int64_t num_atoms) { return num_atoms > 0 ? real_blocks(num_atoms) : 0; }
 
 int mnx_pme_real_f32(const float* pos, const float* q, int64_t n, const float* box, double cutoff, double alpha,

@@ -1048,7 +1048,8 @@ def pme_energy(positions: Tensor, charges: Tensor, box_vectors: Tensor, xmoduli:
     # scratch of the three stages in turn, behind the energy's partial sums and the neighbour flag
     nparts = lib.mnx_pme_real_partials(n)
     head = (8 * nparts + 8 + 255) // 256 * 256
-    ws = _ws(head + max(lib.mnx_nlist_workspace_bytes(n), lib.mnx_pme_spread_workspace_bytes(n, gridx, gridy, gridz),
+    ws = _ws(head + max(lib.mnx_pme_real_workspace_bytes(n, sfx == "f64"),
+                        lib.mnx_pme_spread_workspace_bytes(n, gridx, gridy, gridz),
                         lib.mnx_pme_convolve_workspace_bytes(gridx, gridy, gridz)), dev)
     parts, flag, scratch, size = ptr(ws), ptr(ws) + 8 * nparts, ptr(ws) + head, ws.numel() - head
     dpos = torch.empty_like(pos) if gradients else pos.new_empty((0, 3))
@@ -1104,7 +1105,7 @@ def pme_energy_backward(grad: Tensor, positions: Tensor, charges: Tensor, box_ve
     if dpos.shape[0] != n:  # the forward was told that no gradient is wanted
         dpos, dq = torch.empty_like(pos), torch.empty_like(q)
         parts = torch.empty(lib.mnx_pme_real_partials(n) + 1, dtype=torch.float64, device=dev)
-        ws = _ws(lib.mnx_nlist_workspace_bytes(n), dev)
+        ws = _ws(lib.mnx_pme_real_workspace_bytes(n, sfx == "f64"), dev)
         check(getattr(lib, f"mnx_pme_real_{sfx}")(ptr(pos), ptr(q), n, ptr(b), float(cutoff), float(alpha),
                                                   float(coulomb), ptr(dpos), ptr(dq), ptr(parts),
                                                   ptr(parts) + 8 * (parts.numel() - 1), ptr(ws), ws.numel(),

@@ -49,3 +49,10 @@ def test_neighbour_limit_is_one_value():
 
     text = open(os.path.join(ROOT, "include", "molnex.h")).read()
     assert int(re.search(r"#define MNX_NLIST_MAX_NEIGHBORS (\d+)", text).group(1)) == K.MNX_NLIST_MAX_NEIGHBORS
+
+
+def test_the_real_space_sum_takes_no_neighbour_rows():
+    lib = _lib.load()
+    for n in (1, 2048, 2049, 1_000_000):
+        for f64 in (0, 1):
+            assert lib.mnx_pme_real_workspace_bytes(n, f64) <= (64 if f64 else 48) * n + 4096

@@ -169,18 +169,24 @@ def test_the_neighbour_flag_is_awaited_on_the_tensors_stream(monkeypatch):
     assert seen == [side]
 
 
-@pytest.mark.parametrize("n", [1, 100, 2047, 2048, 2049])
-def test_the_neighbour_flag_is_always_written(n):
+@pytest.mark.parametrize("sfx", ["f32", "f64"])
+@pytest.mark.parametrize("n", [1, 100, 2047, 2048, 2049, 5003])
+def test_the_neighbour_flag_and_the_workspace(n, sfx):
+    """The flag is always written, and nothing behind the workspace that was asked for."""
     from molnex_amd import _lib
 
     lib, ptr = _lib.load(), _lib.ptr
-    pos, q, box = _system(n, 28.0, 3)
+    pos, q, box = (t.to(torch.float32 if sfx == "f32" else torch.float64) for t in _system(n, 28.0, 3))
     parts = torch.zeros(lib.mnx_pme_real_partials(n), dtype=torch.float64, device=DEV)
     flag = torch.full((1,), -1, dtype=torch.int32, device=DEV)
-    ws = torch.empty(lib.mnx_nlist_workspace_bytes(n), dtype=torch.uint8, device=DEV)
-    _lib.check(lib.mnx_pme_real_f64(ptr(pos), ptr(q), n, ptr(box), 4.0, 0.4, 1.0, None, None, ptr(parts), ptr(flag), ptr(ws),
-                                    ws.numel(), torch.cuda.current_stream().cuda_stream), "real")
-    assert flag.item() == 0
+    need = lib.mnx_pme_real_workspace_bytes(n, sfx == "f64")
+    ws = torch.full((need + 65536,), 0x5a, dtype=torch.uint8, device=DEV)
+    dpos, dq = torch.empty_like(pos), torch.empty_like(q)
+    _lib.check(getattr(lib, f"mnx_pme_real_{sfx}")(
+        ptr(pos), ptr(q), n, ptr(box), 4.0, 0.4, 1.0, ptr(dpos), ptr(dq), ptr(parts), ptr(flag), ptr(ws), need,
+        torch.cuda.current_stream().cuda_stream), "real")
+    assert flag.item() == 0 and (ws[need:] == 0x5a).all()
+    assert torch.isfinite(dpos).all() and torch.isfinite(dq).all()
 
 
 def test_opcheck():
