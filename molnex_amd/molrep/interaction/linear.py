@@ -84,15 +84,24 @@ class Linear(nn.Module):
         ok = ok and all(c <= 8 for c in users.values())
         self._hip_plan = _hip_plan(self) if ok else None
 
-    # the gather indices and scales that put ``weight`` into the fragment order of
-    # ``molix::block_linear`` (forward), for callers of that op
+    def __setstate__(self, state):
+        # a module pickled as a whole holds the launch lists of the version that saved it (once also
+        # fragment tables, as buffers): they are derived from the plan again
+        super().__setstate__(state)
+        for name in [b for b in self._buffers if b.startswith("_hip_")]:
+            del self._buffers[name]
+            self._non_persistent_buffers_set.discard(name)
+        self._setup_hip()
+
+    # the gather indices and scales that put the weights into the fragment order of
+    # ``molix::block_linear`` (forward), for callers of that op; on the module's device if it has weights
     @property
     def _hip_idx_f(self) -> torch.Tensor:
-        return _fragments(self)[0].to(self.weight.device)
+        return _fragments(self)[0].to("cpu" if self.weight is None else self.weight.device)
 
     @property
     def _hip_sc_f(self) -> torch.Tensor:
-        return _fragments(self)[1].to(self.weight.device)
+        return _fragments(self)[1].to("cpu" if self.weight is None else self.weight.device)
 
     def forward(self, x: torch.Tensor, weight: torch.Tensor | None = None,
                 weight_indices: torch.Tensor | None = None) -> torch.Tensor:

@@ -99,3 +99,26 @@ def test_polynomial_cutoff_factored_form_matches_expanded_formula():
     x32 = rn / 5.0
     expanded32 = 1 - 28 * x32 ** 6 + 48 * x32 ** 7 - 21 * x32 ** 8
     assert (expanded32.double() - exact).abs().max() > 1e-6  # the cancellation the factored form avoids
+
+
+def test_a_module_pickled_with_other_launch_lists_gets_its_own():
+    """Launch lists are derived from the irreps when a pickled module is read: one saved before the weights were
+    read in place held {"fwd", "bwd"} and fragment tables as buffers."""
+    import copy
+    import io
+
+    for kw in ({}, {"weight_classes": 3}):
+        lin = Linear("8x0e+16x1o", "8x0e+8x1o", **kw)
+        plan = lin._hip_plan
+        old = copy.deepcopy(lin)
+        old._hip_plan = {"fwd": plan["fwd"], "bwd": []}
+        for name in ("idx_f", "sc_f", "idx_b", "sc_b"):
+            torch.nn.Module.register_buffer(old, "_hip_" + name + "_", torch.zeros(3), persistent=False)
+        buf = io.BytesIO()
+        torch.save(old, buf)
+        buf.seek(0)
+        got = torch.load(buf, weights_only=False)
+        assert got._hip_plan == plan and not list(got.buffers())
+        assert torch.equal(got._hip_idx_f, lin._hip_idx_f) and torch.equal(got._hip_sc_f, lin._hip_sc_f)
+        assert got.state_dict().keys() == lin.state_dict().keys()
+    assert Linear("3x0e", "3x0e")._hip_plan is None and copy.deepcopy(Linear("3x0e", "3x0e"))._hip_plan is None
