@@ -247,22 +247,6 @@ __device__ __forceinline__ AcceptTest<T> accept_test(const T* box, bool periodic
     return a;
 }
 
-// Value of lane q (wave-uniform q) broadcast to the wavefront through v_readlane.
-__device__ __forceinline__ int lane_value(int v, int q) { return __builtin_amdgcn_readlane(v, q); }
-__device__ __forceinline__ float lane_value(float v, int q) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), q));
-}
-__device__ __forceinline__ uint64_t lane_value(uint64_t v, int q) {
-    const uint32_t lo = __builtin_amdgcn_readlane(int(v & 0xffffffffu), q),
-                   hi = __builtin_amdgcn_readlane(int(v >> 32), q);
-    return (uint64_t(hi) << 32) | lo;
-}
-__device__ __forceinline__ double lane_value(double v, int q) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane(int(b & 0xffffffff), q), hi = __builtin_amdgcn_readlane(int(b >> 32), q);
-    return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
-}
-
 // Value of lane (lane ^ s) for a power of two s < 64: DPP for 1, 2 (quad permutes) and 8
 // (rotation by 8 within a row of 16), the LDS crossbar without memory (ds_swizzle, xor
 // within 32 lanes) for 4 and 16, ds_bpermute for 32.

@@ -95,3 +95,38 @@ def test_input_with_infinities_and_bad_arguments():
         args = dict(a=x, weight=w, blocks=rows, scales=sc, out_dim=8, transposed=False)
         with pytest.raises(ValueError):
             torch.ops.molix.block_linear_weights(*{**args, **bad}.values())
+
+
+@pytest.mark.parametrize("irr_in,irr_out", [
+    ("8x0e+16x1o+8x1o", "24x0e+8x1o"),
+    ("96x0e+40x1o", "96x0e+72x1o+32x2e"),                     # three tiles, an output block without source
+    ("128x0e+128x0e+128x1o+128x1o+128x1o+128x3o", "128x0e+200x1o+128x3o"),
+])
+@pytest.mark.parametrize("rows", [0, 1, 129, 1000])
+def test_fragment_ordered_weights(irr_in, irr_out, rows):
+    """molix::block_linear and molix::indexed_block_linear (weights put into operand order by the caller) give
+    the bits of the form that reads the parameter: the same products in the same order.  The classes hold no,
+    one and many rows, and some rows are of none."""
+    from molnex_amd.molrep.interaction import Linear
+
+    torch.manual_seed(rows)
+    lin = Linear(irr_in, irr_out).to(DEV)
+    x = torch.randn(rows, lin.irreps_in.dim, device=DEV)
+    idx, sc, fwd, dim = lin._hip_idx_f, lin._hip_sc_f, lin._hip_plan["fwd"], lin.irreps_out.dim
+    with torch.no_grad():
+        w = lin.weight.reshape(-1)
+        assert torch.equal(torch.ops.molix.block_linear(x, w[idx] * sc, fwd, dim), lin(x))
+    if rows == 0:  # the indexed forms take at least one row
+        return
+    ws = torch.randn(4, lin.weight_numel, device=DEV)
+    z = torch.randint(0, 3, (rows,), device=DEV) * 2  # 0, 2, 4: classes 1 and 3 are empty, 4 is none
+    if rows > 100:
+        z[17] = 3
+        z[5] = -1
+    groups = K.class_groups(z, 4)
+    got = torch.ops.molix.indexed_block_linear(x, ws[:, idx] * sc, *groups, fwd, dim)
+    want = torch.ops.molix.block_linear_weights(x, ws, *lin._hip_plan["rows"], dim, False, *groups)
+    assert torch.equal(got, want) and not got[(z < 0) | (z > 3)].any()
+    per_class = torch.cat([lin(x[n:n + 1], weight=ws[c:c + 1]) if 0 <= c < 4 else torch.zeros(1, dim, device=DEV)
+                           for n, c in enumerate(z.tolist()[:40])])
+    assert torch.equal(got[:40], per_class)
