@@ -257,10 +257,7 @@ def gen_fwd(cfg: Cfg, g: int) -> str:
         a(f"    on[{c} * C + cc[k]] = acc[k][{oi[c]}];")
     a("  }")
     a("}")
-    a(f"template <int CPL, bool FULL>\n__global__ void __launch_bounds__(64) {name}({FWD_PARAMS}) {{")
-    a(f"  {name}_body<CPL, FULL, 64>({FWD_ARGS}, xcd_node(blockIdx.x, gridDim.x), threadIdx.x, blockIdx.y);")
-    a("}")
-    return "\n".join(L)
+    return "\n".join(_whole_wave(name, FWD_PARAMS, L) + L)
 
 
 # Parameters of the receiver-walked kernels and of their bodies.  A body works for LW lanes of a wavefront
@@ -276,7 +273,18 @@ BWD_PARAMS = ("const float* __restrict__ x, const float* __restrict__ Y, const f
               "const int32_t* __restrict__ wrow, int64_t N, int C, float* __restrict__ gx, "
               "float* __restrict__ gw, float* __restrict__ gyp, int npart, int pbase")
 BWD_ARGS = "x, Y, w, gout, row_ptr, perm, snd, wrow, N, C, gx, gw, gyp, npart"
-BODY_PARAMS = "const int64_t n, const int lane, const int cblock"
+BODY_PARAMS = "const int64_t n, const int lane, const uint32_t cblock"
+
+
+def _whole_wave(name: str, params: str, body: list[str]) -> list[str]:
+    """The kernel of one path group, a wavefront per receiver, with the body's text in it: called as a function,
+    the body is simplified before it is inlined and comes out differently (64 channels, 0e+1o, l <= 3, 8000
+    receivers: forward 141.3 us, written out 137.6)."""
+    return [f"template <int CPL, bool FULL>\n__global__ void __launch_bounds__(64) {name}({params}) {{",
+            "  constexpr int LW = 64;",
+            "  const int64_t n = xcd_node(blockIdx.x, gridDim.x);",
+            "  const int lane = threadIdx.x;",
+            "  const uint32_t cblock = blockIdx.y;", *body[1:]]
 
 
 def gen_all(cfg: Cfg) -> str:
@@ -416,10 +424,7 @@ def gen_bwd(cfg: Cfg, g: int) -> str:
     for line in flush:
         a(line[2:] if line.startswith("  ") else line)
     a("}")
-    a(f"template <int CPL, bool FULL>\n__global__ void __launch_bounds__(64) {name}({BWD_PARAMS}) {{")
-    a(f"  {name}_body<CPL, FULL, 64>({BWD_ARGS}, pbase, xcd_node(blockIdx.x, gridDim.x), threadIdx.x, blockIdx.y);")
-    a("}")
-    return "\n".join(L)
+    return "\n".join(_whole_wave(name, BWD_PARAMS, L) + L)
 
 # ---------------------------------------------------------------------------
 # Sender-major backward: one wavefront per (sender, channel block, path subgroup)
