@@ -583,16 +583,18 @@ __device__ __forceinline__ int cell_candidate(const CellRanges& cr, int k, const
     return k < cr.total ? atoms_sorted[start + (k - first)] : -1;
 }
 
-// Calls f(j) for every candidate j of atom i (each j at most once), lanes in parallel.
+// Calls f(j) for every candidate j of atom i (each j at most once), lanes in parallel; of the chunks of
+// one wavefront's width, every `waves`-th from number `wave` on.
 template <typename T, typename F>
 __device__ __forceinline__ void for_candidates(const T* pos, int i, int64_t n, const NlGrid& g,
                                                const int32_t* __restrict__ cell_start,
                                                const int32_t* __restrict__ cell_count,
-                                               const int32_t* __restrict__ atoms_sorted, int mode, F&& f) {
+                                               const int32_t* __restrict__ atoms_sorted, int mode, F&& f, int wave = 0,
+                                               int waves = 1) {
     const int lane = threadIdx.x & (kWave - 1);
     if (g.brute) {
         const int64_t end = mode == MNX_NLIST_HALF ? i : n;
-        for (int64_t base = 0; base < end; base += kWave) {
+        for (int64_t base = wave * kWave; base < end; base += waves * kWave) {
             const int64_t j = base + lane;
             f(j < end && j != i ? int(j) : -1);
         }
@@ -601,7 +603,7 @@ __device__ __forceinline__ void for_candidates(const T* pos, int i, int64_t n, c
     int c[3];
     cell_coords<T>(pos, i, g, c);
     const CellRanges cr = cell_ranges(g, c[0], c[1], c[2], cell_start, cell_count, lane);
-    for (int base = 0; base < cr.total; base += kWave) {
+    for (int base = wave * kWave; base < cr.total; base += waves * kWave) {
         int j = cell_candidate(cr, base + lane, atoms_sorted);
         if (mode == MNX_NLIST_HALF ? j >= i : j == i) j = -1;
         f(j);
@@ -637,17 +639,23 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Bitonic sort of `len` ints in LDS by one wavefront, ascending; buf has room for the next power of
-// two of len (padded with INT_MAX).
+// Bitonic sort of `len` ints in LDS, ascending, by one wavefront or (GROUP) the whole workgroup of four;
+// buf has room for the next power of two of len (padded with INT_MAX).
+template <bool GROUP>
 __device__ void lds_sort(int32_t* buf, int len) {
     int m = 1;
     while (m < len) m <<= 1;
-    const int lane = threadIdx.x & (kWave - 1);
-    for (int k = len + lane; k < m; k += kWave) buf[k] = 0x7fffffff;
-    wave_lds_fence();
+    constexpr int kStep = GROUP ? 4 * kWave : kWave;
+    const int first = threadIdx.x & (kStep - 1);
+    auto fence = [] {
+        if (GROUP) __syncthreads();
+        else wave_lds_fence();
+    };
+    for (int k = len + first; k < m; k += kStep) buf[k] = 0x7fffffff;
+    fence();
     for (int size = 2; size <= m; size <<= 1) {
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int t = lane; t < (m >> 1); t += kWave) {
+            for (int t = first; t < (m >> 1); t += kStep) {
                 const int lo = 2 * t - (t & (stride - 1));
                 const int hi = lo + stride;
                 const bool up = (lo & size) == 0;
@@ -657,7 +665,7 @@ __device__ void lds_sort(int32_t* buf, int len) {
                     buf[hi] = a;
                 }
             }
-            wave_lds_fence();
+            fence();
         }
     }
 }
@@ -709,8 +717,10 @@ __device__ __forceinline__ void write_pair(const T* __restrict__ pos, const T* _
 
 // What the emit's stream leaves: atoms with more than kSlots neighbours (listed by the count pass),
 // and every atom of an all-pairs grid.  Candidates are tested again, collected in LDS and sorted: a
-// wavefront each with a list of kMidCap for the former, then one wavefront of the workgroup with the
-// whole buffer for atoms with still more and for all-pairs grids.  Called by whole workgroups.
+// wavefront each with a list of kMidCap for the former, then the whole workgroup, with the whole
+// buffer, for each atom with still more and of all-pairs grids (one wavefront of the four left it idle:
+// 6000 atoms with 1150 neighbours 1459 us, with all four 567; an all-pairs grid of 8000 atoms 728, 387).
+// Called by whole workgroups.
 template <typename T>
 __device__ void emit_rest(int32_t* buf, const T* __restrict__ pos, int64_t n, const T* __restrict__ box, T cutoff,
                           int mode, int layout, const NlGrid& g, const int32_t* __restrict__ cell_start,
@@ -719,23 +729,15 @@ __device__ void emit_rest(int32_t* buf, const T* __restrict__ pos, int64_t n, co
                           int32_t* __restrict__ idx_i, int32_t* __restrict__ idx_j, T* __restrict__ deltas,
                           T* __restrict__ dist, T* __restrict__ shifts) {
     static_assert(kNlCap == 4 * kMidCap, "one list per wavefront");
+    __shared__ int s_found;
     const bool periodic = g.periodic;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+    const uint64_t below = (uint64_t(1) << lane) - 1;
     const AcceptTest<T> at = accept_test<T>(box, periodic, true, cutoff);
-    auto one = [&](int i, int32_t* list, int cap) {
-        int count = 0;
-        wave_lds_fence();  // the list is reused across atoms
-        for_candidates<T>(pos, i, n, g, cell_start, cell_count, atoms_sorted, mode, [&](int j) {
-            const bool ok = j >= 0 && accept<T>(pos, box, i, j, periodic, cutoff, at);
-            const uint64_t m = __ballot(ok);
-            const int before = __popcll(m & ((uint64_t(1) << lane) - 1));
-            if (ok && count + before < cap) list[count + before] = j;
-            count += __popcll(m);
-        });
-        if (count > cap) count = cap;  // more than kNlCap: flagged by the count pass; host reports the error
-        lds_sort(list, count);
+    // the sorted list's pairs, by `step` threads from number `first` on
+    auto write = [&](int i, const int32_t* list, int count, int first, int step) {
         const int64_t base = layout == MNX_NLIST_TRIANGULAR ? 0 : offsets[i];
-        for (int k = lane; k < count; k += kWave) {
+        for (int k = first; k < count; k += step) {
             const int j = list[k];
             const int64_t slot = layout == MNX_NLIST_TRIANGULAR ? int64_t(i) * (i - 1) / 2 + j : base + k;
             if (slot < capacity) write_pair<T>(pos, box, periodic, i, j, slot, idx_i, idx_j, deltas, dist, shifts);
@@ -743,12 +745,44 @@ __device__ void emit_rest(int32_t* buf, const T* __restrict__ pos, int64_t n, co
     };
     __syncthreads();  // the caller's use of the buffer is over
     if (!g.brute)
-        for (int64_t t = int64_t(blockIdx.x) * 4 + wave; t < g.nmid; t += int64_t(gridDim.x) * 4)
-            one(big[t], buf + wave * kMidCap, kMidCap);
-    __syncthreads();
-    if (wave) return;
-    for (int64_t t = blockIdx.x; t < (g.brute ? n : g.nbig); t += gridDim.x)
-        one(g.brute ? int(t) : big[n - 1 - t], buf, kNlCap);
+        for (int64_t t = int64_t(blockIdx.x) * 4 + wave; t < g.nmid; t += int64_t(gridDim.x) * 4) {
+            const int i = big[t];
+            int32_t* list = buf + wave * kMidCap;
+            int count = 0;
+            wave_lds_fence();  // the list is reused across atoms
+            for_candidates<T>(pos, i, n, g, cell_start, cell_count, atoms_sorted, mode, [&](int j) {
+                const bool ok = j >= 0 && accept<T>(pos, box, i, j, periodic, cutoff, at);
+                const uint64_t m = __ballot(ok);
+                const int to = count + __popcll(m & below);
+                if (ok && to < kMidCap) list[to] = j;
+                count += __popcll(m);
+            });
+            count = min(count, kMidCap);
+            lds_sort<false>(list, count);
+            write(i, list, count, lane, kWave);
+        }
+    for (int64_t t = blockIdx.x; t < (g.brute ? n : g.nbig); t += gridDim.x) {
+        const int i = g.brute ? int(t) : big[n - 1 - t];
+        __syncthreads();
+        if (threadIdx.x == 0) s_found = 0;
+        __syncthreads();
+        for_candidates<T>(
+            pos, i, n, g, cell_start, cell_count, atoms_sorted, mode,
+            [&](int j) {
+                const bool ok = j >= 0 && accept<T>(pos, box, i, j, periodic, cutoff, at);
+                const uint64_t m = __ballot(ok);
+                if (m == 0) return;
+                int to = 0;
+                if (lane == 0) to = atomicAdd(&s_found, __popcll(m));
+                to = __builtin_amdgcn_readfirstlane(to) + __popcll(m & below);
+                if (ok && to < kNlCap) buf[to] = j;
+            },
+            wave, 4);
+        __syncthreads();
+        const int count = min(s_found, kNlCap);  // more: flagged by the count pass; the host reports the error
+        lds_sort<true>(buf, count);
+        write(i, buf, count, threadIdx.x, 4 * kWave);
+    }
 }
 
 // ---------------------------------------------------------------------------

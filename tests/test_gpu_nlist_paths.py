@@ -76,6 +76,19 @@ def test_every_row_length_at_once():
     assert _check(pos, (np.eye(3) * 90).astype(np.float32), 4.0) > 1024
 
 
+@pytest.mark.parametrize("n,full", [(4097, True), (2100, True), (4097, False)])
+def test_rows_as_long_as_the_limit(n, full):
+    """Every pair of one crowd: rows of up to 4096 neighbours fill the list that a whole workgroup sorts, on the
+    cell scan of a wide box and on an all-pairs grid."""
+    pos = np.random.default_rng(n).uniform(0, 3, (n, 3)).astype(np.float32)
+    p = torch.from_numpy(pos).to(DEV)
+    wi, wj = np.nonzero(~np.eye(n, dtype=bool) if full else np.tri(n, k=-1, dtype=bool))
+    for edge in (40.0, 14.0):
+        i, j, _, d, _ = ops.neighbor_list(p, 6.0, torch.eye(3, device=DEV) * edge, full)
+        assert np.array_equal(i.cpu().numpy(), wi) and np.array_equal(j.cpu().numpy(), wj)
+        assert torch.equal(d, p[i.long()] - p[j.long()])
+
+
 def test_duplicates_and_another_stream():
     """Coincident atoms are no pairs (distance 0); a list made on another stream equals the default one's."""
     pos = np.random.default_rng(9).uniform(0, 12, (300, 3)).astype(np.float32)
