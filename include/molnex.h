@@ -343,6 +343,17 @@ int mnx_pme_gather_f64(const double* pos, const double* charges, const double* b
  * *energy, dpos [n][3], dq [n] are overwritten; dpos and dq may both be NULL (energy only, no
  * atomics).  The reference computes both in its forward (pme_cpu.cpp:168-205); the torch op
  * here computes the energy in the forward and the derivatives in the backward. */
+size_t mnx_pme_direct_workspace_bytes(int64_t num_atoms, int64_t num_pairs);
+int mnx_pme_direct_f32(const float* pos, const float* charges, int64_t num_atoms, const int32_t* neighbors,
+                       int64_t num_pairs, const float* deltas, const float* distances,
+                       const int32_t* exclusions, int32_t max_excl, double alpha, double coulomb,
+                       float* energy, float* dpos, float* dq, void* workspace, size_t workspace_bytes,
+                       mnx_stream_t stream);
+int mnx_pme_direct_f64(const double* pos, const double* charges, int64_t num_atoms,
+                       const int32_t* neighbors, int64_t num_pairs, const double* deltas,
+                       const double* distances, const int32_t* exclusions, int32_t max_excl,
+                       double alpha, double coulomb, double* energy, double* dpos, double* dq,
+                       void* workspace, size_t workspace_bytes, mnx_stream_t stream);
 /* Real-space Ewald sum and self term of a periodic system within `cutoff` (minimum image), without a
  * pair list: sum over the neighbor list's pairs (bit for bit its geometry) of coulomb q_i q_j
  * erfc(alpha r) / r, minus coulomb alpha / sqrt(pi) sum q^2 (pme_cpu.cpp:95-135,195-215).  The energy
@@ -374,17 +385,6 @@ int mnx_pme_gather_add_f64(const double* pos, const double* q, const double* box
 int mnx_pme_real_f64(const double* pos, const double* q, int64_t n, const double* box, double cutoff, double alpha,
                      double coulomb, double* dpos, double* dq, double* partials, int32_t* overflow, void* ws,
                      size_t ws_bytes, mnx_stream_t stream);
-size_t mnx_pme_direct_workspace_bytes(int64_t num_atoms, int64_t num_pairs);
-int mnx_pme_direct_f32(const float* pos, const float* charges, int64_t num_atoms, const int32_t* neighbors,
-                       int64_t num_pairs, const float* deltas, const float* distances,
-                       const int32_t* exclusions, int32_t max_excl, double alpha, double coulomb,
-                       float* energy, float* dpos, float* dq, void* workspace, size_t workspace_bytes,
-                       mnx_stream_t stream);
-int mnx_pme_direct_f64(const double* pos, const double* charges, int64_t num_atoms,
-                       const int32_t* neighbors, int64_t num_pairs, const double* deltas,
-                       const double* distances, const int32_t* exclusions, int32_t max_excl,
-                       double alpha, double coulomb, double* energy, double* dpos, double* dq,
-                       void* workspace, size_t workspace_bytes, mnx_stream_t stream);
 
 /* ------------------------------------------------------------------------ */
 /* Symmetric contraction of scalar channels, as the reference configures it  */

@@ -32,10 +32,10 @@
 // wavefronts instead of more rows.
 //
 // Bound by the six matrix-core products per value where K is a few hundred (the
-// linear after a 128-channel 0e+1o convolution, 20k nodes, K 256 to 384: 275 us =
-// 570 TFLOP/s of bf16 products, 288 us over four launches before), and by reading
+// linear after a 128-channel 0e+1o convolution, 20k nodes, K 256 to 384: 271 us =
+// 580 TFLOP/s of bf16 products, 288 us over four launches before), and by reading
 // and writing the rows where it is 128 (its transpose, ten input blocks: 263 us
-// against 362 us; the 0e+1o mixing of 50k nodes, 205 MB: 75 us = 2.7 TB/s, 80 us
+// against 362 us; the 0e+1o mixing of 50k nodes, 205 MB: 78 us = 2.6 TB/s, 80 us
 // before).  The launches saved are the rest: one instead of one per block, and no
 // gather of the weights into an operand order first (two more): the whole linear
 // forward, backward and weight gradient takes 4 launches instead of 48.

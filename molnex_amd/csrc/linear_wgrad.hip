@@ -27,9 +27,10 @@
 //
 // Bound by reading x and g through two wavefronts' loads per SIMD: the linear
 // after a 128-channel 0e+1o convolution (20k nodes, ten pairs, 574 MB) takes
-// 217 us = 2.6 TB/s, the two pairs of a 0e+1o mixing (50k nodes, 205 MB) 55 us =
-// 3.7 TB/s, both kernels together.  More, shorter slabs cost partial tiles:
-// 2950 wavefronts 229 / 71 us, 5900 247 / 91 us.  fp32 MFMAs instead of the
+// 200 us = 2.9 TB/s, the two pairs of a 0e+1o mixing (50k nodes, 205 MB) 67 us =
+// 3.1 TB/s, both kernels together (profiles/timed_cases_kernel_stats.md).  More, shorter
+// slabs cost partial tiles (in another session, against 217 and 55 us): 2950 wavefronts
+// 229 / 71 us, 5900 247 / 91 us.  fp32 MFMAs instead of the
 // split took 473 us, per-pair slabs (the gradient rows re-read from HBM) 268 us.
 // The form before, torch gathers of every pair's rows into GEMM operands and a
 // batched library GEMM each, took about 700 us over 30 launches.

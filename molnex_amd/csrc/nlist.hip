@@ -35,8 +35,9 @@
 //
 // Bound by the candidate tests and launches, not by its 36 bytes per pair:
 // 100k atoms, 5.24 M ordered pairs (189 MB written): 206 us in all, the count
-// pass 85 us (1100 vector and as many scalar instructions per wavefront: the
-// tests, the sort and each cell's set-up), the emit 68 us (2.8 TB/s), five binning
+// pass 88 us (1100 vector and as many scalar instructions per wavefront: the
+// tests, the sort and each cell's set-up), the emit 53 us (3.6 TB/s; 67 us with the
+// atoms in another order), five binning
 // and scan launches and the host's read of the total the rest; 283 us with a
 // sorting emit behind accept ballots (130 us), a second sort inside the cells and
 // 18 launches.  96 atoms: 49 us (three launches of 3 us, the host's calls and its

@@ -19,11 +19,17 @@ Ops
 ``molix::radial_hidden``        fused hidden stack of the radial weight MLP (gradient w.r.t. its input)
 ``molix::edge_weights``         output layer of the radial weight MLP (per-edge TP weights), near-fp32 split-fp16 MFMA
 ``molix::bond_vectors``         pos[receiver] - pos[sender] - shift per edge, with its position gradient
-``molix::block_linear``         equivariant (ir_mul) block linear with pre-ordered weights (``cuet.Linear``)
-``molix::indexed_block_linear`` the block linear with one weight set per node class (ElementUpdate)
+``molix::block_linear_weights`` equivariant (ir_mul) block linear, weights read where they lie (``cuet.Linear``), also with
+                                one weight set per node class (ElementUpdate)
+``molix::block_linear_weight_grad`` its weight gradient, every block pair in one launch
+``molix::block_linear``, ``molix::indexed_block_linear`` the same kernel on weights in operand order (no module's; exported
+                                programs of earlier versions call them)
 ``molix::radial_tp``            radial-MLP output layer + tp_scatter, backward through ``molix::tp_weight_grad``
 ``molix::edge_reverse``         the opposite edge of each edge (undirected pairs with identical radial inputs)
 ``molix::radial_tp_pairs``      radial-MLP output layer once per undirected pair + tp_scatter over both directions
+``molix::pme_energy``           PME energy of a periodic system: real-space, reciprocal and self terms in one op each way
+``molix::pair_features``        radial features, both atoms' type embeddings and the envelope of each edge (Allegro)
+``molix::residual_blocks``      weight blocks of a residual linear layer (Allegro's layer tail)
 ``molix::segment_sum``          weighted segment sum of rows by segment id (scatter_sum / MessageAggregation)
 """
 
@@ -1025,7 +1031,8 @@ def pme_energy(positions: Tensor, charges: Tensor, box_vectors: Tensor, xmoduli:
                coulomb: float, gradients: bool) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     """The whole PME energy of a periodic system: the real-space sum over the pairs within ``cutoff``
     (minimum image) and the self term straight from the cell scan (no pair list, no host read of its
-    length), plus the reciprocal sum of ``molix::pme_reciprocal``.
+    length; sums in a fixed order), plus the reciprocal sum of ``molix::pme_reciprocal``.  Raises where an
+    atom has more than 4096 neighbours of lower index, the half list's limit.
 
     Returns ``(energy, spectrum, dpos, dq)``: the convolved half spectrum and, with ``gradients``, the
     derivatives of the real-space and self terms (else empty), which the backward uses; those three

@@ -76,8 +76,7 @@ def test_energy_and_gradients(n, edge, cut, mesh, order, kind, dtype, tol):
     want = _composed(pme, pos, q, box)
     got = _run(pme, pos, q, box)
     _close(got, want, tol, pme.coulomb * pme.alpha * float((q.double() ** 2).sum()))
-    # bitwise the same again where the sums have a fixed order (all pairs); the cell scan's lists arrive in
-    # any order, and its fp64 sums differ in their last bits
+    # bitwise the same again (the cell scan: test_the_same_bits_every_time)
     again = _run(pme, pos, q, box)
     if n <= 2048:
         assert all(torch.equal(a, b) for a, b in zip(got, again))
